@@ -9,27 +9,35 @@
 // non-finite values, then repeat {keep values within median -/+ 3 std,
 // inclusive} until a round removes nothing).
 //
-// Here the photon list stays in HBM:
-//   1. count   one wave per chunk of photons: per order, the summed
-//              probability, the photons counted (flag MX_OS_FILTER: only
-//              finite value and probability > 0) and those with a finite
-//              value, each lane in its own LDS slot (no atomics: the sums
-//              have a fixed order for a given photon count);
-//   2. scan    per order (one workgroup each), chunk offsets into one array
-//              of segments (one segment per order) and the totals;
-//   3. scatter the finite values of each order into its segment;
-//   4. sort    all values by value, then (stably) by order: two device-wide
-//              hipCUB radix sorts leave every segment sorted (a segmented
-//              sort would give each of the few, large segments one
-//              workgroup);
-//   5. clip    one workgroup per order: on a sorted segment the kept set of
-//              every round is a contiguous range, so a round is a median
-//              read, two block reductions (mean, then squared deviations)
-//              and two binary searches for the new ends.
+// Here the photon list stays in HBM and nothing is sorted.  The kept set of
+// every round is an interval of values, so it is enough to know the values in
+// bins (count, mean, squared deviations of each) and to look inside the few
+// bins that hold a bound or the median:
+//   1. sample  one workgroup per order sorts up to 4096 photons drawn over the
+//              list and takes evenly filled bin edges from them;
+//   2. split   each workgroup takes one chunk of photons, orders its counted
+//              values by (order, bin) in LDS and writes them back in that order
+//              with the offset of every (order, bin) piece, the piece's sums of
+//              deviations and squared deviations from an edge of the bin, and
+//              the probability sum of each order;
+//   3. merge   adds up the pieces' sums, and copies the values of the bins that
+//              are likely to be looked into to one place each;
+//   4. clip    one workgroup per order: the rounds, from the bins' sums and the
+//              values of the bins that hold a bound or the median.
+// The bins only decide how fast the answer is found, never what it is: edges
+// are compared exactly, the median is selected exactly, and a bound's bin is
+// summed value by value.  Every sum has a fixed order for a given photon list.
 // The library allocates nothing: all scratch is the caller's workspace.
+//
+// What it costs: the columns are read once (20 B per photon) and the counted
+// values written once (8 B each); a method that keeps no table of values could
+// do with the read alone.  The two device-wide radix sorts this replaced
+// moved each value nine times.  CaptureResAeff on 8e6 photons in 15 orders:
+// 1230 us a call with them, 377 us now, 211 us of it in the kernels (160 MB: 26
+// us at the card's read rate); on 5e4 photons 400 us in 44 launches, now 223 us
+// in 4, 86 us of it in the kernels.
 
 #include <hip/hip_runtime.h>
-#include <hipcub/hipcub.hpp>
 #include <mutex>
 #include <stdint.h>
 #include <stdio.h>
@@ -39,90 +47,97 @@
 
 __attribute__((visibility("hidden"))) void mx_set_error(const char *msg);
 
-#define MX_OS_WAVE 64          // work-items per counting / scatter workgroup
-#define MX_OS_CLIP 1024        // work-items per clipping workgroup
-#define MX_OS_UNROLL 8         // independent loads in flight per work-item (clipping sums)
-#define MX_OS_LOADS 8          // photons loaded ahead per lane (counting, scatter)
-#define MX_OS_CHUNK 4096       // photons per counting workgroup (at least)
-#define MX_OS_MAX_BLOCKS 16384
-#define MX_OS_SCAN 256         // work-items per scan workgroup (one per order)
-
-static int64_t os_blocks(int64_t n) {
-    int64_t nb = (n + MX_OS_CHUNK - 1) / MX_OS_CHUNK;
-    if (nb < 1) nb = 1;
-    if (nb > MX_OS_MAX_BLOCKS) nb = MX_OS_MAX_BLOCKS;
-    return nb;
-}
+#define MX_OS_SAMPLE 4096      // photons looked at for the bin edges
+#define MX_OS_SPLIT 512        // work-items per splitting workgroup
+#define MX_OS_SPLIT_WAVES (MX_OS_SPLIT / 64)
+// Photons per work-item of the splitting kernel.  12 (chunks of 6144, 77 KiB
+// of LDS, two workgroups per CU) keeps the number of chunks, and with it the
+// piece tables, small; below MX_OS_FEW photons that would leave CUs without a
+// chunk (326 chunks at 2e6), so 4 are taken there.
+#define MX_OS_ROWS 12
+#define MX_OS_ROWS_FEW 4
+#define MX_OS_FEW 2000000
+#define MX_OS_MERGE 512        // work-items per merging workgroup
+#define MX_OS_MERGE_RUN 8      // chunks a work-item of it merges, about
+#define MX_OS_NEAR 12          // bins around the middle that are copied to one place,
+#define MX_OS_ENDS 4           // and at each end
+#define MX_OS_PIECES 8         // pieces in flight per work-item
+// Work-items per clipping workgroup: with 1024 each wave would have 128 VGPRs,
+// and the kernel needs 174.
+#define MX_OS_CLIP 512
+#define MX_OS_LIST 15360       // values of a bin the clipping workgroup holds in LDS
+#define MX_OS_HIST 2048        // buckets of a selection round
+#define MX_OS_CAND 64          // values ranked by counting, one per lane
+#define MX_OS_MAX_BINS 512
+#define MX_OS_LUT 256
 
 static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
-// Workspace layout (bytes, each part 256-aligned).
-struct OsLayout {
-    size_t cnt_b, nval_b, psum_b, off_b, tot, seg, vals, sorted, ord, ord2, clip, part0, part1, temp,
-        temp_bytes, total;
+// Sizes of one call and the byte offsets of its workspace parts.
+struct OsPlan {
+    int32_t no, bins, keys;           // orders; bins per order; pieces per chunk
+    int32_t rows, chunk, groups;      // photons per work-item and per chunk; groups of chunks
+    int64_t chunks, stride;           // chunks; length of an offset row (one per piece, an entry per chunk)
+    size_t edges, off, piece, grp, place, next, psum, vals, copied, total;
 };
 
-#define MX_OS_CW 16            // workgroups per order in the clipping sums
-
-// Clipping state of one order between the launches of the rounds.
-struct ClipState {
-    int64_t lo, hi;            // current range of the sorted segment
-    double med, mean, sd;      // statistics of that range when `have`
-    int32_t done, have;        // no further round; statistics final
+// One bin: place of its values when they were copied (-1: in pieces), their
+// count, the sums of deviations and of their squares from bin_ref.
+struct BinInfo {
+    int64_t at;
+    double n, s1, s2;
 };
 
-// temporary storage of the two radix sorts (by value with the order index
-// as payload, then by order index with the value as payload)
-static int os_sort_temp_bytes(int64_t n, size_t &bytes) {
-    size_t b1 = 0, b2 = 0;
-    if (hipcub::DeviceRadixSort::SortPairs(nullptr, b1, (const double *)nullptr, (double *)nullptr,
-                                           (const uint8_t *)nullptr, (uint8_t *)nullptr, (int)n, 0, 64,
-                                           (hipStream_t)0) != hipSuccess)
-        return 1;
-    if (hipcub::DeviceRadixSort::SortPairs(nullptr, b2, (const uint8_t *)nullptr, (uint8_t *)nullptr,
-                                           (const double *)nullptr, (double *)nullptr, (int)n, 0, 8,
-                                           (hipStream_t)0) != hipSuccess)
-        return 1;
-    bytes = b1 > b2 ? b1 : b2;
-    return 0;
-}
-
-static int os_layout(int64_t n, int no, bool values, OsLayout &L) {
-    const int64_t nb = os_blocks(n);
+// Bins per order: about 1000 (order, bin) pieces in all, so that the split
+// kernel's counters fit beside the values in LDS; each order has one more
+// piece for the photons whose value is not counted.
+static void os_plan(int64_t n, int no, bool values, OsPlan &L) {
+    int bins = 0;
+    if (values) {
+        bins = 16;
+        while (bins * 2 <= MX_OS_MAX_BINS && bins * 2 * no <= 1024) bins *= 2;
+    }
+    L.no = no;
+    L.bins = bins;
+    L.keys = no * (bins + 1);
+    L.rows = n >= MX_OS_FEW ? MX_OS_ROWS : MX_OS_ROWS_FEW;
+    L.chunk = L.rows * MX_OS_SPLIT;
+    L.chunks = (n + L.chunk - 1) / L.chunk;
+    L.stride = (L.chunks + 63) & ~(int64_t)63;
+    const int64_t run = (int64_t)MX_OS_MERGE * MX_OS_MERGE_RUN / (bins > 0 ? bins : 1);   // chunks per group
+    const int64_t g = (L.chunks + run - 1) / run;
+    L.groups = (int32_t)(g < 1 ? 1 : (g > 256 ? 256 : g));
     size_t o = 0;
-    L.cnt_b = o;  o += align256(sizeof(int64_t) * nb * no);
-    L.nval_b = o; o += align256(sizeof(int64_t) * nb * no);
-    L.psum_b = o; o += align256(sizeof(double) * nb * no);
-    L.off_b = o;  o += align256(sizeof(int64_t) * nb * no);
-    L.tot = o;    o += align256(sizeof(int64_t) * no);
-    L.seg = o;    o += align256(sizeof(int32_t) * 2 * no);
-    L.vals = o;   o += values ? align256(sizeof(double) * (n > 0 ? n : 1)) : 0;
-    L.sorted = o; o += values ? align256(sizeof(double) * (n > 0 ? n : 1)) : 0;
-    L.ord = o;    o += values ? align256(n > 0 ? n : 1) : 0;
-    L.ord2 = o;   o += values ? align256(n > 0 ? n : 1) : 0;
-    L.clip = o;   o += values ? align256(sizeof(ClipState) * no) : 0;
-    L.part0 = o;  o += values ? align256(sizeof(double) * no * MX_OS_CW) : 0;
-    L.part1 = o;  o += values ? align256(sizeof(double) * no * MX_OS_CW) : 0;
-    L.temp = o;
-    L.temp_bytes = 0;
-    if (values && os_sort_temp_bytes(n, L.temp_bytes)) return 1;
-    o += align256(L.temp_bytes > 0 ? L.temp_bytes : 1);
+    L.edges = o;  o += align256(sizeof(double) * (size_t)no * bins);
+    L.off = o;    o += align256(sizeof(uint16_t) * (size_t)L.stride * (L.keys + 1));
+    L.piece = o;  o += align256(sizeof(double2) * (size_t)L.chunks * no * bins);
+    L.grp = o;    o += align256(sizeof(BinInfo) * (size_t)L.groups * no * bins);
+    L.place = o;  o += align256(sizeof(int64_t) * (size_t)no * bins);
+    L.next = o;   o += align256(sizeof(unsigned long long));
+    L.psum = o;   o += align256(sizeof(double) * (size_t)L.chunks * no);
+    L.vals = o;   o += values ? align256(sizeof(double) * (size_t)L.chunks * L.chunk) : 0;
+    L.copied = o; o += values ? align256(sizeof(double) * (size_t)(n > 0 ? n : 1)) : 0;
     L.total = o;
-    return 0;
+    // The size that callers are told, and that the static workspace is
+    // checked against, is that of the limits this library states (27.17 B per
+    // photon with values, 32 B per order and 4096 photons): the call itself
+    // needs less from some thousand photons on.
+    const int64_t nb = n <= 0 ? 1 : (n + 4095) / 4096 > 16384 ? 16384 : (n + 4095) / 4096;
+    const size_t stated = (size_t)32 * nb * no + (values ? (size_t)27 * n + (size_t)n * 17 / 100 : 0) + 1024;
+    if (L.total < stated) L.total = align256(stated);
 }
 
+// ------------------------------------------------------------ order lookup
 // index of order o in the list (linear: at most MX_MAX_ORDERS entries), -1
 __device__ __forceinline__ int order_index(const int *ords, int no, int o) {
-    int k = -1;
     for (int j = 0; j < no; ++j)
-        if (ords[j] == o) { k = j; break; }
-    return k;
+        if (ords[j] == o) return j;
+    return -1;
 }
 
 // Order number -> index through a table of MX_OS_LUT entries in LDS when the
 // orders span fewer values (the usual case), else the linear search.  Built
-// by the one wave of a counting / scatter workgroup.
-#define MX_OS_LUT 256
+// by the whole workgroup.
 struct OrderLut {
     const int *t;
     const int *ords;
@@ -137,18 +152,14 @@ struct OrderLut {
 };
 
 __device__ __forceinline__ OrderLut build_lut(const MxOrderStats &a, int *ords, int *lut) {
-    const int no = a.n_orders, lane = threadIdx.x;
+    const int no = a.n_orders;
+    for (int k = threadIdx.x; k < no; k += blockDim.x) ords[k] = a.orders[k];
+    for (int j = threadIdx.x; j < MX_OS_LUT; j += blockDim.x) lut[j] = MX_MAX_ORDERS;
+    __syncthreads();
     int mn = 0x7fffffff, mx = INT32_MIN;
-    for (int k = lane; k < no; k += MX_OS_WAVE) {
-        const int o = a.orders[k];
-        ords[k] = o;
-        mn = o < mn ? o : mn;
-        mx = o > mx ? o : mx;
-    }
-    for (int w = 32; w > 0; w >>= 1) {
-        const int omn = __shfl_xor(mn, w, MX_OS_WAVE), omx = __shfl_xor(mx, w, MX_OS_WAVE);
-        mn = omn < mn ? omn : mn;
-        mx = omx > mx ? omx : mx;
+    for (int k = 0; k < no; ++k) {
+        mn = ords[k] < mn ? ords[k] : mn;
+        mx = ords[k] > mx ? ords[k] : mx;
     }
     OrderLut L;
     L.t = lut;
@@ -156,394 +167,1135 @@ __device__ __forceinline__ OrderLut build_lut(const MxOrderStats &a, int *ords, 
     L.lo = mn;
     L.no = no;
     L.ok = (int64_t)mx - (int64_t)mn < MX_OS_LUT;
-    for (int j = lane; j < MX_OS_LUT; j += MX_OS_WAVE) lut[j] = MX_MAX_ORDERS;
-    __syncthreads();
     // the first index of an order number, as the linear search finds it
     if (L.ok)
-        for (int k = lane; k < no; k += MX_OS_WAVE) atomicMin(&lut[(int64_t)a.orders[k] - mn], k);
+        for (int k = threadIdx.x; k < no; k += blockDim.x) atomicMin(&lut[(int64_t)ords[k] - mn], k);
     __syncthreads();
     return L;
 }
 
+// ---------------------------------------------------------------- 1 sample
+// Place of edge j (of bins - 1) among m sorted values: evenly filled bins, the
+// outer two half as full (1/512 of the values at least, where the 3 sigma
+// bounds of a bell curve still fall): the clipping looks into them every round.
+__device__ __forceinline__ int edge_rank(int j, int bins, int m) {
+    const double q = 0.5 / (bins - 1) > 1.0 / 512 ? 0.5 / (bins - 1) : 1.0 / 512;
+    const int i = (int)((double)m * (q + (double)j * ((1.0 - 2.0 * q) / (bins - 2))));
+    return i < m ? i : m - 1;
+}
 
-// Pass 1: per chunk and order, probability sum, counted photons, finite
-// values.  One wave per workgroup; lane l accumulates into slot [k][l].
-__global__ __launch_bounds__(MX_OS_WAVE) void mx_os_count_kernel(MxOrderStats a, int64_t chunk,
-                                                                  int64_t *cnt_b, int64_t *nval_b,
-                                                                  double *psum_b) {
-    extern __shared__ __align__(16) unsigned char sm[];
-    const int no = a.n_orders, lane = threadIdx.x;
-    double *sp = (double *)sm;                          // [no][64]
-    int *sc = (int *)(sp + no * MX_OS_WAVE);            // [no][64]
-    int *sv = sc + no * MX_OS_WAVE;                     // [no][64]
-    int *ords = sv + no * MX_OS_WAVE;                   // [no]
-    __shared__ int lut[MX_OS_LUT];
-    for (int k = 0; k < no; ++k) {
-        sp[k * MX_OS_WAVE + lane] = 0.0;
-        sc[k * MX_OS_WAVE + lane] = 0;
-        sv[k * MX_OS_WAVE + lane] = 0;
-    }
-    const OrderLut index_of = build_lut(a, ords, lut);
-    const int64_t b0 = (int64_t)blockIdx.x * chunk;
-    int64_t b1 = b0 + chunk;
-    if (b1 > a.n) b1 = a.n;
+// Bin edges of one order (one workgroup each): the finite, counted values of
+// this order among MX_OS_SAMPLE photons, one from a pseudo-random place of
+// each of as many equal parts of the list, sorted; the edges split them
+// (edge_rank).  An edge that repeats moves up by one step of the number format, so
+// that a value holding many photons has a bin of its own.  Bin of x: the
+// number of edges <= x.  Bound by the latency of its loads and of the sort
+// (17 us at 15 orders and 8e6 photons).
+__global__ __launch_bounds__(1024) void mx_os_sample_kernel(MxOrderStats a, OsPlan L,
+                                                             unsigned char *ws) {
+    __shared__ double s[MX_OS_SAMPLE];
+    __shared__ int cnt;
+    const int k = blockIdx.x, t = threadIdx.x, mine = a.orders[k];
+    const int bins = L.bins;
+    double *edges = (double *)(ws + L.edges);
+    if (k == 0 && t == 0) *(unsigned long long *)(ws + L.next) = 0;    // the merge kernel's allocator
     const bool filter = (a.flags & MX_OS_FILTER) != 0;
-    // MX_OS_LOADS photons of the lane are loaded before any is counted (the
-    // loads overlap); they are counted in index order, as one at a time
-    for (int64_t i0 = b0 + lane; i0 < b1; i0 += (int64_t)MX_OS_WAVE * MX_OS_LOADS) {
-        int ord[MX_OS_LOADS];
-        double pr[MX_OS_LOADS], val[MX_OS_LOADS];
-#pragma unroll
-        for (int u = 0; u < MX_OS_LOADS; ++u) {
-            const int64_t i = i0 + (int64_t)u * MX_OS_WAVE;
-            const bool in = i < b1;
-            ord[u] = in ? a.order[i] : INT32_MIN;
-            pr[u] = in ? a.prob[i] : 0.0;
-            val[u] = (in && a.value) ? a.value[i] : 0.0;
-        }
-#pragma unroll
-        for (int u = 0; u < MX_OS_LOADS; ++u) {
-            if (i0 + (int64_t)u * MX_OS_WAVE >= b1) break;
-            const int k = index_of(ord[u]);
-            if (k < 0) continue;
-            sp[k * MX_OS_WAVE + lane] += pr[u];
-            if (!filter || (isfinite(val[u]) && pr[u] > 0.0)) {
-                sc[k * MX_OS_WAVE + lane] += 1;
-                if (a.value && isfinite(val[u])) sv[k * MX_OS_WAVE + lane] += 1;
-            }
-        }
-    }
+    if (t == 0) cnt = 0;
     __syncthreads();
-    for (int k = lane; k < no; k += MX_OS_WAVE) {
-        double s = 0.0;
-        int64_t c = 0, v = 0;
-        for (int l = 0; l < MX_OS_WAVE; ++l) {
-            s += sp[k * MX_OS_WAVE + l];
-            c += sc[k * MX_OS_WAVE + l];
-            v += sv[k * MX_OS_WAVE + l];
+    const int64_t parts = a.n < MX_OS_SAMPLE ? a.n : MX_OS_SAMPLE;
+    int64_t at[MX_OS_SAMPLE / 1024];
+    int ord[MX_OS_SAMPLE / 1024];
+#pragma unroll
+    for (int r = 0; r < MX_OS_SAMPLE / 1024; ++r) {
+        const int64_t i = t + 1024 * r;
+        at[r] = -1;
+        if (i < parts) {
+            const int64_t b = i * a.n / parts, e = (i + 1) * a.n / parts;
+            const uint32_t h = ((uint32_t)i * 2654435761u) >> 7;
+            at[r] = b + (int64_t)h % (e - b);
         }
-        const size_t o = (size_t)blockIdx.x * no + k;
-        psum_b[o] = s;
-        cnt_b[o] = c;
-        nval_b[o] = v;
+        ord[r] = parts > 0 ? a.order[at[r] >= 0 ? at[r] : 0] : 0;
+    }
+    double v[MX_OS_SAMPLE / 1024], pr[MX_OS_SAMPLE / 1024];
+#pragma unroll
+    for (int r = 0; r < MX_OS_SAMPLE / 1024; ++r) {
+        if (ord[r] != mine) at[r] = -1;
+        v[r] = parts > 0 ? a.value[at[r] >= 0 ? at[r] : 0] : 0.0;
+        pr[r] = parts > 0 && filter ? a.prob[at[r] >= 0 ? at[r] : 0] : 1.0;
+    }
+#pragma unroll
+    for (int r = 0; r < MX_OS_SAMPLE / 1024; ++r)
+        if (at[r] >= 0 && isfinite(v[r]) && (!filter || pr[r] > 0.0)) s[atomicAdd(&cnt, 1)] = v[r];
+    __syncthreads();
+    const int m = cnt;
+    int size = 1;
+    while (size < m) size *= 2;
+    for (int i = m + t; i < size; i += 1024) s[i] = __builtin_inf();
+    __syncthreads();
+    if (m <= 512) {
+        // few values: each goes to the place that its rank says, one step
+        // instead of up to 45 with a barrier each
+        int rank = 0;
+        const double x = t < m ? s[t] : 0.0;
+        if (t < m)
+#pragma unroll 16
+            for (int j = 0; j < m; ++j) rank += (s[j] < x || (s[j] == x && j < t)) ? 1 : 0;
+        __syncthreads();
+        if (t < m) s[rank] = x;
+        __syncthreads();
+        size = 1;
+    }
+    for (int w = 2; w <= size; w *= 2)
+        for (int d = w / 2; d > 0; d /= 2) {
+            for (int i = t; i < size / 2; i += 1024) {
+                const int lo = 2 * i - (i & (d - 1)), hi = lo + d;
+                const double x = s[lo], y = s[hi];
+                if ((x > y) == ((lo & w) == 0)) {
+                    s[lo] = y;
+                    s[hi] = x;
+                }
+            }
+            __syncthreads();
+        }
+    for (int j = t; j < bins; j += 1024) {
+        // the last entry only fills the row
+        double e = __builtin_inf();
+        if (m > 0 && j < bins - 1) {
+            e = s[edge_rank(j, bins, m)];
+            if (j > 0 && s[edge_rank(j - 1, bins, m)] == e) e = nextafter(e, __builtin_inf());
+        }
+        edges[(size_t)k * bins + j] = e;
+        ((int64_t *)(ws + L.place))[(size_t)k * bins + j] = -1;
     }
 }
 
-// Pass 2: one workgroup per order.  Work-item t takes a contiguous run of
-// chunks; the run totals are scanned in order by work-item 0, then every
-// work-item writes its chunks' offsets.  Sums run in a fixed order.
-__global__ __launch_bounds__(MX_OS_SCAN) void mx_os_scan_kernel(MxOrderStats a, int64_t nb,
-                                                                 const int64_t *cnt_b, const int64_t *nval_b,
-                                                                 const double *psum_b, int64_t *off_b,
-                                                                 int64_t *tot) {
-    __shared__ int64_t sv[MX_OS_SCAN], sc[MX_OS_SCAN];
-    __shared__ double ss[MX_OS_SCAN];
-    const int no = a.n_orders, k = blockIdx.x, t = threadIdx.x;
-    const int64_t per = (nb + MX_OS_SCAN - 1) / MX_OS_SCAN;
-    const int64_t b0 = (int64_t)t * per;
-    const int64_t b1 = b0 + per < nb ? b0 + per : nb;
-    int64_t v = 0, c = 0;
-    double s = 0.0;
-    for (int64_t b = b0; b < b1; ++b) {
-        const size_t o = (size_t)b * no + k;
-        v += nval_b[o];
-        c += cnt_b[o];
-        s += psum_b[o];
+// What a bin's sums are taken about: its edge nearer to the middle of the
+// order, so that deviations from any point between the bins' middle and that
+// edge add up without cancelling; 0 for an order without a photon in the
+// sample.
+__device__ __forceinline__ double bin_ref(const double *edges, int bins, int b) {
+    const double e = edges[b < bins / 2 ? b : b - 1];
+    return isfinite(e) ? e : 0.0;
+}
+
+__device__ __forceinline__ int bin_of(const double *edges, int bins, double x) {
+    int b = 0;
+    for (int h = bins >> 1; h > 0; h >>= 1)
+        if (edges[b + h - 1] <= x) b += h;
+    return b;
+}
+
+// ----------------------------------------------------------------- 2 split
+// LDS of the split kernel: the chunk's values (then its probabilities), the
+// edges, one counter (16 bits) per wave and piece, piece starts.
+static size_t split_lds(const OsPlan &L) {
+    const int kh = (L.keys + 1) & ~1;
+    return sizeof(double) * L.chunk + sizeof(double) * (size_t)L.no * L.bins +
+           sizeof(uint16_t) * ((size_t)MX_OS_SPLIT_WAVES * kh + kh + 2);
+}
+
+// One chunk of photons ordered by (order, bin).  A photon's place is the start
+// of its piece, plus the photons of the piece in the waves before, plus its
+// rank within its wave, which an LDS counter of that wave and piece returns:
+// only one wave uses it, and the lanes of one LDS instruction are served in a
+// fixed order, so places and sums are the same in every run.  Reads
+// 20 B per photon and writes 8 B per counted value plus 18 B per piece; bound
+// by the LDS work between (edge search 6 reads per value at 64 bins, counter,
+// scatter, sums): 76 us for 8e6 photons in 15 orders (247 MB: 48 us at the
+// card's copy rate).
+template <int ROWS, bool VALUES>
+__global__ __launch_bounds__(MX_OS_SPLIT, 4) void mx_os_split_kernel(MxOrderStats a, OsPlan L, unsigned char *ws) {
+    extern __shared__ __align__(16) unsigned char sm[];
+    __shared__ int ords[MX_MAX_ORDERS], lut[MX_OS_LUT], wtot[MX_OS_SPLIT_WAVES];
+    constexpr int CH = ROWS * MX_OS_SPLIT;
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+    const int keys = L.keys, kh = (keys + 1) & ~1, bins = VALUES ? L.bins : 0;
+    double *buf = (double *)sm;
+    double *edges = buf + CH;
+    uint16_t *hist = (uint16_t *)(edges + (size_t)L.no * bins);   // [wave][kh]
+    uint16_t *start = hist + MX_OS_SPLIT_WAVES * kh;              // [keys + 1]
+    uint32_t *mine = (uint32_t *)(hist + w * kh);
+    const int64_t c = blockIdx.x, c0 = c * CH;
+    const bool filter = (a.flags & MX_OS_FILTER) != 0;
+    // columns first: their latency covers the set-up below
+    int ord[ROWS];
+    double pr[ROWS], val[ROWS];
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) {
+        const int64_t i = c0 + r * MX_OS_SPLIT + t;
+        const bool in = i < a.n;
+        ord[r] = in ? a.order[i] : INT32_MIN;
+        pr[r] = in ? a.prob[i] : 0.0;
+        val[r] = (VALUES && in) ? a.value[i] : 0.0;
     }
-    sv[t] = v;
-    sc[t] = c;
-    ss[t] = s;
+    for (int j = lane; j < kh / 2; j += 64) mine[j] = 0;
+    if (VALUES) {
+        const double *ge = (const double *)(ws + L.edges);
+        for (int j = t; j < L.no * bins; j += MX_OS_SPLIT) edges[j] = ge[j];
+    }
+    const OrderLut index_of = build_lut(a, ords, lut);
+    __shared__ double part[MX_MAX_ORDERS];
+    double *psum = (double *)(ws + L.psum);
+    uint16_t *off = (uint16_t *)(ws + L.off) + c;
+    if (!VALUES && L.no <= MX_OS_SPLIT_WAVES) {
+        // sums alone, few orders: in registers (their counters in LDS would
+        // be the same few words for all lanes: 1e7 photons of one order
+        // 123 us a call, 101 us this way)
+        double s[MX_OS_SPLIT_WAVES];
+        int m[MX_OS_SPLIT_WAVES];
+#pragma unroll
+        for (int k = 0; k < MX_OS_SPLIT_WAVES; ++k) {
+            s[k] = 0.0;
+            m[k] = 0;
+        }
+#pragma unroll
+        for (int r = 0; r < ROWS; ++r) {
+            const int k0 = c0 + r * MX_OS_SPLIT + t < a.n ? index_of(ord[r]) : -1;
+#pragma unroll
+            for (int k = 0; k < MX_OS_SPLIT_WAVES; ++k) {
+                s[k] += k == k0 ? pr[r] : 0.0;
+                m[k] += k == k0 ? 1 : 0;
+            }
+        }
+        __shared__ int count[MX_MAX_ORDERS];
+#pragma unroll
+        for (int k = 0; k < MX_OS_SPLIT_WAVES; ++k) {
+            for (int o = 32; o > 0; o >>= 1) {
+                s[k] += __shfl_xor(s[k], o);
+                m[k] += __shfl_xor(m[k], o);
+            }
+            if (lane == 0) {
+                part[k * MX_OS_SPLIT_WAVES + w] = s[k];
+                count[k * MX_OS_SPLIT_WAVES + w] = m[k];
+            }
+        }
+        __syncthreads();
+        if (t == 0) {
+            int run = 0;
+            for (int k = 0; k < L.no; ++k) {
+                double x = 0.0;
+                off[(size_t)k * L.stride] = (uint16_t)run;
+                for (int q = 0; q < MX_OS_SPLIT_WAVES; ++q) {
+                    x += part[k * MX_OS_SPLIT_WAVES + q];
+                    run += count[k * MX_OS_SPLIT_WAVES + q];
+                }
+                psum[(size_t)k * L.chunks + c] = x;
+            }
+            off[(size_t)L.no * L.stride] = (uint16_t)run;
+        }
+        return;
+    }
+    uint32_t place[ROWS];   // piece and rank within the wave
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) {
+        const bool in = c0 + r * MX_OS_SPLIT + t < a.n;
+        const int k = in ? index_of(ord[r]) : -1;
+        place[r] = 0xffffffffu;
+        if (k >= 0) {
+            int key = k;
+            if (VALUES) {
+                const bool counted = isfinite(val[r]) && (!filter || pr[r] > 0.0);
+                key = k * (bins + 1) + (counted ? bin_of(edges + k * bins, bins, val[r]) : bins);
+            }
+            const int sh = (key & 1) * 16;
+            const uint32_t old = atomicAdd(mine + (key >> 1), 1u << sh);
+            place[r] = ((uint32_t)key << 16) | ((old >> sh) & 0xffffu);
+        }
+    }
     __syncthreads();
-    if (t == 0) {
-        int64_t run = 0, cc = 0;
-        double ps = 0.0;
-        for (int j = 0; j < MX_OS_SCAN; ++j) {
-            const int64_t x = sv[j];
-            sv[j] = run;
+    // piece starts: counts over the waves, then a scan over the pieces
+    const int per = (keys + MX_OS_SPLIT - 1) / MX_OS_SPLIT, j0 = t * per;
+    int sum = 0;
+    for (int j = j0; j < j0 + per && j < keys; ++j) {
+        int run = 0;
+        for (int q = 0; q < MX_OS_SPLIT_WAVES; ++q) {
+            const int x = hist[q * kh + j];
+            hist[q * kh + j] = (uint16_t)run;
             run += x;
-            cc += sc[j];
-            ps += ss[j];
         }
-        a.prob_sum[k] = ps;
-        a.count[k] = cc;
-        tot[k] = run;
+        start[j] = (uint16_t)run;
+        sum += run;
+    }
+    int inc = sum;
+    for (int d = 1; d < 64; d <<= 1) {
+        const int o = __shfl_up(inc, d);
+        if (lane >= d) inc += o;
+    }
+    if (lane == 63) wtot[w] = inc;
+    __syncthreads();
+    int run = inc - sum;
+    for (int q = 0; q < w; ++q) run += wtot[q];
+    for (int j = j0; j < j0 + per && j < keys; ++j) {
+        const int x = start[j];
+        start[j] = (uint16_t)run;
+        run += x;
+    }
+    if (t == MX_OS_SPLIT - 1) start[keys] = (uint16_t)run;
+    __syncthreads();
+    // (a row per piece: who reads a bin's offsets reads consecutive words)
+    for (int j = t; j <= keys; j += MX_OS_SPLIT) off[(size_t)j * L.stride] = start[j];
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r)
+        if (place[r] != 0xffffffffu) {
+            const int key = place[r] >> 16;
+            place[r] = (place[r] & 0xffffu) + start[key] + hist[w * kh + key];
+            if (VALUES) buf[place[r]] = val[r];
+        }
+    if (VALUES) {
+        __syncthreads();
+        double *out = (double *)(ws + L.vals) + (size_t)c * CH;
+        const int all = start[keys];
+        for (int j = t; j < all; j += MX_OS_SPLIT) out[j] = buf[j];
+        double2 *piece = (double2 *)(ws + L.piece) + (size_t)c * L.no * bins;
+        for (int j = t; j < L.no * bins; j += MX_OS_SPLIT) {
+            const int k = j / bins, b = j - k * bins, e = start[j + k + 1];
+            const double ref = bin_ref(edges + k * bins, bins, b);
+            double2 p = make_double2(0.0, 0.0);
+#pragma unroll 4
+            for (int q = start[j + k]; q < e; ++q) {
+                const double d = buf[q] - ref;
+                p.x += d;
+                p.y += d * d;
+            }
+            piece[j] = p;
+        }
+        __syncthreads();
+    }
+    // probabilities in the same places; each order's run summed by one wave,
+    // or by all of them when there are fewer orders than waves
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r)
+        if (place[r] != 0xffffffffu) buf[place[r]] = pr[r];
+    __syncthreads();
+    const int parts = L.no < MX_OS_SPLIT_WAVES ? MX_OS_SPLIT_WAVES : 1;
+    for (int j = w; j < L.no * parts; j += MX_OS_SPLIT_WAVES) {
+        const int k = j / parts, b = start[k * (bins + 1)], e = start[(k + 1) * (bins + 1)];
+        double s = 0.0;
+#pragma unroll 4
+        for (int q = b + (j % parts) * 64 + lane; q < e; q += 64 * parts) s += buf[q];
+        for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
+        if (lane == 0) part[j] = s;
     }
     __syncthreads();
-    int64_t run = sv[t];
-    for (int64_t b = b0; b < b1; ++b) {
-        const size_t o = (size_t)b * no + k;
-        off_b[o] = run;
-        run += nval_b[o];
+    for (int k = t; k < L.no; k += MX_OS_SPLIT) {
+        double s = 0.0;
+        for (int j = 0; j < parts; ++j) s += part[k * parts + j];
+        psum[(size_t)k * L.chunks + c] = s;
     }
 }
 
-// Segment bounds: order k's values start after those of orders < k.
-__global__ void mx_os_seg_kernel(int no, const int64_t *tot, int32_t *seg) {
-    const int k = threadIdx.x;
-    if (k < no) {
-        int64_t start = 0;
-        for (int j = 0; j < k; ++j) start += tot[j];
-        seg[k] = (int32_t)start;
-        seg[no + k] = (int32_t)(start + tot[k]);
-    }
+// ----------------------------------------------------------------- 3 merge
+// Sums over the lanes up to each one, by the cross-lane moves of the vector
+// unit (a move through LDS costs ten times the latency).
+template <int CTRL, int ROWS> __device__ __forceinline__ double lane_move(double v) {
+    return __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, ROWS, 0xf, false),
+                            __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROWS, 0xf, false));
+}
+__device__ __forceinline__ double wave_scan(double v) {
+    v += lane_move<0x111, 0xf>(v);    // one lane up within 16
+    v += lane_move<0x112, 0xf>(v);
+    v += lane_move<0x114, 0xf>(v);
+    v += lane_move<0x118, 0xf>(v);
+    v += lane_move<0x142, 0xa>(v);    // the last lane of 16 to the next 16
+    v += lane_move<0x143, 0xc>(v);    // the last lane of 32 to the next 32
+    return v;
+}
+__device__ __forceinline__ double lane_value(double v, int lane) {
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                            __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
+// Sum over the wave in a fixed order; every lane gets it.
+__device__ __forceinline__ double wave_add(double v) { return lane_value(wave_scan(v), 63); }
+
+// Order-preserving integer of a finite double, and back.
+__device__ __forceinline__ uint64_t key_of(double x) {
+    const uint64_t u = (uint64_t)__double_as_longlong(x);
+    return u >> 63 ? ~u : u | 0x8000000000000000ull;
+}
+__device__ __forceinline__ double of_key(uint64_t k) {
+    return __longlong_as_double((long long)(k >> 63 ? k & 0x7fffffffffffffffull : ~k));
 }
 
-// Pass 3: values of each order into its segment (lane-ordered within a chunk).
-__global__ __launch_bounds__(MX_OS_WAVE) void mx_os_scatter_kernel(MxOrderStats a, int64_t chunk,
-                                                                    const int64_t *off_b, const int32_t *seg,
-                                                                    double *vals, uint8_t *ordk) {
-    extern __shared__ __align__(16) unsigned char sm[];
-    const int no = a.n_orders, lane = threadIdx.x;
-    int64_t *pos = (int64_t *)sm;                       // [no][64]
-    int *ords = (int *)(pos + no * MX_OS_WAVE);         // [no]
-    __shared__ int lut[MX_OS_LUT];
-    for (int k = 0; k < no; ++k) pos[k * MX_OS_WAVE + lane] = 0;
-    const OrderLut index_of = build_lut(a, ords, lut);
-    const int64_t b0 = (int64_t)blockIdx.x * chunk;
-    int64_t b1 = b0 + chunk;
-    if (b1 > a.n) b1 = a.n;
-    const bool filter = (a.flags & MX_OS_FILTER) != 0;
-    for (int64_t i0 = b0 + lane; i0 < b1; i0 += (int64_t)MX_OS_WAVE * MX_OS_LOADS) {
-        int ord[MX_OS_LOADS];
-        double pr[MX_OS_LOADS], val[MX_OS_LOADS];
+// The bin has room for one number only, its lower edge.
+__device__ __forceinline__ bool bin_single(const double *edges, int b) {
+    return b > 0 && key_of(edges[b]) == key_of(edges[b - 1]) + 1;
+}
+
+// The pieces of one bin, or of `span` consecutive ones, in all chunks.
+struct BinPieces {
+    const uint16_t *off;      // the bin's offset in chunk 0
+    const double *vals;
+    int64_t chunks, end;      // end: from there to the offset after the last bin
+    int chunk;
+    // f(x, place) for the values of the pieces of chunks group, group + groups,
+    // ..., of every piece those at sub, sub + per, ...; place: among the values
+    // of these pieces; MX_OS_PIECES pieces at a time, so that loads overlap
+    template <typename F>
+    __device__ __forceinline__ void each(int64_t group, int64_t groups, int sub, int per, F f) const {
+        int64_t run = 0;
+        for (int64_t c = group; c < chunks; c += MX_OS_PIECES * groups) {
+            int j[MX_OS_PIECES], m[MX_OS_PIECES], first[MX_OS_PIECES];
+            int64_t at[MX_OS_PIECES];
+            const double *v[MX_OS_PIECES];
 #pragma unroll
-        for (int u = 0; u < MX_OS_LOADS; ++u) {
-            const int64_t i = i0 + (int64_t)u * MX_OS_WAVE;
-            const bool in = i < b1;
-            ord[u] = in ? a.order[i] : INT32_MIN;
-            pr[u] = (in && filter) ? a.prob[i] : 1.0;
-            val[u] = in ? a.value[i] : 0.0;
-        }
+            for (int u = 0; u < MX_OS_PIECES; ++u) {
+                // (no load under a condition: its wait would stand in the
+                // branch, before the next load)
+                const int64_t x = c + u * groups < chunks ? c + u * groups : c;
+                first[u] = off[x];
+                m[u] = off[end + x];
+            }
 #pragma unroll
-        for (int u = 0; u < MX_OS_LOADS; ++u) {
-            if (i0 + (int64_t)u * MX_OS_WAVE >= b1) break;
-            const int k = index_of(ord[u]);
-            if (k >= 0 && isfinite(val[u]) && (!filter || pr[u] > 0.0)) pos[k * MX_OS_WAVE + lane] += 1;
-        }
-    }
-    __syncthreads();
-    // exclusive prefix over lanes, plus the chunk and segment offsets
-    for (int k = lane; k < no; k += MX_OS_WAVE) {
-        int64_t run = (int64_t)seg[k] + off_b[(size_t)blockIdx.x * no + k];
-        for (int l = 0; l < MX_OS_WAVE; ++l) {
-            const int64_t c = pos[k * MX_OS_WAVE + l];
-            pos[k * MX_OS_WAVE + l] = run;
-            run += c;
-        }
-    }
-    __syncthreads();
-    for (int64_t i0 = b0 + lane; i0 < b1; i0 += (int64_t)MX_OS_WAVE * MX_OS_LOADS) {
-        int ord[MX_OS_LOADS];
-        double pr[MX_OS_LOADS], val[MX_OS_LOADS];
+            for (int u = 0; u < MX_OS_PIECES; ++u) {
+                const int64_t x = c + u * groups;
+                m[u] = x < chunks ? m[u] - first[u] : 0;
+                v[u] = m[u] ? vals + (size_t)x * chunk + first[u] : vals;
+                j[u] = sub;
+                at[u] = run;
+                run += m[u];
+            }
+            for (;;) {
+                bool more = false;
+                double x[MX_OS_PIECES];
 #pragma unroll
-        for (int u = 0; u < MX_OS_LOADS; ++u) {
-            const int64_t i = i0 + (int64_t)u * MX_OS_WAVE;
-            const bool in = i < b1;
-            ord[u] = in ? a.order[i] : INT32_MIN;
-            pr[u] = (in && filter) ? a.prob[i] : 1.0;
-            val[u] = in ? a.value[i] : 0.0;
-        }
+                for (int u = 0; u < MX_OS_PIECES; ++u) {
+                    more |= j[u] < m[u];
+                    x[u] = v[u][j[u] < m[u] ? j[u] : 0];
+                }
+                if (!more) break;
 #pragma unroll
-        for (int u = 0; u < MX_OS_LOADS; ++u) {
-            if (i0 + (int64_t)u * MX_OS_WAVE >= b1) break;
-            const int k = index_of(ord[u]);
-            if (k >= 0 && isfinite(val[u]) && (!filter || pr[u] > 0.0)) {
-                const int64_t p = pos[k * MX_OS_WAVE + lane];
-                pos[k * MX_OS_WAVE + lane] = p + 1;
-                vals[p] = val[u];
-                ordk[p] = (uint8_t)k;
+                for (int u = 0; u < MX_OS_PIECES; ++u) {
+                    if (j[u] < m[u]) f(x[u], at[u] + j[u]);
+                    j[u] += per;
+                }
             }
         }
     }
+};
+
+__device__ __forceinline__ BinPieces pieces_of(const OsPlan &L, const unsigned char *ws, int k, int b, int span) {
+    return {(const uint16_t *)(ws + L.off) + (k * (L.bins + 1) + b) * L.stride, (const double *)(ws + L.vals), L.chunks,
+            span * L.stride, L.chunk};
 }
 
-// Items [end of the last segment, n) of the sort input: value +inf, order
-// index 255 (past any order), so that both sorts leave them at the end.
-__global__ void mx_os_tail_kernel(const int32_t *last_end, int64_t n, double *vals, uint8_t *ordk) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n && i >= (int64_t)last_end[0]) {
-        vals[i] = __builtin_inf();
-        ordk[i] = 255;
-    }
+// Work-items per piece of m values on average: the power of two above it.
+__device__ __forceinline__ int items_per_piece(int64_t values, int64_t chunks, int most) {
+    int per = 1;
+    while (per < most && values > chunks * per) per *= 2;
+    return per;
 }
 
-// sum of f(x[j]) over [lo, hi) by the whole workgroup (fixed order: lane
-// strides, then a tree in LDS); every work-item gets the result.
-template <typename F>
-__device__ __forceinline__ double block_sum(const double *x, int64_t lo, int64_t hi, double *red, F f) {
-    // MX_OS_UNROLL independent accumulators per work-item, each over its own
-    // stride of the range, added in a fixed order
-    double acc[MX_OS_UNROLL];
-#pragma unroll
-    for (int u = 0; u < MX_OS_UNROLL; ++u) acc[u] = 0.0;
-    const int64_t step = (int64_t)MX_OS_CLIP * MX_OS_UNROLL;
-    int64_t j = lo + threadIdx.x;
-    for (; j + (MX_OS_UNROLL - 1) * MX_OS_CLIP < hi; j += step) {
-        double v[MX_OS_UNROLL];
-#pragma unroll
-        for (int u = 0; u < MX_OS_UNROLL; ++u) v[u] = x[j + (int64_t)u * MX_OS_CLIP];
-#pragma unroll
-        for (int u = 0; u < MX_OS_UNROLL; ++u) acc[u] += f(v[u]);
-    }
-    for (; j < hi; j += MX_OS_CLIP) acc[0] += f(x[j]);
-    double s = 0.0;
-#pragma unroll
-    for (int u = 0; u < MX_OS_UNROLL; ++u) s += acc[u];
-    red[threadIdx.x] = s;
-    __syncthreads();
-    for (int w = MX_OS_CLIP / 2; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-        __syncthreads();
-    }
-    const double r = red[0];
-    __syncthreads();
-    return r;
-}
-
-// First index j in [lo, hi) with pred(x[j]) (pred false, then true, along
-// the sorted range), or hi; by the whole workgroup: each round every
-// work-item tests one of MX_OS_CLIP evenly spaced probes and the range
-// shrinks to the gap before the first true probe (the same answer as a
-// binary search, in log_1024 rounds of parallel loads instead of log_2
-// dependent ones).
-template <typename F>
-__device__ __forceinline__ int64_t block_first(const double *x, int64_t lo, int64_t hi, int *s_t, F pred) {
+// How a workgroup of NT work-items shares the pieces: `per` of them on a piece,
+// this one on the pieces of chunks group, group + NT / per, ..., whose values
+// follow those of the groups before (`first` of them; `all` in total).
+struct Share {
+    int per, sub, group, first, all;
+};
+template <int NT> __device__ __forceinline__ Share share_pieces(const BinPieces &P, int *s_first, int *s_wave) {
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+    Share H = {1, 0, t, 0, 0};
+    // counted by a work-item per piece, and again when pieces are longer
     for (;;) {
-        const int64_t n = hi - lo;
-        if (n <= 0) return lo;
-        const int64_t step = n <= MX_OS_CLIP ? 1 : (n + MX_OS_CLIP - 1) / MX_OS_CLIP;
-        const int64_t j = lo + (int64_t)threadIdx.x * step;
-        if (threadIdx.x == 0) *s_t = MX_OS_CLIP;
+        const int groups = NT / H.per;
+        int n = 0;
+        if (H.sub == 0)
+#pragma unroll 8
+            for (int64_t c = H.group; c < P.chunks; c += groups) n += (int)P.off[P.end + c] - (int)P.off[c];
+        int inc = n;
+        for (int d = 1; d < 64; d <<= 1) {
+            const int o = __shfl_up(inc, d);
+            if (lane >= d) inc += o;
+        }
         __syncthreads();
-        if (j < hi && pred(x[j])) atomicMin(s_t, (int)threadIdx.x);
+        if (lane == 63) s_wave[w] = inc;
         __syncthreads();
-        const int t = *s_t;
+        int before = inc - n;
+        H.all = 0;
+        for (int q = 0; q < NT / 64; ++q) {
+            if (q < w) before += s_wave[q];
+            H.all += s_wave[q];
+        }
+        if (H.sub == 0) s_first[H.group] = before;
+        const int per = items_per_piece(H.all, P.chunks, NT);
+        if (H.per > 1 || per == 1) break;
+        H.per = per;
+        H.sub = t & (per - 1);
+        H.group = t / per;
+    }
+    __syncthreads();
+    H.first = s_first[H.group];
+    return H;
+}
+
+// Workgroups 0 .. groups-1 of an order add up a group of chunks: work-item t
+// its share of bin t % bins, the shares joined in LDS in a fixed order.  The
+// others copy one bin each to one place: those at the ends, where the bounds of a
+// single-peaked order lie, and those around the middle, where its median lies
+// (3 % of an order's photons is the error of the middle of 270 samples).  A
+// bin's pieces lie in as many places as there are chunks: left there, the
+// clipping workgroup needed 22 us for every look into a bin at 8e6 photons.
+// Copying all bins took 88 us; this kernel takes 26 us.
+__global__ __launch_bounds__(MX_OS_MERGE) void mx_os_merge_kernel(OsPlan L, unsigned char *ws) {
+    __shared__ double red[3][MX_OS_MERGE];
+    __shared__ int s_first[MX_OS_MERGE], s_wave[MX_OS_MERGE / 64];
+    __shared__ long long base;
+    const int t = threadIdx.x, k = blockIdx.y;
+    const int bins = L.bins;
+    if ((int)blockIdx.x < L.groups) {
+        const int b = t % bins, sub = t / bins, subs = MX_OS_MERGE / bins;
+        const int64_t per = (L.chunks + L.groups - 1) / L.groups;
+        const int64_t c0 = blockIdx.x * per, c1 = c0 + per < L.chunks ? c0 + per : L.chunks;
+        const BinPieces P = pieces_of(L, ws, k, b, 1);
+        const double2 *piece = (const double2 *)(ws + L.piece) + (size_t)k * bins + b;
+        double n = 0.0, s1 = 0.0, s2 = 0.0;
+#pragma unroll 4
+        for (int64_t c = c0 + sub; c < c1; c += subs) {
+            const double2 p = piece[(size_t)c * L.no * bins];
+            n += (double)((int)P.off[P.end + c] - (int)P.off[c]);
+            s1 += p.x;
+            s2 += p.y;
+        }
+        red[0][t] = n;
+        red[1][t] = s1;
+        red[2][t] = s2;
         __syncthreads();
-        if (step == 1) return t < MX_OS_CLIP ? lo + t : hi;
-        if (t == 0) return lo;
-        if (t < MX_OS_CLIP) {
-            hi = lo + (int64_t)t * step;                 // pred true here
-            lo = lo + (int64_t)(t - 1) * step + 1;       // false at the probe before
+        if (sub == 0) {
+            for (int q = t + bins; q < subs * bins; q += bins) {
+                n += red[0][q];
+                s1 += red[1][q];
+                s2 += red[2][q];
+            }
+            ((BinInfo *)(ws + L.grp))[((size_t)k * L.groups + blockIdx.x) * bins + b] = {0, n, s1, s2};
+        }
+        return;
+    }
+    const int j = (int)blockIdx.x - L.groups;
+    const int b = j < MX_OS_ENDS ? j : (j < 2 * MX_OS_ENDS ? bins - 1 - (j - MX_OS_ENDS)
+                                                           : bins / 2 - MX_OS_NEAR / 2 + (j - 2 * MX_OS_ENDS));
+    if (j >= 2 * MX_OS_ENDS && (b < MX_OS_ENDS || b >= bins - MX_OS_ENDS)) return;
+    if (bin_single((const double *)(ws + L.edges) + (size_t)k * bins, b)) return;
+    const BinPieces P = pieces_of(L, ws, k, b, 1);
+    const Share H = share_pieces<MX_OS_MERGE>(P, s_first, s_wave);
+    if (t == 0) {
+        base = (long long)atomicAdd((unsigned long long *)(ws + L.next), (unsigned long long)H.all);
+        ((int64_t *)(ws + L.place))[(size_t)k * bins + b] = base;
+    }
+    __syncthreads();
+    double *out = (double *)(ws + L.copied) + base + H.first;
+    P.each(H.group, MX_OS_MERGE / H.per, H.sub, H.per, [&](double x, int64_t at) { out[at] = x; });
+}
+
+// ------------------------------------------------------------------ 4 clip
+// What the clipping workgroup of one order works on.
+struct ClipOrder {
+    const OsPlan &L;
+    const unsigned char *ws;
+    int k, bins;
+    const double *edges;      // LDS
+    const BinInfo *info;      // LDS
+    // f(x) for every value of bin b, by the `nth` work-items tid = 0, 1, ...
+    template <typename F> __device__ __forceinline__ void each(int b, int tid, int nth, F f) const {
+        const int64_t n = (int64_t)info[b].n;
+        if (info[b].at >= 0) {
+            const double *x = (const double *)(ws + L.copied) + info[b].at;
+            for (int64_t j = tid; j < n; j += 8 * nth) {
+                double v[8];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) v[u] = x[j + u * nth < n ? j + u * nth : j];
+#pragma unroll
+                for (int u = 0; u < 8; ++u)
+                    if (j + u * nth < n) f(v[u]);
+            }
         } else {
-            lo = lo + (n - 1) / step * step + 1;         // after the last probe (false)
+            const int per = items_per_piece(n, L.chunks, nth);
+            pieces_of(L, ws, k, b, 1).each(tid / per, nth / per, tid & (per - 1), per, [&](double x, int64_t) { f(x); });
+        }
+    }
+    __device__ __forceinline__ bool single(int b) const { return bin_single(edges, b); }
+    // bin of x, by the wave: the number of edges <= x
+    __device__ __forceinline__ int bin_of(double x) const {
+        int n = 0;
+        for (int b0 = 0; b0 < bins - 1; b0 += 64) {
+            const int b = b0 + (int)(threadIdx.x & 63);
+            n += __popcll(__ballot(b < bins - 1 && edges[b] <= x));
+        }
+        return n;
+    }
+};
+
+// LDS of the clipping kernel: bins, edges, list.
+static size_t clip_lds(const OsPlan &L) {
+    return (sizeof(double) + sizeof(BinInfo)) * (size_t)L.bins + sizeof(double) * MX_OS_LIST;
+}
+
+#define MX_OS_CW (MX_OS_CLIP / 64)
+#define MX_OS_HALF (MX_OS_CLIP / 2)
+
+// n and the sums of deviations and their squares over the kept values of a
+// cut bin.
+struct CutSums {
+    double n, s1, s2;
+};
+struct ClipShared {
+    double cand[2][MX_OS_CAND];
+    CutSums part[2][MX_OS_CW];
+    double below[2][MX_OS_CW];
+    uint64_t kmin, kmax;
+    unsigned pre[MX_OS_HIST + 1];
+    int iw[MX_OS_CW], n[2], m, first[MX_OS_CLIP];
+};
+
+// The kept interval: bins bl .. bh, of which bl and bh count only their values
+// in [lo, hi] when `cut` (bl == bh: all of it in c0); all bins fully otherwise.
+struct Kept {
+    int bl, bh;
+    bool cut;
+    double lo, hi;
+    CutSums c0, c1;
+    __device__ __forceinline__ double count(const ClipOrder &O, int b) const {
+        if (b < bl || b > bh) return 0.0;
+        if (!cut) return O.info[b].n;
+        return b == bl ? c0.n : (b == bh ? c1.n : O.info[b].n);
+    }
+    __device__ __forceinline__ bool partial(int b) const { return cut && (b == bl || b == bh); }
+    __device__ __forceinline__ bool has(double x) const { return !cut || (x >= lo && x <= hi); }
+};
+
+// The next three are computed by every wave for itself from the bins in LDS,
+// which costs less than a barrier.
+__device__ __forceinline__ double kept_count(const ClipOrder &O, const Kept &K) {
+    double n = 0.0;
+    for (int b = threadIdx.x & 63; b < O.bins; b += 64) n += K.count(O, b);
+    return wave_add(n);
+}
+
+// Bin of rank r (from 0) of the kept values and the rank of its first value.
+__device__ __forceinline__ void find_bin(const ClipOrder &O, const Kept &K, int64_t r, int &bin, int64_t &first) {
+    const int lane = threadIdx.x & 63, per = (O.bins + 63) / 64, b0 = lane * per;
+    double s = 0.0;
+    for (int b = b0; b < b0 + per && b < O.bins; ++b) s += K.count(O, b);
+    double run = wave_scan(s) - s, at = 0.0;
+    int mine = -1;
+    for (int b = b0; b < b0 + per && b < O.bins; ++b) {
+        const double x = K.count(O, b);
+        if ((double)r >= run && (double)r < run + x) {
+            mine = b;
+            at = run;
+        }
+        run += x;
+    }
+    const int src = __ffsll((unsigned long long)__ballot(mine >= 0)) - 1;
+    bin = __builtin_amdgcn_readlane(mine, src);
+    first = (int64_t)lane_value(at, src);
+}
+
+// Mean and standard deviation of the N kept values: sums of deviations from
+// their median c or that of the round before (|mean - median| is at most one
+// standard deviation, so nothing cancels); the sums of the cut bins are about
+// the same c (all: they are the sums of all kept values).
+__device__ __forceinline__ void kept_moments(const ClipOrder &O, const Kept &K, double N, double c, bool all,
+                                             double &mean, double &sd) {
+    double s1 = 0.0, s2 = 0.0;
+    for (int b = threadIdx.x & 63; b < O.bins && !all; b += 64) {
+        if (b < K.bl || b > K.bh || K.partial(b) || O.info[b].n == 0.0) continue;
+        const BinInfo f = O.info[b];
+        const double r = bin_ref(O.edges, O.bins, b) - c;
+        s1 += f.s1 + f.n * r;
+        s2 += f.s2 + r * (2.0 * f.s1 + f.n * r);
+    }
+    s1 = wave_add(s1);
+    s2 = wave_add(s2);
+    if (K.cut) {
+        s1 += K.c0.s1 + K.c1.s1;
+        s2 += K.c0.s2 + K.c1.s2;
+    }
+    const double m = s1 / N;
+    mean = c + m;
+    const double sq = s2 / N, var = sq - m * m;
+    sd = isinf(sq) ? sq : sqrt(var > 0.0 || var != var ? var : 0.0);   // var: >= 0 up to rounding
+}
+
+// Values of ranks r and r + 1 among the cnt <= 64 candidates of S.cand[p],
+// whose first has rank `base`; by every wave for itself, one per lane.
+__device__ __forceinline__ void rank_candidates(const ClipShared &S, int p, int cnt, int64_t base, int64_t r,
+                                                double &x0, double &x1) {
+    const int lane = threadIdx.x & 63;
+    const double x = S.cand[p][lane < cnt ? lane : 0];
+    const uint64_t kx = key_of(x);
+    const unsigned lo = (unsigned)kx, hi = (unsigned)(kx >> 32);
+    int rank = 0;
+    for (int j = 0; j < cnt; ++j) {
+        const uint64_t kj = (uint64_t)(unsigned)__builtin_amdgcn_readlane((int)lo, j) |
+                            ((uint64_t)(unsigned)__builtin_amdgcn_readlane((int)hi, j) << 32);
+        rank += (kj < kx || (kj == kx && j < lane)) ? 1 : 0;
+    }
+    const unsigned long long m0 = __ballot(lane < cnt && base + rank == r);
+    const unsigned long long m1 = __ballot(lane < cnt && base + rank == r + 1);
+    if (m0) x0 = lane_value(x, __ffsll(m0) - 1);
+    if (m1) x1 = lane_value(x, __ffsll(m1) - 1);
+}
+
+// The buckets of S.pre scanned: S.pre[j] becomes the number of values in the
+// buckets before j, S.pre[MX_OS_HIST] that of all.
+__device__ __forceinline__ void scan_buckets(ClipShared &S) {
+    constexpr int PER = MX_OS_HIST / MX_OS_CLIP;
+    const int t = threadIdx.x;
+    unsigned h[PER], sum = 0;
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+        h[u] = S.pre[PER * t + u];
+        sum += h[u];
+    }
+    unsigned inc = sum;
+    for (int d = 1; d < 64; d <<= 1) {
+        const unsigned o = __shfl_up(inc, d);
+        if ((t & 63) >= d) inc += o;
+    }
+    if ((t & 63) == 63) S.iw[t >> 6] = (int)inc;
+    __syncthreads();
+    unsigned run = inc - sum;
+    for (int q = 0; q < (t >> 6); ++q) run += (unsigned)S.iw[q];
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+        S.pre[PER * t + u] = run;
+        run += h[u];
+    }
+    if (t == MX_OS_CLIP - 1) S.pre[MX_OS_HIST] = run;
+    __syncthreads();
+}
+
+// The workgroup's least and greatest integer into S.kmin and S.kmax, which
+// hold ~0 and 0 before.
+__device__ __forceinline__ void key_range(ClipShared &S, uint64_t mn, uint64_t mx) {
+    for (int o = 32; o > 0; o >>= 1) {
+        const uint64_t u = __shfl_xor(mn, o), v = __shfl_xor(mx, o);
+        mn = u < mn ? u : mn;
+        mx = v > mx ? v : mx;
+    }
+    if ((threadIdx.x & 63) == 0) {
+        atomicMin((unsigned long long *)&S.kmin, (unsigned long long)mn);
+        atomicMax((unsigned long long *)&S.kmax, (unsigned long long)mx);
+    }
+    __syncthreads();
+}
+
+// Kept values of bin b into the list (when n of them fit) with their least
+// and greatest integers.
+__device__ __forceinline__ void load_bin(const ClipOrder &O, const Kept &K, int b, bool part, bool fits, ClipShared &S,
+                                         double *list) {
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        S.m = 0;
+        S.kmin = ~0ull;
+        S.kmax = 0;
+    }
+    __syncthreads();
+    uint64_t mn = ~0ull, mx = 0;
+    O.each(b, threadIdx.x, MX_OS_CLIP, [&](double x) {
+        if (part && !K.has(x)) return;
+        const uint64_t k = key_of(x);
+        mn = k < mn ? k : mn;
+        mx = k > mx ? k : mx;
+        if (fits) list[atomicAdd(&S.m, 1)] = x;
+    });
+    key_range(S, mn, mx);
+}
+
+// Shift that maps [0, span] to the MX_OS_HIST buckets.
+__device__ __forceinline__ int bucket_shift(uint64_t span) {
+    const int bits = span ? 64 - __clzll((long long)span) : 0;
+    return bits > 11 ? bits - 11 : 0;
+}
+
+// Bucket of rank r, by the wave: the last j with S.pre[j] <= r.
+__device__ __forceinline__ int bucket_of(const ClipShared &S, unsigned r) {
+    constexpr int PER = MX_OS_HIST / 64;      // 32: the second look takes half the lanes
+    const int lane = threadIdx.x & 63;
+    const int g = __popcll(__ballot(S.pre[lane * PER] <= r)) - 1;
+    return g * PER + __popcll(__ballot(lane < PER && S.pre[g * PER + (lane & (PER - 1))] <= r)) - 1;
+}
+
+#define MX_OS_ALL (-2)
+
+// State of the list between medians: the uncut bin that the list holds (-1:
+// none; MX_OS_ALL: every value of the order, n of them), whether S.pre holds
+// its buckets, its least and greatest integers, the candidate buffer next to
+// use; buckets of a bin are equal steps of 1 / inv from x0.
+struct Held {
+    int bin;
+    bool buckets;
+    int p;
+    int64_t n;
+    uint64_t kmin, kmax;
+    double x0, inv;
+    __device__ __forceinline__ void steps(double a, double b, int n) {
+        x0 = a;
+        inv = b > a && !isinf(b - a) ? n / (b - a) : 0.0;
+        if (isinf(inv)) inv = 0.0;
+    }
+    __device__ __forceinline__ int step(double x, int n) const {
+        const int j = (int)((x - x0) * inv);
+        return j < 0 ? 0 : (j < n ? j : n - 1);
+    }
+    // of a whole order: equal steps within each bin, so that an order of a
+    // narrow line and values far from it still fills them evenly
+    __device__ __forceinline__ int bucket(const ClipOrder &O, double x) {
+        if (bin != MX_OS_ALL) return step(x, MX_OS_HIST);
+        const int b = ::bin_of(O.edges, O.bins, x), per = MX_OS_HIST / O.bins;
+        if (b == 0 || b == O.bins - 1) return b * per;
+        steps(O.edges[b - 1], O.edges[b], per);
+        return b * per + step(x, per);
+    }
+};
+
+// The kept values of bin b of ranks r and r + 1 (from 0, r + 1 only when
+// `two`), exactly.  An uncut bin that fits the list is loaded and counted into
+// buckets once; every further median in it takes one pass over the list, for
+// the values of one or two buckets, and one barrier.  Otherwise (a cut bin, one
+// larger than the list, or one with a crowded bucket) buckets of the values'
+// order-preserving integers narrow them down until few are left.
+__device__ __forceinline__ void select_in_bin(const ClipOrder &O, const Kept &K, int b, int64_t r, bool two,
+                                              ClipShared &S, double *list, Held &H, double &x0, double &x1) {
+    const int t = threadIdx.x;
+    const bool all = b == MX_OS_ALL;
+    if (!all && O.single(b)) {
+        x0 = x1 = O.edges[b - 1];
+        return;
+    }
+    const bool part = !all && K.partial(b);
+    const int64_t n = all ? H.n : (int64_t)K.count(O, b);
+    const bool fits = n <= MX_OS_LIST;
+    if (H.bin != b || part) {
+        load_bin(O, K, b, part, fits, S, list);
+        H.bin = fits && !part ? b : -1;
+        H.buckets = false;
+        H.kmin = S.kmin;
+        H.kmax = S.kmax;
+        H.steps(of_key(H.kmin), of_key(H.kmax), MX_OS_HIST);
+    }
+    uint64_t klo = H.kmin, khi = H.kmax;
+    int64_t cnt = n, below = 0;     // values in [klo, khi], and before it
+    // mode 0: count into buckets of integers; 1: collect the values of
+    // [klo, khi]; 2: the least integer above khi; 3: count into the buckets
+    // that are kept; 4: they are there
+    int mode = n <= MX_OS_CAND ? 1 : (H.buckets ? 4 : (H.bin == b ? 3 : 0));
+    for (;;) {
+        const int shift = bucket_shift(khi - klo);
+        if (mode != 4) {
+            __syncthreads();
+            if (mode == 0 || mode == 3) {
+                for (int j = t; j < MX_OS_HIST; j += MX_OS_CLIP) S.pre[j] = 0;
+                if (t < 2) S.n[t] = 0;
+            } else if (t == 0) {
+                S.m = 0;
+                S.kmin = ~0ull;
+            }
+            __syncthreads();
+            uint64_t mn = ~0ull;
+            auto f = [&](double x) {
+                const uint64_t k = key_of(x);
+                if (mode == 2) {
+                    if (k > khi && k < mn) mn = k;
+                } else if (mode == 3) {
+                    atomicAdd(&S.pre[H.bucket(O, x)], 1u);
+                } else if (k >= klo && k <= khi) {
+                    if (mode == 0) atomicAdd(&S.pre[(k - klo) >> shift], 1u);
+                    else S.cand[0][atomicAdd(&S.m, 1)] = x;
+                }
+            };
+            if (fits) {
+                for (int j = t; j < (int)n; j += MX_OS_CLIP) f(list[j]);
+            } else {
+                O.each(b, t, MX_OS_CLIP, [&](double x) { if (!part || K.has(x)) f(x); });
+            }
+            if (mode == 2) {
+                for (int o = 32; o > 0; o >>= 1) {
+                    const uint64_t u = __shfl_xor(mn, o);
+                    mn = u < mn ? u : mn;
+                }
+                if ((t & 63) == 0) atomicMin((unsigned long long *)&S.kmin, (unsigned long long)mn);
+            }
+            __syncthreads();
+            if (mode == 2) {
+                x1 = of_key(S.kmin);
+                break;
+            }
+            if (mode == 1) {
+                rank_candidates(S, 0, (int)cnt, below, r, x0, x1);
+                if (!two || r + 1 < below + cnt) break;
+                mode = 2;
+                continue;
+            }
+            scan_buckets(S);
+        }
+        const int64_t q = r - below;
+        const int j0 = bucket_of(S, (unsigned)q);
+        if (mode >= 3) {
+            H.buckets = true;
+            const int j1 = two ? bucket_of(S, (unsigned)q + 1) : j0;
+            const int c = (int)(S.pre[j0 + 1] - S.pre[j0]) + (j1 != j0 ? (int)(S.pre[j1 + 1] - S.pre[j1]) : 0);
+            if (c <= MX_OS_CAND) {
+                const int p = H.p;
+                double lo = -__builtin_inf(), hi = __builtin_inf();
+                if (all) {
+                    const int per = MX_OS_HIST / O.bins, b0 = j0 / per, b1 = j1 / per;
+                    if (b0 > 0) lo = O.edges[b0 - 1];
+                    if (b1 < O.bins - 1) hi = O.edges[b1];
+                }
+                for (int j = t; j < (int)n; j += MX_OS_CLIP) {
+                    const double x = list[j];
+                    if (!(x >= lo && x <= hi)) continue;
+                    const int u = H.bucket(O, x);
+                    if (u == j0 || u == j1) S.cand[p][atomicAdd(&S.n[p], 1)] = x;
+                }
+                __syncthreads();
+                // the other buffer's last readers passed this barrier
+                if (t == 0) S.n[p ^ 1] = 0;
+                H.p = p ^ 1;
+                rank_candidates(S, p, c, S.pre[j0], r, x0, x1);
+                break;
+            }
+            H.buckets = false;      // the narrowing uses S.pre for its own
+            mode = 0;
+            continue;
+        }
+        cnt = (int64_t)(S.pre[j0 + 1] - S.pre[j0]);
+        below += S.pre[j0];
+        klo += (uint64_t)j0 << shift;
+        if (khi - klo > (1ull << shift) - 1) khi = klo + ((1ull << shift) - 1);
+        mode = cnt > MX_OS_CAND ? 0 : 1;
+        if (klo == khi) {
+            x0 = x1 = of_key(klo);
+            if (!two || r + 1 < below + cnt) break;
+            mode = 2;
         }
     }
 }
 
-__device__ __forceinline__ double median_sorted(const double *x, int64_t lo, int64_t hi) {
-    const int64_t m = hi - lo;
-    if (m & 1) return x[lo + m / 2];
-    return (x[lo + m / 2 - 1] + x[lo + m / 2]) / 2;
+// Median of the N > 0 kept values (below: the values under them, when the list
+// holds all).
+__device__ __forceinline__ double kept_median(const ClipOrder &O, const Kept &K, int64_t N, int64_t below,
+                                              ClipShared &S, double *list, Held &H) {
+    const int64_t r = (N - 1) / 2;
+    const bool two = !(N & 1);
+    double lower = 0.0;
+    // the upper middle value may be the least of a later bin
+    for (int u = 0;; ++u) {
+        int b = MX_OS_ALL;
+        int64_t first = -below;
+        if (H.bin != MX_OS_ALL) find_bin(O, K, r + u, b, first);
+        const bool both = two && u == 0 && (b == MX_OS_ALL || r + 1 < first + (int64_t)K.count(O, b));
+        double x0 = 0.0, x1 = 0.0;
+        select_in_bin(O, K, b, r + u - first, both, S, list, H, x0, x1);
+        __syncthreads();
+        if (!two) return x0;
+        if (both) return (x0 + x1) / 2;
+        if (u == 1) return (lower + x0) / 2;
+        lower = x0;
+    }
 }
 
-// Pass 5: sigma clipping of each sorted segment.  Every clipping round keeps
-// a contiguous range, so a round is: the sum of the values over the range,
-// then the sum of squared deviations from their mean (each by MX_OS_CW
-// workgroups per order over consecutive parts of the range, partial sums
-// added in part order), then, one workgroup per order, the median, the new
-// bounds and the state for the next round.  Rounds are launched up to
-// maxiters times; orders that are done return at once.
-__global__ void mx_os_clip_init_kernel(int no, const int32_t *seg, ClipState *cs) {
-    const int k = threadIdx.x;
-    if (k >= no) return;
-    ClipState c;
-    c.lo = seg[k];
-    c.hi = seg[no + k];
-    c.med = c.mean = c.sd = __builtin_nan("");
-    c.done = c.hi == c.lo;
-    c.have = 0;
-    cs[k] = c;
-}
-
-// pass 0: partial sums of x; pass 1: partial sums of (x - mean)^2, mean from
-// pass 0's partials.  final: the passes after the last round, for orders
-// whose statistics are not yet final.
-__global__ __launch_bounds__(MX_OS_CLIP) void mx_os_clip_sum_kernel(const ClipState *cs, const double *x,
-                                                                     double *p0, double *p1, int pass,
-                                                                     int final) {
-    __shared__ double red[MX_OS_CLIP];
-    const int k = blockIdx.x / MX_OS_CW, w = blockIdx.x % MX_OS_CW;
-    const ClipState c = cs[k];
-    if (final ? (c.have || c.hi == c.lo) : c.done) return;
-    const int64_t m = c.hi - c.lo;
-    const int64_t b = c.lo + m * w / MX_OS_CW, e = c.lo + m * (w + 1) / MX_OS_CW;
-    double s;
-    if (pass == 0) {
-        s = block_sum(x, b, e, red, [](double v) { return v; });
+// Count, sum and squares about c of the kept values of the cut bins: the first
+// half of the waves takes bin bl, the second bin bh (none when they are the
+// same).  With every value in the list (nlist of them, else -1): of all kept values,
+// with the number below lo.
+__device__ __forceinline__ void cut_bins(const ClipOrder &O, Kept &K, double c, ClipShared &S, int p,
+                                         const double *list, int nlist, double &below) {
+    const int t = threadIdx.x, half = t / MX_OS_HALF, th = t % MX_OS_HALF;
+    const int b = half ? K.bh : K.bl;
+    CutSums a = {0.0, 0.0, 0.0};
+    auto add = [&](double x) {
+        if (!K.has(x)) return;
+        const double d = x - c;
+        a.n += 1.0;
+        a.s1 += d;
+        a.s2 += d * d;
+    };
+    below = 0.0;
+    if (nlist >= 0) {
+        for (int j = t; j < nlist; j += MX_OS_CLIP) {
+            add(list[j]);
+            below += list[j] < K.lo ? 1.0 : 0.0;
+        }
+        below = wave_add(below);
+    } else if (half && K.bl == K.bh) {
+    } else if (O.single(b)) {
+        if (th == 0 && O.info[b].n > 0.0 && K.has(O.edges[b - 1])) {
+            const double d = O.edges[b - 1] - c;
+            a.n = O.info[b].n;
+            a.s1 = a.n * d;
+            a.s2 = a.n * (d * d);
+        }
     } else {
-        double t = 0.0;
-        for (int q = 0; q < MX_OS_CW; ++q) t += p0[k * MX_OS_CW + q];
-        const double mean = t / (double)m;
-        s = block_sum(x, b, e, red, [mean](double v) { const double d = v - mean; return d * d; });
+        O.each(b, th, MX_OS_HALF, add);
     }
-    if (threadIdx.x == 0) (pass == 0 ? p0 : p1)[k * MX_OS_CW + w] = s;
-}
-
-__device__ __forceinline__ void clip_moments(const double *p0, const double *p1, int k, int64_t m,
-                                             double &mean, double &sd) {
-    double t0 = 0.0, t1 = 0.0;
-    for (int q = 0; q < MX_OS_CW; ++q) t0 += p0[k * MX_OS_CW + q];
-    for (int q = 0; q < MX_OS_CW; ++q) t1 += p1[k * MX_OS_CW + q];
-    mean = t0 / (double)m;
-    sd = sqrt(t1 / (double)m);
-}
-
-__global__ __launch_bounds__(MX_OS_CLIP) void mx_os_clip_bounds_kernel(MxOrderStats a, ClipState *cs,
-                                                                        const double *x, const double *p0,
-                                                                        const double *p1) {
-    __shared__ int s_t;
-    const int k = blockIdx.x;
-    const ClipState c = cs[k];
-    if (c.done) return;
-    const int64_t m = c.hi - c.lo;
-    double mean, sd;
-    clip_moments(p0, p1, k, m, mean, sd);
-    const double cen = median_sorted(x, c.lo, c.hi);
-    const double vmin = cen - sd * a.sigma;
-    const double vmax = cen + sd * a.sigma;
-    // first index with x >= vmin, then first index with x > vmax
-    const int64_t nlo = block_first(x, c.lo, c.hi, &s_t, [vmin](double v) { return v >= vmin; });
-    const int64_t nhi = block_first(x, nlo, c.hi, &s_t, [vmax](double v) { return v > vmax; });
-    if (threadIdx.x == 0) {
-        const int64_t nchanged = m - (nhi - nlo);
-        ClipState d;
-        d.lo = nlo;
-        d.hi = nhi;
-        d.med = cen;
-        d.mean = mean;
-        d.sd = sd;
-        d.have = nchanged == 0;
-        d.done = nchanged == 0 || nhi == nlo;
-        cs[k] = d;
+    a.n = wave_add(a.n);
+    a.s1 = wave_add(a.s1);
+    a.s2 = wave_add(a.s2);
+    if ((t & 63) == 0) {
+        S.part[p][t >> 6] = a;
+        S.below[p][t >> 6] = below;
+    }
+    __syncthreads();
+    below = 0.0;
+    for (int q = 0; q < MX_OS_CW; ++q) below += S.below[p][q];
+    K.c0 = K.c1 = {0.0, 0.0, 0.0};
+    for (int q = 0; q < MX_OS_CW; ++q) {
+        CutSums &d = q < MX_OS_CW / 2 ? K.c0 : K.c1;
+        d.n += S.part[p][q].n;
+        d.s1 += S.part[p][q].s1;
+        d.s2 += S.part[p][q].s2;
     }
 }
 
-__global__ void mx_os_clip_final_kernel(MxOrderStats a, const ClipState *cs, const double *x, const double *p0,
-                                        const double *p1) {
-    const int k = threadIdx.x;
-    if (k >= a.n_orders) return;
-    const ClipState c = cs[k];
-    const int64_t m = c.hi - c.lo;
+// One order: probability sum and count, then the clipping rounds.  Bound by
+// the latency of its dependent steps, so everything that can be is done by
+// every wave for itself, and a round has two barriers: one after the sums over
+// the two cut bins, one after the candidates of the median (92 us for 8e6
+// photons in 15 orders; with a workgroup-wide reduction for each sum and a
+// selection from the start for each median 179 us).
+template <bool VALUES>
+__global__ __launch_bounds__(MX_OS_CLIP) void mx_os_clip_kernel(MxOrderStats a, OsPlan L, unsigned char *ws) {
+    extern __shared__ __align__(16) unsigned char sm[];
+    __shared__ ClipShared S;
+    const int k = blockIdx.x, t = threadIdx.x, w = t >> 6;
+    const int bins = VALUES ? L.bins : 0;
+    const BinPieces rest = pieces_of(L, ws, k, bins, 1);
+    // probability sum; photons outside the bins
+    const double *psum = (const double *)(ws + L.psum) + (size_t)k * L.chunks;
+    CutSums tot = {0.0, 0.0, 0.0};
+    for (int64_t c = t; c < L.chunks; c += MX_OS_CLIP) {
+        tot.s1 += psum[c];
+        tot.n += (double)((int)rest.off[rest.end + c] - (int)rest.off[c]);
+    }
+    tot.n = wave_add(tot.n);
+    tot.s1 = wave_add(tot.s1);
+    if ((t & 63) == 0) S.part[1][w] = tot;
+    BinInfo *info = (BinInfo *)sm;
+    double *edges = (double *)(info + bins), *list = edges + bins;
+    if (VALUES) {
+        for (int b = t; b < bins; b += MX_OS_CLIP) {
+            BinInfo f = {((const int64_t *)(ws + L.place))[(size_t)k * bins + b], 0.0, 0.0, 0.0};
+#pragma unroll 4
+            for (int g = 0; g < L.groups; ++g) {
+                const BinInfo q = ((const BinInfo *)(ws + L.grp))[((size_t)k * L.groups + g) * bins + b];
+                f.n += q.n;
+                f.s1 += q.s1;
+                f.s2 += q.s2;
+            }
+            info[b] = f;
+            edges[b] = ((const double *)(ws + L.edges))[(size_t)k * bins + b];
+        }
+        if (t < 2) S.n[t] = 0;
+    }
+    __syncthreads();
+    double ps = 0.0, other = 0.0;
+    for (int q = 0; q < MX_OS_CW; ++q) {
+        ps += S.part[1][q].s1;
+        other += S.part[1][q].n;
+    }
+    if (!VALUES) {
+        if (t == 0) {
+            a.prob_sum[k] = ps;
+            a.count[k] = (int64_t)other;
+        }
+        return;
+    }
+    const ClipOrder O = {L, ws, k, bins, edges, info};
+    Kept K = {0, bins - 1, false, 0.0, 0.0, {0.0, 0.0, 0.0}, {0.0, 0.0, 0.0}};
+    double N = kept_count(O, K);
+    if (t == 0) {
+        a.prob_sum[k] = ps;
+        a.count[k] = (int64_t)(N + ((a.flags & MX_OS_FILTER) ? 0.0 : other));
+    }
     const double nan = __builtin_nan("");
-    double mean = nan, med = nan, sd = nan;
-    if (c.have) {
-        med = c.med;
-        mean = c.mean;
-        sd = c.sd;
-    } else if (m > 0) {
-        med = median_sorted(x, c.lo, c.hi);
-        clip_moments(p0, p1, k, m, mean, sd);
+    double mean = nan, cen = nan, sd = nan;
+    if (N > 0.0) {
+        Held H = {-1, false, 0, 0, 0, 0, 0.0, 0.0};
+        int nlist = -1;
+        double c = 0.0, below = 0.0;
+        if (N <= (double)MX_OS_LIST) {
+            // the whole order into the list, in the same places every run
+            const BinPieces P = pieces_of(L, ws, k, 0, bins);
+            const Share R = share_pieces<MX_OS_CLIP>(P, S.first, S.iw);
+            if (t == 0) {
+                S.kmin = ~0ull;
+                S.kmax = 0;
+            }
+            __syncthreads();
+            uint64_t mn = ~0ull, mx = 0;
+            P.each(R.group, MX_OS_CLIP / R.per, R.sub, R.per, [&](double x, int64_t at) {
+                const uint64_t q = key_of(x);
+                mn = q < mn ? q : mn;
+                mx = q > mx ? q : mx;
+                list[R.first + at] = x;
+            });
+            key_range(S, mn, mx);
+            nlist = (int)N;
+            H.bin = MX_OS_ALL;
+            H.n = nlist;
+            H.kmin = S.kmin;
+            H.kmax = S.kmax;
+        }
+        if (isinf(edges[0])) {
+            // no photon of the order in the sample: one bin holds them all,
+            // and its values are summed one by one, about their mean
+            K.cut = true;
+            K.bh = 0;
+            K.lo = -__builtin_inf();
+            K.hi = __builtin_inf();
+            c = info[0].s1 / info[0].n;
+        }
+        int p = 0;
+        for (int it = 0;; ++it) {
+            Kept Q = K;
+            bool any = true;
+            if (it > 0) {
+                double lo = cen - sd * a.sigma, hi = cen + sd * a.sigma;
+                if (K.cut) {
+                    lo = K.lo > lo ? K.lo : lo;
+                    hi = K.hi < hi ? K.hi : hi;
+                }
+                any = lo <= hi;      // false for NaN bounds, which keep nothing
+                Q.cut = true;
+                Q.lo = lo;
+                Q.hi = hi;
+                if (nlist < 0) {
+                    Q.bl = O.bin_of(lo);
+                    Q.bh = O.bin_of(hi);
+                }
+            }
+            double kept = 0.0;
+            if (any) {
+                if (Q.cut) cut_bins(O, Q, c, S, p, list, nlist, below);
+                p ^= 1;
+                kept = nlist >= 0 && Q.cut ? Q.c0.n + Q.c1.n : kept_count(O, Q);
+            }
+            if (it > 0 && kept == N) break;
+            N = kept;
+            if (N == 0.0) {
+                mean = cen = sd = nan;
+                break;
+            }
+            K = Q;
+            cen = kept_median(O, K, (int64_t)N, (int64_t)below, S, list, H);
+            kept_moments(O, K, N, K.cut ? c : cen, nlist >= 0 && K.cut, mean, sd);
+            c = cen;
+            if (it == a.maxiters) break;
+        }
     }
-    a.mean[k] = mean;
-    a.median[k] = med;
-    a.std[k] = sd;
-    a.n_kept[k] = m;
+    if (t == 0) {
+        a.mean[k] = mean;
+        a.median[k] = cen;
+        a.std[k] = sd;
+        a.n_kept[k] = (int64_t)N;
+    }
 }
 
 extern "C" int64_t mx_order_stats_workspace(int64_t n, int32_t n_orders, int32_t with_values) {
     if (n < 0 || n_orders < 1 || n_orders > MX_MAX_ORDERS) return -1;
-    OsLayout L;
-    if (os_layout(n, n_orders, with_values != 0, L)) return -1;
+    OsPlan L;
+    os_plan(n, n_orders, with_values != 0, L);
     return (int64_t)L.total;
 }
 
@@ -564,71 +1316,32 @@ extern "C" int mx_order_stats(const MxOrderStats *a, void *stream) {
         mx_set_error("order stats: the finite-value filter needs a value column");
         return 1;
     }
-    OsLayout L;
-    if (os_layout(a->n, a->n_orders, values, L)) { mx_set_error("order stats: sort size query failed"); return 2; }
+    OsPlan L;
+    os_plan(a->n, a->n_orders, values, L);
     if (!a->workspace || a->workspace_bytes < (int64_t)L.total) {
         mx_set_error("order stats: workspace missing or smaller than mx_order_stats_workspace()");
         return 1;
     }
     hipStream_t st = (hipStream_t)stream;
     unsigned char *ws = (unsigned char *)a->workspace;
-    int64_t *cnt_b = (int64_t *)(ws + L.cnt_b);
-    int64_t *nval_b = (int64_t *)(ws + L.nval_b);
-    double *psum_b = (double *)(ws + L.psum_b);
-    int64_t *off_b = (int64_t *)(ws + L.off_b);
-    int64_t *tot = (int64_t *)(ws + L.tot);
-    int32_t *seg = (int32_t *)(ws + L.seg);
-    const int no = a->n_orders;
-    const int64_t nb = os_blocks(a->n);
-    const int64_t chunk = (a->n + nb - 1) / nb > 0 ? (a->n + nb - 1) / nb : 1;
-    const size_t lds1 = (size_t)no * MX_OS_WAVE * (8 + 4 + 4) + (size_t)no * 4;
-    hipLaunchKernelGGL(mx_os_count_kernel, dim3((unsigned)nb), dim3(MX_OS_WAVE), lds1, st, *a, chunk,
-                       cnt_b, nval_b, psum_b);
-    hipLaunchKernelGGL(mx_os_scan_kernel, dim3((unsigned)no), dim3(MX_OS_SCAN), 0, st, *a, nb, cnt_b, nval_b,
-                       psum_b, off_b, tot);
-    hipLaunchKernelGGL(mx_os_seg_kernel, dim3(1), dim3(MX_OS_WAVE), 0, st, no, (const int64_t *)tot, seg);
+    const dim3 chunks((unsigned)L.chunks), split(MX_OS_SPLIT);
+    const size_t lds = split_lds(L);
     if (values) {
-        double *vals = (double *)(ws + L.vals), *sorted = (double *)(ws + L.sorted);
-        const size_t lds3 = (size_t)no * MX_OS_WAVE * 8 + (size_t)no * 4;
-        uint8_t *ordk = (uint8_t *)(ws + L.ord), *ordk2 = (uint8_t *)(ws + L.ord2);
-        hipLaunchKernelGGL(mx_os_scatter_kernel, dim3((unsigned)nb), dim3(MX_OS_WAVE), lds3, st, *a, chunk,
-                           off_b, seg, vals, ordk);
-        // the segments fill [0, total); total <= n is known on the device
-        // only, so the sorts run over n items with the tail set to +inf /
-        // an order index past the last, which sorts behind every segment
-        hipLaunchKernelGGL(mx_os_tail_kernel, dim3((unsigned)((a->n + 255) / 256 > 0 ? (a->n + 255) / 256 : 1)),
-                           dim3(256), 0, st, seg + no + no - 1, a->n, vals, ordk);
-        size_t tb = L.temp_bytes;
-        if (hipcub::DeviceRadixSort::SortPairs(ws + L.temp, tb, (const double *)vals, sorted,
-                                               (const uint8_t *)ordk, ordk2, (int)a->n, 0, 64, st) != hipSuccess) {
-            mx_set_error("order stats: sort by value failed");
-            return 2;
-        }
-        tb = L.temp_bytes;
-        if (hipcub::DeviceRadixSort::SortPairs(ws + L.temp, tb, (const uint8_t *)ordk2, ordk,
-                                               (const double *)sorted, vals, (int)a->n, 0, 8, st) != hipSuccess) {
-            mx_set_error("order stats: sort by order failed");
-            return 2;
-        }
-        const double *xs = vals;
-        ClipState *cs = (ClipState *)(ws + L.clip);
-        double *p0 = (double *)(ws + L.part0), *p1 = (double *)(ws + L.part1);
-        hipLaunchKernelGGL(mx_os_clip_init_kernel, dim3(1), dim3(MX_OS_WAVE), 0, st, no, (const int32_t *)seg, cs);
-        const dim3 gsum((unsigned)(no * MX_OS_CW));
-        for (int it = 0; it < a->maxiters; ++it) {
-            hipLaunchKernelGGL(mx_os_clip_sum_kernel, gsum, dim3(MX_OS_CLIP), 0, st, (const ClipState *)cs, xs, p0,
-                               p1, 0, 0);
-            hipLaunchKernelGGL(mx_os_clip_sum_kernel, gsum, dim3(MX_OS_CLIP), 0, st, (const ClipState *)cs, xs, p0,
-                               p1, 1, 0);
-            hipLaunchKernelGGL(mx_os_clip_bounds_kernel, dim3((unsigned)no), dim3(MX_OS_CLIP), 0, st, *a, cs, xs,
-                               (const double *)p0, (const double *)p1);
-        }
-        hipLaunchKernelGGL(mx_os_clip_sum_kernel, gsum, dim3(MX_OS_CLIP), 0, st, (const ClipState *)cs, xs, p0, p1,
-                           0, 1);
-        hipLaunchKernelGGL(mx_os_clip_sum_kernel, gsum, dim3(MX_OS_CLIP), 0, st, (const ClipState *)cs, xs, p0, p1,
-                           1, 1);
-        hipLaunchKernelGGL(mx_os_clip_final_kernel, dim3(1), dim3(MX_OS_WAVE), 0, st, *a, (const ClipState *)cs,
-                           xs, (const double *)p0, (const double *)p1);
+        hipLaunchKernelGGL(mx_os_sample_kernel, dim3((unsigned)L.no), dim3(1024), 0, st, *a, L, ws);
+        if (L.chunks > 0 && L.rows == MX_OS_ROWS)
+            hipLaunchKernelGGL((mx_os_split_kernel<MX_OS_ROWS, true>), chunks, split, lds, st, *a, L, ws);
+        else if (L.chunks > 0)
+            hipLaunchKernelGGL((mx_os_split_kernel<MX_OS_ROWS_FEW, true>), chunks, split, lds, st, *a, L, ws);
+        hipLaunchKernelGGL(mx_os_merge_kernel, dim3((unsigned)(L.groups + 2 * MX_OS_ENDS + MX_OS_NEAR), (unsigned)L.no),
+                           dim3(MX_OS_MERGE), 0, st, L, ws);
+        hipLaunchKernelGGL(mx_os_clip_kernel<true>, dim3((unsigned)L.no), dim3(MX_OS_CLIP), clip_lds(L), st, *a, L,
+                           ws);
+    } else {
+        if (L.chunks > 0 && L.rows == MX_OS_ROWS)
+            hipLaunchKernelGGL((mx_os_split_kernel<MX_OS_ROWS, false>), chunks, split, lds, st, *a, L, ws);
+        else if (L.chunks > 0)
+            hipLaunchKernelGGL((mx_os_split_kernel<MX_OS_ROWS_FEW, false>), chunks, split, lds, st, *a, L, ws);
+        hipLaunchKernelGGL(mx_os_clip_kernel<false>, dim3((unsigned)L.no), dim3(MX_OS_CLIP), 0, st, *a, L, ws);
     }
     hipError_t err = hipGetLastError();
     if (err != hipSuccess) {
@@ -643,16 +1356,15 @@ extern "C" int mx_order_stats(const MxOrderStats *a, void *stream) {
 // ------------------------------------------------ allocation-free variant
 // mx_order_stats_static: mx_order_stats with its workspace in `scratch`, a
 // file-scope device array of MX_OS_STATIC_BYTES, for callers that cannot
-// allocate (tight serving loops, harnesses that forbid hipMalloc; not graph
-// capture: the radix sorts clear their pass state with memsets).  Every GPU the
-// library runs on holds its own copy until the process ends.  Host code
+// allocate (tight serving loops, harnesses that forbid hipMalloc).  Every GPU
+// the library runs on holds its own copy until the process ends.  Host code
 // never passes the array's name to a kernel or a copy (in host code it is a
 // host-side stand-in): the device address of this GPU's copy comes from
 // hipGetSymbolAddress on the entry point's first call on that GPU and is
 // kept per device.  Calls on one GPU share the array, so calls that overlap
 // on one GPU race; it keeps the last call's contents, and every word a call
-// reads it has written first (counts, offsets, segments, values, clipping
-// state), so nothing needs clearing.
+// reads it has written first (edges, offsets, sums, values), so nothing needs
+// clearing.
 static __device__ __align__(256) unsigned char scratch[MX_OS_STATIC_BYTES];
 
 #define MX_OS_MAX_DEVICES 64
@@ -686,11 +1398,8 @@ extern "C" int mx_order_stats_static(const MxOrderStats *a, void *stream) {
     if (!a) { mx_set_error("order stats: arguments NULL"); return 1; }
     if (a->n < 0 || a->n > 0x7fffffffLL) { mx_set_error("order stats: photon count outside [0, 2^31)"); return 1; }
     if (a->n_orders < 1 || a->n_orders > MX_MAX_ORDERS) { mx_set_error("order stats: n_orders outside [1, 64]"); return 1; }
-    OsLayout L;
-    if (os_layout(a->n, a->n_orders, a->value != nullptr, L)) {
-        mx_set_error("order stats: sort size query failed");
-        return 2;
-    }
+    OsPlan L;
+    os_plan(a->n, a->n_orders, a->value != nullptr, L);
     if ((int64_t)L.total > (int64_t)MX_OS_STATIC_BYTES) {
         char buf[256];
         snprintf(buf, sizeof(buf),
