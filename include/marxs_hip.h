@@ -351,6 +351,43 @@ typedef struct MxPoseArgs {
 
 int mx_facet_pose(const MxPoseArgs *args, void *stream);
 
+/* One loss and gradient of L = centroid + RMS width (poses and periods ->
+ * facet frames -> replay of every photon -> chain rule back) for photons
+ * ordered by facet: the results of mx_facet_pose mode 0, mx_adjoint with
+ * MX_AJ_SUMS and mx_facet_pose mode 2, up to the order of the sums, which is
+ * fixed.  A task is a run of photons of one facet: task[3 j] its facet,
+ * [task[3 j + 1], task[3 j + 2]) its photons (an empty run: no task); the
+ * tasks of facet f are task_first[f] .. task_first[f + 1] - 1, and a photon
+ * in no task does not count.  photons: n, pos, dir, energy, weight, order,
+ * ccd, ccd_t, y_shift, n_ccd, coord and precision are read.  pose: everything
+ * but mode, grad13 and moments is used.  No reference counterpart. */
+#define MX_AJ_PART 32
+typedef struct MxAdjointStep {
+    MxAdjointArgs photons;
+    MxPoseArgs pose;
+    const int32_t *task;       /* [n_tasks][3] */
+    const int32_t *task_first; /* [n_facet + 1] */
+    double *part;              /* [n_tasks][MX_AJ_PART] scratch */
+    double *grad_theta;        /* [n_facet][6], may be NULL */
+    double *grad_period;       /* [n_facet], may be NULL */
+    double *loss_out;          /* [1], may be NULL */
+    double *theta_out;         /* [n_facet][6] copy of pose.theta, may be NULL */
+    double *period_out;        /* [n_facet] copy of pose.period, may be NULL */
+    double *moments_out;       /* [3] sum w, sum w (y - y_shift), sum w (y - y_shift)^2, may be NULL */
+    int32_t n_tasks;           /* task_first[n_facet] at least */
+    int32_t reserved;
+} MxAdjointStep;
+
+int mx_adjoint_step(const MxAdjointStep *args, void *stream);
+
+/* The work list of mx_adjoint_step for photons whose facets (`facet`, [n],
+ * ascending; those outside 0 .. n_facet-1 are left out) are given: runs of at
+ * most `size` photons.  n_tasks entries are written, n_facet + n / size at
+ * least; those past the last task are empty.  All pointers are device
+ * pointers.  No reference counterpart. */
+int mx_adjoint_tasks(const int32_t *facet, int64_t n, int32_t n_facet, int32_t size,
+                     int32_t *task_first, int32_t *task, int32_t n_tasks, void *stream);
+
 /* ------------------------------------------------------------ per-order statistics
  * Figures of merit of a traced photon list, per grating order, without
  * leaving HBM.  Replaces the host loops of effectivearea_from_photonlist

@@ -9,7 +9,8 @@ import os
 
 import torch  # noqa: F401  (loads the HIP runtime first)
 
-__all__ = ['lib', 'MxTables', 'MxPhotons', 'MxAdjointArgs', 'MxBatch', 'MxPoseArgs', 'MxOrderStats',
+__all__ = ['lib', 'MxTables', 'MxPhotons', 'MxAdjointArgs', 'MxBatch', 'MxPoseArgs', 'MxAdjointStep',
+           'MxOrderStats',
            'MX_MAX_FCOLS', 'MX_MAX_ICOLS', 'MX_NSTATUS', 'MX_MAX_ORDERS', 'MX_OS_FILTER', 'LIB_PATH',
            'check']
 
@@ -68,6 +69,13 @@ class MxPoseArgs(ctypes.Structure):
                 ('y_shift', ctypes.c_double)]
 
 
+class MxAdjointStep(ctypes.Structure):
+    _fields_ = [('photons', MxAdjointArgs), ('pose', MxPoseArgs), ('task', P), ('task_first', P),
+                ('part', P), ('grad_theta', P), ('grad_period', P), ('loss_out', P),
+                ('theta_out', P), ('period_out', P), ('moments_out', P),
+                ('n_tasks', ctypes.c_int32), ('reserved', ctypes.c_int32)]
+
+
 class MxOrderStats(ctypes.Structure):
     _fields_ = [('n', ctypes.c_int64), ('order', P), ('value', P), ('prob', P), ('orders', P),
                 ('n_orders', ctypes.c_int32), ('flags', ctypes.c_int32), ('sigma', ctypes.c_double),
@@ -79,6 +87,7 @@ class MxOrderStats(ctypes.Structure):
 MX_AJ_GEOM = 16
 MX_AJ_NGRAD = 13
 MX_AJ_SUMS = 1
+MX_AJ_PART = 32
 MX_MAX_ORDERS = 64
 MX_OS_FILTER = 1
 MX_OS_STATIC_BYTES = 64 << 20
@@ -111,6 +120,11 @@ def _load():
     lib.mx_adjoint.argtypes = [ctypes.POINTER(MxAdjointArgs), P]
     lib.mx_facet_pose.restype = ctypes.c_int
     lib.mx_facet_pose.argtypes = [ctypes.POINTER(MxPoseArgs), P]
+    lib.mx_adjoint_step.restype = ctypes.c_int
+    lib.mx_adjoint_step.argtypes = [ctypes.POINTER(MxAdjointStep), P]
+    lib.mx_adjoint_tasks.restype = ctypes.c_int
+    lib.mx_adjoint_tasks.argtypes = [P, ctypes.c_int64, ctypes.c_int32, ctypes.c_int32, P, P,
+                                     ctypes.c_int32, P]
     lib.mx_order_stats_workspace.restype = ctypes.c_int64
     lib.mx_order_stats_workspace.argtypes = [ctypes.c_int64, ctypes.c_int32, ctypes.c_int32]
     lib.mx_order_stats.restype = ctypes.c_int

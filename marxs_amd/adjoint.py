@@ -31,6 +31,8 @@ from .compiler import compile_tree, STAGE_GRATING, STAGE_DETECTOR
 __all__ = ['facet_geometry', 'FacetLoss', 'AdjointProblem', 'ChunkedAdjoint', 'entrance_chunk',
            'euler_sxyz_torch', 'central_differences']
 
+TASK = 128      # photons of one facet that a workgroup of the fused step takes
+
 
 def _rot(axis, a):
     c, s = torch.cos(a), torch.sin(a)
@@ -229,20 +231,62 @@ class AdjointProblem:
         pb['sums'] = pb['accum'][:F * 26].view(F, 26)
         pb['moments'] = pb['accum'][F * 26:]
         # shift of the moments: the weighted mean coordinate at the base pose
-        y = self.coordinates(self.geometry(self.theta0, self.period0))
+        pose = _lib.MxPoseArgs(n_facet=F, mode=0, theta=self.theta0.data_ptr(), period=self.period0.data_ptr(),
+                               **{k: pb[k].data_ptr() for k in ('gu', 't0', 'rpost', 'zoom', 'extra', 'geom')})
+        _lib.check(_lib.lib.mx_facet_pose(ctypes.byref(pose), ctypes.c_void_p(
+            torch.cuda.current_stream(self.device).cuda_stream)))
+        y = self.coordinates(pb['geom'])
         ok = ~torch.isnan(y)
         w = torch.where(ok, self.weight, torch.zeros_like(self.weight))
         self.y_shift = float((w * torch.where(ok, y, torch.zeros_like(y))).sum() / w.sum())
         # stream compaction: the fused kernels visit only the photons that
-        # carry weight on a facet and a detector
+        # carry weight on a facet and a detector, ordered by facet
         idx = torch.nonzero((self.weight != 0) & (self.facet >= 0) & (self.ccd >= 0)).flatten()
+        facet, by_facet = torch.sort(self.facet[idx], stable=True)
+        idx = idx[by_facet]
         pb['src'] = {'n': int(idx.numel()), 'idx': idx,
                      'pos': self.pos[:, idx].contiguous(), 'dir': self.dir[:, idx].contiguous(),
                      'energy': self.energy[idx].contiguous(), 'weight': self.weight[idx].contiguous(),
                      'facet': self.facet[idx].contiguous(), 'order': self.order[idx].contiguous(),
                      'ccd': self.ccd[idx].contiguous()}
+        self._tasks(pb, facet.contiguous())
         self._pb = pb
         return pb
+
+    def _tasks(self, pb, facet):
+        """Work list of the fused step (``mx_adjoint_step``): runs of up to
+        ``TASK`` photons of one facet in the facet-ordered photons; longer
+        runs where that would make more than 4096, so that forming a facet's
+        frame stays small beside its photons.  The number of entries is an
+        upper bound, those past the last task are empty."""
+        n, F = facet.numel(), self.F
+        size = TASK * max(1, -(-n // (TASK * 4096)))
+        count = F + n // size
+        i32 = dict(dtype=torch.int32, device=self.device)
+        pb['task_first'], pb['task'] = torch.empty(F + 1, **i32), torch.empty((count, 3), **i32)
+        pb['part'] = torch.empty((count, _lib.MX_AJ_PART), dtype=torch.float64, device=self.device)
+        stream = torch.cuda.current_stream(self.device).cuda_stream
+        _lib.check(_lib.lib.mx_adjoint_tasks(facet.data_ptr(), n, F, size, pb['task_first'].data_ptr(),
+                                             pb['task'].data_ptr(), count, ctypes.c_void_p(stream)))
+
+    def _step_args(self, precision):
+        """Arguments of ``mx_adjoint_step`` on the buffers (a copy of those
+        built once per precision); loss and gradients go to the buffers."""
+        pb = self._pose_buffers()
+        s = pb.setdefault('step', {}).get(precision)
+        if s is None:
+            s = _lib.MxAdjointStep()
+            s.photons = self._args(pb['geom'], precision, src=pb['src'])
+            s.pose = self._pose_args(2)
+            s.task, s.task_first, s.part = (pb[k].data_ptr() for k in ('task', 'task_first', 'part'))
+            s.moments_out = pb['moments'].data_ptr()
+            s.n_tasks = pb['task'].shape[0]
+            pb['step'][precision] = s
+        s = _lib.MxAdjointStep.from_buffer_copy(s)
+        s.photons.coord = self.coord
+        s.photons.ccd_t = self.ccd_t.data_ptr()
+        s.photons.y_shift = s.pose.y_shift = self.y_shift
+        return s
 
     def restrict_to_traced(self, y_traced, rtol=1e-10):
         """Zero the weight of photons whose traced detector coordinate the
@@ -273,24 +317,19 @@ class AdjointProblem:
 
     def launch_loss_and_grad(self, precision=32, stream=None):
         """Launch the fused evaluation on the parameters held in
-        ``buffers['theta']``/``['period']`` (asynchronous): one fill of the
-        accumulators, the pose chain, one replay of every photon that
-        accumulates the moments and the per-facet sums A = sum w dy/dg,
-        B = sum w (y - s) dy/dg (``MX_AJ_SUMS``), then the chain rule back to
-        the poses with dL/dg = A / W + (B - a A) / (W sigma) (L = mu + sigma,
-        dL/dy_i = w_i / W (1 + (y_i - mu) / sigma)).  Results:
-        ``buffers['loss']`` and ``buffers['grad7']`` (d/d theta, d/d period)."""
-        pb = self._pose_buffers()
+        ``buffers['theta']``/``['period']`` (asynchronous): every task of
+        photons forms its facet's frame, replays its photons and sums the
+        moments and A = sum w dy/dg, B = sum w (y - s) dy/dg; then, per facet,
+        the chain rule back to the poses with dL/dg = A / W + (B - a A) / (W
+        sigma) (L = mu + sigma, dL/dy_i = w_i / W (1 + (y_i - mu) / sigma)).
+        Results: ``buffers['loss']`` and ``buffers['grad7']`` (d/d theta, d/d
+        period)."""
+        s = self._step_args(precision)
+        pb = self._pb
+        s.pose.theta, s.pose.period = pb['theta'].data_ptr(), pb['period'].data_ptr()
         if stream is None:
             stream = torch.cuda.current_stream(self.device).cuda_stream
-        pb['accum'].zero_()
-        _lib.check(_lib.lib.mx_facet_pose(ctypes.byref(self._pose_args(0)), ctypes.c_void_p(stream)))
-        one = self._args(pb['geom'], precision, grad=pb['accum'], moments=pb['moments'], src=pb['src'])
-        one.flags = _lib.MX_AJ_SUMS
-        one.lds_accumulate = int(self.F <= 315)
-        one.y_shift = self.y_shift
-        _launch(one, stream)
-        _lib.check(_lib.lib.mx_facet_pose(ctypes.byref(self._pose_args(2)), ctypes.c_void_p(stream)))
+        _lib.check(_lib.lib.mx_adjoint_step(ctypes.byref(s), ctypes.c_void_p(stream)))
 
     @property
     def buffers(self):
@@ -300,11 +339,25 @@ class AdjointProblem:
         """L = centroid + RMS width and its gradient with respect to the 6-DOF
         poses and periods, without autograd: returns (L, dL/dtheta (F, 6),
         dL/dperiod (F,)), all on the device."""
-        pb = self._pose_buffers()
-        pb['theta'].copy_(theta)
-        pb['period'].copy_(period)
-        self.launch_loss_and_grad(precision)
-        return pb['loss'][0].clone(), pb['grad7'][:, :6].clone(), pb['grad7'][:, 6].clone()
+        s = self._step_args(precision)
+        pb = self._pb
+        loss, grad_theta, grad_period = (torch.empty(shape, dtype=torch.float64, device=self.device)
+                                         for shape in ((), (self.F, 6), (self.F,)))
+        # the kernels read the parameters where they are, and leave a copy in
+        # the buffers, unless they have another layout
+        for name, x, out in (('theta', theta, 'theta_out'), ('period', period, 'period_out')):
+            held = pb[name]
+            if (type(x) is torch.Tensor and x.dtype == torch.float64 and x.device == held.device and
+                    x.shape == held.shape and x.is_contiguous() and not x.is_neg()):
+                setattr(s.pose, name, x.data_ptr())
+                setattr(s, out, held.data_ptr())
+            else:
+                held.copy_(x)
+                setattr(s.pose, name, held.data_ptr())
+        s.loss_out, s.grad_theta, s.grad_period = (t.data_ptr() for t in (loss, grad_theta, grad_period))
+        stream = torch.cuda.current_stream(self.device).cuda_stream
+        _lib.check(_lib.lib.mx_adjoint_step(ctypes.byref(s), ctypes.c_void_p(stream)))
+        return loss, grad_theta, grad_period
 
     def capture(self, precision=32):
         """hipGraph of :meth:`launch_loss_and_grad` (replay after writing new
