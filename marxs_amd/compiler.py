@@ -725,6 +725,19 @@ def _param_records32(tables, st):
     return rec
 
 
+def _detector_records(tables, st):
+    """Interaction records of a detector stage, 18 float64 words per element:
+    FP64 frame (centre, e_x, e_y, e_z), pixel size, centre pixels, 1 / pixel
+    size, then id and pixel numbers as int32."""
+    n = len(st.elements)
+    rec = np.zeros((n, 18))
+    rec[:, 0:12] = tables.elem_t[st.elem0:st.elem0 + n, 0:12]
+    rec[:, 12:16] = tables.elem_p[st.elem0:st.elem0 + n, 6:10]
+    iv = rec.view(np.int32)
+    iv[:, 32:35] = tables.elem_i[st.elem0:st.elem0 + n][:, [0, 4, 5]]
+    return rec
+
+
 def _build_lds(tables, budget32=None, budget64=None):
     """Byte images staged into LDS by every workgroup (one per precision).
 
@@ -741,7 +754,8 @@ def _build_lds(tables, budget32=None, budget64=None):
     [22] FP32 parameters, [24]/[25]/[30] FP32 tight cell offsets/items/
     successors, [26]/[27]/[31] the same FP64, [36]/[37]/[38] FP32 loose cell
     offsets/items/successors, [39]/[40]/[41] the same FP64; sel_i[6]/[7]
-    selector block FP32/FP64.
+    selector block FP32/FP64.  [51]/[52] detector records FP32/FP64 (0 =
+    global memory).
     """
     budget32 = LDS_BUDGET32 if budget32 is None else budget32
     budget64 = LDS_BUDGET64 if budget64 is None else budget64
@@ -899,6 +913,15 @@ def _build_lds(tables, budget32=None, budget64=None):
             c0, c1 = (36, 37) if prec == 32 else (39, 40)
             si[s, c0] = add(g['cell_start_l'].astype(np.uint16))
             si[s, c1] = add(g['items_l'].astype(np.uint16))
+        # what a detector hit reads besides its test record: small, so it goes
+        # after everything that is read more often
+        for s, st in enumerate(tables.stages):
+            si[s, 51 if prec == 32 else 52] = 0
+            if st.kind != STAGE_DETECTOR or si[s, 20 if prec == 32 else 21] < 0:
+                continue
+            recs = _detector_records(tables, st)
+            if off > 0 and off + _align(recs.nbytes) <= budget:
+                si[s, 51 if prec == 32 else 52] = add(recs)
         img = np.zeros(_align(max(off, 16)), dtype=np.uint8)
         for o, b in parts:
             img[o:o + b.nbytes] = b

@@ -39,6 +39,7 @@
 #define MX_E2W 1.2398419292004202e-06   /* keV -> mm, marxs/__init__.py:14 */
 #define MX_E2W_F 1.2398419292004202e-06f
 #define MX_ORDER_NONE (-2147483647 - 1)
+#define MX_DR 18                /* float64 words of a detector record in LDS */
 #ifndef MX_BLOCK32
 #define MX_BLOCK32 1024         /* one workgroup per CU holds the LDS image   */
 #endif
@@ -97,16 +98,8 @@ __device__ __forceinline__ d3 unit3(d3 v) {
 }
 
 // FinitePlane.intersect, marxs/math/geometry.py:233-253
-__device__ __forceinline__ bool plane_test64(const double *__restrict__ et, d3 p, d3 d,
+__device__ __forceinline__ bool plane_math64(d3 c, d3 ex, d3 ey, d3 ez, double hy, double hz, d3 p, d3 d,
                                              d3 &q, double &ly, double &lz) {
-    // records are 16-byte aligned: 16-byte loads
-    const double2 a0 = ((const double2 *)et)[0], a1 = ((const double2 *)et)[1];
-    const double2 a2 = ((const double2 *)et)[2], a3 = ((const double2 *)et)[3];
-    const double2 a4 = ((const double2 *)et)[4], a5 = ((const double2 *)et)[5];
-    const double2 a6 = ((const double2 *)et)[6];
-    d3 c = mk(a0.x, a0.y, a1.x), ex = mk(a1.y, a2.x, a2.y);
-    d3 ey = mk(a3.x, a3.y, a4.x), ez = mk(a4.y, a5.x, a5.y);
-    const double hy = a6.x, hz = a6.y;
     double kn = dot3(sub3(c, p), ex);
     double kd = dot3(d, ex);
     double k = kn / kd;
@@ -117,10 +110,22 @@ __device__ __forceinline__ bool plane_test64(const double *__restrict__ et, d3 p
     return (kd != 0.0) && (k >= 0.0) && (fabs(ly) <= hy) && (fabs(lz) <= hz);
 }
 
+__device__ __forceinline__ bool plane_test64(const double *__restrict__ et, d3 p, d3 d,
+                                             d3 &q, double &ly, double &lz) {
+    // records are 16-byte aligned: 16-byte loads
+    const double2 a0 = ((const double2 *)et)[0], a1 = ((const double2 *)et)[1];
+    const double2 a2 = ((const double2 *)et)[2], a3 = ((const double2 *)et)[3];
+    const double2 a4 = ((const double2 *)et)[4], a5 = ((const double2 *)et)[5];
+    const double2 a6 = ((const double2 *)et)[6];
+    return plane_math64(mk(a0.x, a0.y, a1.x), mk(a1.y, a2.x, a2.y), mk(a3.x, a3.y, a4.x), mk(a4.y, a5.x, a5.y),
+                        a6.x, a6.y, p, d, q, ly, lz);
+}
+
 // The same test for the FP32 path's final detector coordinate: the division
 // is a float reciprocal refined by one Newton step in double (relative error
 // ~1e-14, far below the FP32 path's error budget).
-__device__ __forceinline__ void plane_hit64_fast(const double *__restrict__ et, d3 p, d3 d,
+template <typename PT>
+__device__ __forceinline__ void plane_hit64_fast(PT et, d3 p, d3 d,
                                                  d3 &q, double &ly, double &lz) {
     d3 c = ld3(et), ex = ld3(et + 3), ey = ld3(et + 6), ez = ld3(et + 9);
     double kn = dot3(sub3(c, p), ex);
@@ -195,15 +200,9 @@ __device__ __forceinline__ d3 tod(f3 v) { return mk((double)v.x, (double)v.y, (d
 // ray-plane test in a stage-local frame: p is relative to the stage origin
 // and the ray parameter must satisfy k >= kmin (kmin <= 0 when p was moved
 // forward along the ray).
-__device__ __forceinline__ bool plane_test32(const float *__restrict__ et, f3 p, f3 d, float kmin,
+__device__ __forceinline__ bool plane_math32(f3 c, f3 ex, f3 ey, f3 ez, float hy, float hz, f3 p, f3 d, float kmin,
                                              float &k, float &ly, float &lz) {
 #pragma clang fp contract(fast)
-    // records are 64-byte aligned: four 16-byte loads
-    const float4 r0 = ((const float4 *)et)[0], r1 = ((const float4 *)et)[1];
-    const float4 r2 = ((const float4 *)et)[2], r3 = ((const float4 *)et)[3];
-    f3 c = mkf(r0.x, r0.y, r0.z), ex = mkf(r0.w, r1.x, r1.y);
-    f3 ey = mkf(r1.z, r1.w, r2.x), ez = mkf(r2.y, r2.z, r2.w);
-    const float hy = r3.x, hz = r3.y;
     f3 dp = subf(c, p);
     float kn = dotf(dp, ex);
     float kd = dotf(d, ex);
@@ -211,6 +210,15 @@ __device__ __forceinline__ bool plane_test32(const float *__restrict__ et, f3 p,
     ly = k * dotf(d, ey) - dotf(dp, ey);
     lz = k * dotf(d, ez) - dotf(dp, ez);
     return (kd != 0.0f) && (k >= kmin) && (fabsf(ly) <= hy) && (fabsf(lz) <= hz);
+}
+
+__device__ __forceinline__ bool plane_test32(const float *__restrict__ et, f3 p, f3 d, float kmin,
+                                             float &k, float &ly, float &lz) {
+    // records are 64-byte aligned: four 16-byte loads
+    const float4 r0 = ((const float4 *)et)[0], r1 = ((const float4 *)et)[1];
+    const float4 r2 = ((const float4 *)et)[2], r3 = ((const float4 *)et)[3];
+    return plane_math32(mkf(r0.x, r0.y, r0.z), mkf(r0.w, r1.x, r1.y), mkf(r1.z, r1.w, r2.x), mkf(r2.y, r2.z, r2.w),
+                        r3.x, r3.y, p, d, kmin, k, ly, lz);
 }
 
 __device__ __forceinline__ f3 ptrans32(f3 d1, f3 d2, f3 pol) {
@@ -1496,6 +1504,137 @@ __device__ __forceinline__ int scan_next(ETP et, bool list, ITP items, int tb, i
     return -1;
 }
 
+// ------------------------------------------- lens and detector interactions
+// PerfectLens.specific_process_photons, marxs/optics/mirror.py:53-82.  ep: the
+// element's parameters; refl: offset of its reflectivity record (-1: none).
+// Reflectivity is applied by the extended kernel only (tables with such a lens
+// set ext_stages); the plain kernel, which keeps the code out of its register
+// allocation, reports a record as a bad argument.
+template <int PREC, bool EXT, typename PP>
+__device__ __forceinline__ void lens_perfect(const MxTables &T, PP ep, int refl, d3 q, const Counters &cnt, Ray &R) {
+    d3 popt = ld3(ep);
+    double f = ep[6];
+    double ang;   // angle between the old and the new direction
+    if (!EXT && refl >= 0) {
+        count(cnt, MX_ST_BAD_ARGS);
+        refl = -1;
+    }
+    if (PREC == 64) {
+        d3 dn = unit3(R.d);
+        d3 fp = mk(popt.x + f * dn.x, popt.y + f * dn.y, popt.z + f * dn.z);
+        d3 nd = unit3(sub3(fp, q));
+        if (refl >= 0) ang = acos64<EXT>(fabs(dot3(nd, dn)));
+        R.pol = ptrans64(R.d, nd, R.pol);
+        R.d = nd;
+    } else {
+        f3 dn = unitf(R.df);
+        d3 fp = mk(popt.x + f * (double)dn.x, popt.y + f * (double)dn.y, popt.z + f * (double)dn.z);
+        f3 nd = unitf(tof(sub3(fp, q)));
+        if (refl >= 0) {
+            // atan2(|a x b|, |a . b|) keeps the digits of small angles
+            const f3 cr = crossf(nd, dn);
+            ang = (double)atan2f(sqrtf(dotf(cr, cr)), fabsf(dotf(nd, dn)));
+        }
+        R.polf = ptrans32(R.df, nd, R.polf);
+        R.df = nd;
+    }
+    if (refl >= 0) {
+        // probability *= reflectivity(energy, angle / 4) ** 2
+        // (mirror.py:72-82), a degree-1 tensor spline
+        const double r = lens_reflectivity(T.sel_d + refl, R.energy, ang / 4);
+        const double pf = r * r;
+        if (pf < 0.0 || pf > 1.0) count(cnt, MX_ST_PROB_RANGE);
+        R.prob = R.prob * pf;
+    }
+}
+
+template <int PREC, typename TP, typename PP>
+__device__ __forceinline__ void lens_thin(TP et, PP ep, d3 q, Ray &R) {
+    if (PREC == 64) {
+        thin_lens64(ld3(et), ep[6], q, R.d, R.pol);
+    } else {
+        d3 dd = tod(R.df), pp = tod(R.polf);
+        thin_lens64(ld3(et), ep[6], q, dd, pp);
+        R.df = tof(dd);
+        R.polf = tof(pp);
+    }
+}
+
+// FlatDetector, marxs/optics/detector.py:59-75.  et: the element's FP64 frame;
+// px: pixel size, centre pixels, 1 / pixel size; npx, npy: pixels.  The FP32
+// path forms the coordinate (and q, ly, lz) again in FP64.
+template <int PREC, typename SIP, typename TP, typename PP>
+__device__ __forceinline__ void detector_hit(const MxPhotons &P, SIP si, TP et, PP px, int npx, int npy, int64_t i,
+                                             d3 &q, double &ly, double &lz, const Ray &R) {
+    double dp0, dp1;
+    if (PREC == 32) {
+        // final detector coordinate in FP64
+        double y64, z64;
+        plane_hit64_fast(et, R.p, tod(R.df), q, y64, z64);
+        ly = y64; lz = z64;
+        const double ip = px[3];   // 1 / pixsize
+        dp0 = ly * ip + px[1];
+        dp1 = lz * ip + px[2];
+    } else {
+        dp0 = ly / px[0] + px[1];
+        dp1 = lz / px[0] + px[2];
+    }
+    put_f(P, si[15], i, dp0);
+    put_f(P, si[16], i, dp1);
+    put_i(P, si[17], i, pixel_index(dp0, npx));
+    put_i(P, si[18], i, pixel_index(dp1, npy));
+}
+
+// A lens or detector stage of one element without a culling grid: its records
+// are read with scalar loads.  In array_stage the element index is a lane's
+// own, so every lane loads the same words, and waits for the stores of the
+// stage before.
+template <int PREC, bool EXT>
+__device__ __forceinline__ void single_stage(const MxTables &T, const MxPhotons &P, const cptr<int> si,
+                                             const cptr<double> sd, const cptr<float> sf, const int64_t i,
+                                             const Counters &cnt, Ray &R) {
+    const int kind = si[0], e0 = si[2];
+    const cptr<double> et = cp(T.elem_t) + (size_t)e0 * MX_ET, ep = cp(T.elem_p) + (size_t)e0 * MX_EP;
+    const cptr<int> ei = cp(T.elem_i) + (size_t)e0 * MX_EI;
+    d3 q;
+    double ly, lz;
+    bool hit;
+    if (cnt.tests) count(cnt, MX_ST_TESTS);
+    if (PREC == 64) {
+        hit = plane_math64(ld3(et), ld3(et + 3), ld3(et + 6), ld3(et + 9), et[12], et[13], R.p, R.d, q, ly, lz);
+    } else {
+#pragma clang fp contract(fast)
+        const cptr<float> er = cp(T.elem_t32) + (size_t)e0 * MX_ET;
+        f3 r0 = tof(sub3(R.p, ld3(sd)));
+        f3 a = ldf3(sf);
+        float da = dotf(R.df, a), kadv = 0.0f;
+        if (da != 0.0f && da == da) {
+            kadv = fdiv_fast(-dotf(r0, a), da);
+            if (!(fabsf(kadv) < 1e30f)) kadv = 0.0f;
+        }
+        const f3 pr = mkf(r0.x + kadv * R.df.x, r0.y + kadv * R.df.y, r0.z + kadv * R.df.z);
+        float kf, yy, zz;
+        hit = plane_math32(ldf3(er), ldf3(er + 3), ldf3(er + 6), ldf3(er + 9), er[12], er[13], pr, R.df, -kadv, kf, yy,
+                           zz);
+        const float kk = kadv + kf;
+        ly = yy;
+        lz = zz;
+        q = mk(R.p.x + (double)kk * (double)R.df.x, R.p.y + (double)kk * (double)R.df.y,
+               R.p.z + (double)kk * (double)R.df.z);
+    }
+    if (!hit) {
+        put_defaults(P, si, i);
+        return;
+    }
+    if (kind == MX_STAGE_LENS_PERFECT) lens_perfect<PREC, EXT>(T, ep, ei[6], q, cnt, R);
+    else if (kind == MX_STAGE_LENS_THIN) lens_thin<PREC>(et, ep, q, R);
+    else detector_hit<PREC>(P, si, et, ep + 6, ei[4], ei[5], i, q, ly, lz, R);
+    put_f(P, si[10], i, ly);
+    put_f(P, si[11], i, lz);
+    put_i(P, si[12], i, ei[0]);
+    R.p = q;
+}
+
 // ------------------------------------------------------------- split trace
 // A trace can be split at one stack stage S: the first kernel runs every
 // stage with the plain kernel's code and, at S, stops each photon at its
@@ -1745,7 +1884,7 @@ __device__ __forceinline__ bool array_stage(const MxTables &T, const MxPhotons &
 
         // ---- interaction with element `hit`
         const size_t eg = (size_t)(e0 + hit);
-        const double *et = T.elem_t + eg * MX_ET;
+        const double *et = (L && PREC == 64) ? (const double *)rec_l + (size_t)hit * MX_ET : T.elem_t + eg * MX_ET;
         const double *ep = T.elem_p + eg * MX_EP;
         const int *ei = T.elem_i + eg * MX_EI;
         int id;
@@ -1820,77 +1959,23 @@ __device__ __forceinline__ bool array_stage(const MxTables &T, const MxPhotons &
             put_f(P, si[42], i, ly);
             put_f(P, si[43], i, lz);
         } else if (kind == MX_STAGE_DETECTOR) {
-            id = ei[0];
-            double dp0, dp1;
-            if (PREC == 32) {
-                // final detector coordinate in FP64
-                double y64, z64;
-                plane_hit64_fast(et, R.p, tod(R.df), q, y64, z64);
-                ly = y64; lz = z64;
-                const double ip = ep[9];   // 1 / pixsize
-                dp0 = ly * ip + ep[7];
-                dp1 = lz * ip + ep[8];
+            if (L && si[PREC == 64 ? 52 : 51] > 0) {
+                // frame, pixel parameters and ids of the element in LDS: read
+                // from global memory they wait for every store before them
+                const double *dr = (const double *)(lds + si[PREC == 64 ? 52 : 51]) + (size_t)hit * MX_DR;
+                const int *di = (const int *)(dr + 16);
+                id = di[0];
+                detector_hit<PREC>(P, si, dr, dr + 12, di[1], di[2], i, q, ly, lz, R);
             } else {
-                dp0 = ly / ep[6] + ep[7];
-                dp1 = lz / ep[6] + ep[8];
+                id = ei[0];
+                detector_hit<PREC>(P, si, et, ep + 6, ei[4], ei[5], i, q, ly, lz, R);
             }
-            put_f(P, si[15], i, dp0);
-            put_f(P, si[16], i, dp1);
-            put_i(P, si[17], i, pixel_index(dp0, ei[4]));
-            put_i(P, si[18], i, pixel_index(dp1, ei[5]));
         } else if (kind == MX_STAGE_LENS_PERFECT) {
-            // PerfectLens.specific_process_photons, mirror.py:53-82
             id = ei[0];
-            d3 popt = ld3(ep);
-            double f = ep[6];
-            double ang;   // angle between the old and the new direction
-            // offset of the reflectivity record (-1: none); a one-element
-            // stage reads it with a scalar load.  Reflectivity is applied by
-            // the extended kernel only (tables with such a lens set
-            // ext_stages); the plain kernel, which keeps the code out of its
-            // register allocation, reports a record as a bad argument.
-            int refl = n_el == 1 ? cp(T.elem_i)[(size_t)e0 * MX_EI + 6] : ei[6];
-            if (!EXT && refl >= 0) {
-                count(cnt, MX_ST_BAD_ARGS);
-                refl = -1;
-            }
-            if (PREC == 64) {
-                d3 dn = unit3(R.d);
-                d3 fp = mk(popt.x + f * dn.x, popt.y + f * dn.y, popt.z + f * dn.z);
-                d3 nd = unit3(sub3(fp, q));
-                if (refl >= 0) ang = acos64<EXT>(fabs(dot3(nd, dn)));
-                R.pol = ptrans64(R.d, nd, R.pol);
-                R.d = nd;
-            } else {
-                f3 dn = unitf(R.df);
-                d3 fp = mk(popt.x + f * (double)dn.x, popt.y + f * (double)dn.y, popt.z + f * (double)dn.z);
-                f3 nd = unitf(tof(sub3(fp, q)));
-                if (refl >= 0) {
-                    // atan2(|a x b|, |a . b|) keeps the digits of small angles
-                    const f3 cr = crossf(nd, dn);
-                    ang = (double)atan2f(sqrtf(dotf(cr, cr)), fabsf(dotf(nd, dn)));
-                }
-                R.polf = ptrans32(R.df, nd, R.polf);
-                R.df = nd;
-            }
-            if (refl >= 0) {
-                // probability *= reflectivity(energy, angle / 4) ** 2
-                // (mirror.py:72-82), a degree-1 tensor spline
-                const double r = lens_reflectivity(T.sel_d + refl, R.energy, ang / 4);
-                const double pf = r * r;
-                if (pf < 0.0 || pf > 1.0) count(cnt, MX_ST_PROB_RANGE);
-                R.prob = R.prob * pf;
-            }
+            lens_perfect<PREC, EXT>(T, ep, n_el == 1 ? cp(T.elem_i)[(size_t)e0 * MX_EI + 6] : ei[6], q, cnt, R);
         } else {  // MX_STAGE_LENS_THIN
             id = ei[0];
-            if (PREC == 64) {
-                thin_lens64(ld3(et), ep[6], q, R.d, R.pol);
-            } else {
-                d3 dd = tod(R.df), pp = tod(R.polf);
-                thin_lens64(ld3(et), ep[6], q, dd, pp);
-                R.df = tof(dd);
-                R.polf = tof(pp);
-            }
+            lens_thin<PREC>(et, ep, q, R);
         }
         // process_photons bookkeeping, optics/base.py:201-209
         put_f(P, si[10], i, ly);
@@ -1926,6 +2011,44 @@ __device__ __forceinline__ void init_ray(const MxTables &T, const MxPhotons &P, 
                     ? P.uniforms[(int64_t)T.first_draw_slot * P.uniform_stride + i] : 0.0;
 }
 
+// An aperture stage with its two draws (aperture.py:68-78,92-95,138-146).
+template <int PREC>
+__device__ __forceinline__ void aperture_stage(const MxTables &T, const MxPhotons &P, const cptr<int> si,
+                                               const double u0, const double u1, Ray &R) {
+    const int64_t i = R.i;
+    const int kind = si[0], e0 = si[2];
+    const cptr<double> et = cp(T.elem_t) + (size_t)e0 * MX_ET;
+    const cptr<double> ep = cp(T.elem_p) + (size_t)e0 * MX_EP;
+    double x, y, f;
+    if (kind == MX_STAGE_APERTURE_CIRCLE) {
+        if (PREC == 64) {
+            double phi = ep[6] + ep[7] * u0;
+            double r = sqrt(ep[8] + ep[9] * u1);
+            x = r * cos(phi);
+            y = r * sin(phi);
+        } else {
+            float phi = (float)ep[6] + (float)ep[7] * (float)u0;
+            float r = sqrtf((float)ep[8] + (float)ep[9] * (float)u1);
+            float sp, cp;
+            sincosf(phi, &sp, &cp);
+            x = (double)(r * cp);
+            y = (double)(r * sp);
+        }
+    } else {
+        x = u0 * 2. - 1.;
+        y = u1 * 2. - 1.;
+    }
+    d3 c = ld3(et), vy = ld3(ep), vz = ld3(ep + 3);
+    R.p = mk(c.x + x * vy.x + y * vz.x, c.y + x * vy.y + y * vz.y, c.z + x * vy.z + y * vz.z);
+    if (PREC == 64) f = dot3(R.d, ld3(ep + 10));
+    else f = (double)dotf(R.df, ldf3(cp(T.elem_p32) + (size_t)e0 * MX_EP + 10));
+    f = f < 0.0 ? 0.0 : (f > 1.0 ? 1.0 : f);
+    R.prob = R.prob * f;
+    put_f(P, si[10], i, x);
+    put_f(P, si[11], i, y);
+    put_i(P, si[12], i, cp(T.elem_i)[(size_t)e0 * MX_EI]);
+}
+
 // Stage s (wave-uniform) for one photon.
 template <int PREC, bool EXT, bool BZ = EXT>
 __device__ __forceinline__ void run_stage(const MxTables &T, const MxPhotons &P, const int s,
@@ -1937,39 +2060,9 @@ __device__ __forceinline__ void run_stage(const MxTables &T, const MxPhotons &P,
         const int kind = si[0], e0 = si[2];
 
         if (kind == MX_STAGE_APERTURE_CIRCLE || kind == MX_STAGE_APERTURE_RECT) {
-            // aperture.py:68-78,92-95,138-146
-            const cptr<double> et = cp(T.elem_t) + (size_t)e0 * MX_ET;
-            const cptr<double> ep = cp(T.elem_p) + (size_t)e0 * MX_EP;
-            double u0 = draw(T, P, R, si[4], si[5], 0, i, cnt);
-            double u1 = draw(T, P, R, si[4], si[5], 1, i, cnt);
-            double x, y, f;
-            if (kind == MX_STAGE_APERTURE_CIRCLE) {
-                if (PREC == 64) {
-                    double phi = ep[6] + ep[7] * u0;
-                    double r = sqrt(ep[8] + ep[9] * u1);
-                    x = r * cos(phi);
-                    y = r * sin(phi);
-                } else {
-                    float phi = (float)ep[6] + (float)ep[7] * (float)u0;
-                    float r = sqrtf((float)ep[8] + (float)ep[9] * (float)u1);
-                    float sp, cp;
-                    sincosf(phi, &sp, &cp);
-                    x = (double)(r * cp);
-                    y = (double)(r * sp);
-                }
-            } else {
-                x = u0 * 2. - 1.;
-                y = u1 * 2. - 1.;
-            }
-            d3 c = ld3(et), vy = ld3(ep), vz = ld3(ep + 3);
-            R.p = mk(c.x + x * vy.x + y * vz.x, c.y + x * vy.y + y * vz.y, c.z + x * vy.z + y * vz.z);
-            if (PREC == 64) f = dot3(R.d, ld3(ep + 10));
-            else f = (double)dotf(R.df, ldf3(cp(T.elem_p32) + (size_t)e0 * MX_EP + 10));
-            f = f < 0.0 ? 0.0 : (f > 1.0 ? 1.0 : f);
-            R.prob = R.prob * f;
-            put_f(P, si[10], i, x);
-            put_f(P, si[11], i, y);
-            put_i(P, si[12], i, cp(T.elem_i)[(size_t)e0 * MX_EI]);
+            const double u0 = draw(T, P, R, si[4], si[5], 0, i, cnt);
+            const double u1 = draw(T, P, R, si[4], si[5], 1, i, cnt);
+            aperture_stage<PREC>(T, P, si, u0, u1, R);
             return;
         }
         if (kind == MX_STAGE_CATSUPPORT) {
@@ -1988,7 +2081,12 @@ __device__ __forceinline__ void run_stage(const MxTables &T, const MxPhotons &P,
             count(cnt, MX_ST_BAD_ARGS);
             return;
         }
-        if (si[PREC == 64 ? 21 : 20] >= 0) array_stage<PREC, true, EXT, 0, BZ>(T, P, s, i, use_grid, cnt, lds, R);
+        if (si[1] == 1 && !(si[3] & 1) && (kind == MX_STAGE_LENS_PERFECT || kind == MX_STAGE_LENS_THIN ||
+                                           kind == MX_STAGE_DETECTOR))
+            single_stage<PREC, EXT>(T, P, si, cp(T.stage_d) + (size_t)s * MX_SD, cp(T.stage_f) + (size_t)s * MX_SD, i,
+                                    cnt, R);
+        else if (si[PREC == 64 ? 21 : 20] >= 0)
+            array_stage<PREC, true, EXT, 0, BZ>(T, P, s, i, use_grid, cnt, lds, R);
         else array_stage<PREC, false, EXT, 0, BZ>(T, P, s, i, use_grid, cnt, lds, R);
     }
 }
@@ -2010,8 +2108,20 @@ __device__ __forceinline__ void trace_one(const MxTables &T, const MxPhotons &P,
                                           const bool use_grid, const Counters &cnt,
                                           const unsigned char *lds) {
     Ray R;
+    // a first stage that is an aperture: its draws are loaded with the photon's
+    // columns (one wait, before the first store) and the stage runs before the
+    // loop, so that they are not held through it
+    const cptr<int> s0 = cp(T.stage_i);
+    const bool aper = T.n_stages > 0 && (s0[0] == MX_STAGE_APERTURE_CIRCLE || s0[0] == MX_STAGE_APERTURE_RECT) &&
+                      s0[5] >= 2;
+    double u0 = 0.0, u1 = 0.0;
+    if (aper) {
+        u0 = P.uniforms[(int64_t)s0[4] * P.uniform_stride + i];
+        u1 = P.uniforms[(int64_t)(s0[4] + 1) * P.uniform_stride + i];
+    }
     init_ray(T, P, i, R);
-    for (int s_ = 0; s_ < T.n_stages; ++s_) {
+    if (aper) aperture_stage<PREC>(T, P, s0, u0, u1, R);
+    for (int s_ = aper ? 1 : 0; s_ < T.n_stages; ++s_) {
         // the stage index is the same in every lane: keep it (and all stage
         // metadata derived from it) in scalar registers
         const int s = __builtin_amdgcn_readfirstlane(s_);
