@@ -52,17 +52,13 @@
 #ifndef MX_BLOCK_EXT32
 #define MX_BLOCK_EXT32 768      /* the FP32 kernels with stack or tube stages */
 #endif
-// Default workgroups per CU of the persistent grid (one resides at a time:
-// the LDS image; each stages it again), whose waves take chunks of 64
-// photons from their workgroup's share: measured on the 600-facet
-// workloads, 1e7 photons (FP32 / FP64 kernel ms at 1, 2, 4 per CU): plain
-// facets 0.944 0.925 0.943 / 1.301 1.309 1.326; interpolated efficiency
-// 0.984 0.976 0.994 / 1.498 1.507 1.533; CATL1L2Stack (extended kernel)
-// 1.931 1.938 1.956 / (split trace) 2.737 2.719 2.718; mirror scatter,
-// facets and Rowland tube (extended) 1.657 1.649 1.664 / 1.906 1.916 1.945.
-#define MX_DEFAULT_WG_PER_CU32 2
-#define MX_DEFAULT_WG_PER_CU64 1
-#define MX_DEFAULT_WG_PER_CU_EXT 1
+// Default workgroups per CU of the persistent grid.  One is resident at a time
+// (registers and the LDS image), and its waves share its photons evenly
+// (photon_chunks), so that every further one only stages the image again and
+// waits for its slowest wave again: 600 facets, FP32, 1 / 2 / 4 per CU: 3e5
+// photons 49 / 58 / 58 us, 2.5e6 219 / 232 / 256 us, 1e7 743 / 755 / 778 us;
+// FP64 2.5e6 326 / 338 / 359 us; CATL1L2Stack facets FP32 453 / 468 / 487 us.
+#define MX_DEFAULT_WG_PER_CU 1
 #ifndef MX_REGROUP_DEFAULT_FRAC
 #define MX_REGROUP_DEFAULT_FRAC 256  /* exchange when <= this/256 of the rays interact */
 #endif
@@ -2319,6 +2315,30 @@ __device__ __forceinline__ void trace_chunk(const MxTables &T, const MxPhotons &
     if (R.i >= 0) finish_ray<PREC>(P, R);
 }
 
+// The LDS image of a workgroup (up to 160 KB).  Loads of one work-item are
+// issued MX_STAGE at a time before the first of them is stored: one by one,
+// each waited for a trip to L2, 98 KB over 1024 work-items 5500 cycles.
+#define MX_STAGE 8
+template <int BS>
+__device__ __forceinline__ void stage_image(unsigned char *lds, const unsigned char *image, int bytes) {
+    const uint4 *src = (const uint4 *)image;
+    uint4 *dst = (uint4 *)lds;
+    const int nvec = (bytes + 15) >> 4;
+    for (int v = (int)threadIdx.x; v < nvec; v += MX_STAGE * BS) {
+        uint4 x[MX_STAGE];
+#pragma unroll
+        for (int k = 0; k < MX_STAGE; ++k) {
+            const int j = v + k * BS;
+            x[k] = src[j < nvec ? j : nvec - 1];
+        }
+#pragma unroll
+        for (int k = 0; k < MX_STAGE; ++k) {
+            const int j = v + k * BS;
+            if (j < nvec) dst[j] = x[k];
+        }
+    }
+}
+
 // The photon loop of a persistent workgroup: its contiguous share of the n
 // photons (rounded up to 64), in chunks of 64 consecutive photons, one per
 // lane, that its waves take in turn from an LDS counter (*next, zero before
@@ -2378,12 +2398,7 @@ __global__ __launch_bounds__(BS) void mx_trace_kernel(MxTables T_arg, MxPhotons 
     }
     const int lds_bytes = PREC == 64 ? T.lds_bytes64 : T.lds_bytes32;
     if (threadIdx.x < MX_NCOUNT) s_count[threadIdx.x] = 0;
-    if (lds_bytes > 0) {
-        const uint4 *src = (const uint4 *)(PREC == 64 ? T.lds_image64 : T.lds_image32);
-        uint4 *dst = (uint4 *)lds;
-        const int nvec = (lds_bytes + 15) >> 4;
-        for (int v = threadIdx.x; v < nvec; v += BS) dst[v] = src[v];
-    }
+    stage_image<BS>(lds, (const unsigned char *)(PREC == 64 ? T.lds_image64 : T.lds_image32), lds_bytes);
     __shared__ unsigned s_next;
     if (threadIdx.x == 0) s_next = 0;
     __syncthreads();
@@ -2499,12 +2514,8 @@ __device__ __forceinline__ void trace_one_split_b(const MxTables &T, const MxPho
     }                                                                                                   \
     const int lds_bytes = PREC == 64 ? T.lds_bytes64 : T.lds_bytes32;                                   \
     if (threadIdx.x < MX_NCOUNT) s_count[threadIdx.x] = 0;                                              \
-    if (lds_bytes > 0) {                                                                                \
-        const uint4 *src = (const uint4 *)(PREC == 64 ? T.lds_image64 : T.lds_image32);                 \
-        uint4 *dst = (uint4 *)lds;                                                                      \
-        const int nvec = (lds_bytes + 15) >> 4;                                                         \
-        for (int v = threadIdx.x; v < nvec; v += (BSZ)) dst[v] = src[v];                                \
-    }                                                                                                   \
+    stage_image<BSZ>(lds, (const unsigned char *)(PREC == 64 ? T.lds_image64 : T.lds_image32),          \
+                     lds_bytes);                                                                        \
     __syncthreads();                                                                                    \
     const Counters cnt = {s_count, (flags & MX_FLAG_COUNT_TESTS) != 0};                                 \
     const bool use_grid = !(flags & MX_FLAG_NO_GRID)
@@ -2595,12 +2606,7 @@ __global__ __launch_bounds__(BS) void mx_trace_regroup_kernel(MxTables T_arg, Mx
     }
     const int lds_bytes = PREC == 64 ? T.lds_bytes64 : T.lds_bytes32;
     if (threadIdx.x < MX_NCOUNT) s_count[threadIdx.x] = 0;
-    if (lds_bytes > 0) {
-        const uint4 *src = (const uint4 *)(PREC == 64 ? T.lds_image64 : T.lds_image32);
-        uint4 *dst = (uint4 *)lds;
-        const int nvec = (lds_bytes + 15) >> 4;
-        for (int v = threadIdx.x; v < nvec; v += BS) dst[v] = src[v];
-    }
+    stage_image<BS>(lds, (const unsigned char *)(PREC == 64 ? T.lds_image64 : T.lds_image32), lds_bytes);
     __syncthreads();
     const Counters cnt = {s_count, (flags & MX_FLAG_COUNT_TESTS) != 0};
     const bool use_grid = !(flags & MX_FLAG_NO_GRID);
@@ -2659,12 +2665,7 @@ __global__ __launch_bounds__(BS) void mx_trace_batched_kernel(
         const MxPhotons &P = *(const MxPhotons *)((const __attribute__((address_space(4))) MxPhotons *)phs + v);
         if (v != cur) {
             const int nb = PREC == 64 ? T.lds_bytes64 : T.lds_bytes32;
-            if (nb > 0) {
-                const uint4 *src = (const uint4 *)(PREC == 64 ? T.lds_image64 : T.lds_image32);
-                uint4 *dst = (uint4 *)lds;
-                const int nvec = (nb + 15) >> 4;
-                for (int k = threadIdx.x; k < nvec; k += BS) dst[k] = src[k];
-            }
+            stage_image<BS>(lds, (const unsigned char *)(PREC == 64 ? T.lds_image64 : T.lds_image32), nb);
             cur = v;
             __syncthreads();
         }
@@ -2789,9 +2790,7 @@ extern "C" int mx_trace(const MxTables *tables, const MxPhotons *photons, int32_
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) cus = 0;
     if (cus <= 0) cus = 256;
     int per_cu = (flags >> 8) & 0xff;   // workgroups per CU; 0 = default
-    if (per_cu <= 0)
-        per_cu = ext ? MX_DEFAULT_WG_PER_CU_EXT
-                     : (precision == MX_PREC_FP64 ? MX_DEFAULT_WG_PER_CU64 : MX_DEFAULT_WG_PER_CU32);
+    if (per_cu <= 0) per_cu = MX_DEFAULT_WG_PER_CU;
     int64_t grid = (int64_t)cus * per_cu;
     if (grid > nblk) grid = nblk;
     // regrouping: the exchange buffer after the LDS image, at least 64 ray
@@ -2823,6 +2822,14 @@ extern "C" int mx_trace(const MxTables *tables, const MxPhotons *photons, int32_
             }
             return 0;
         }
+    }
+    // Fewer photons than the work-items of one workgroup per CU: spread their
+    // chunks of 64 over the CUs instead of filling one CU after another, so
+    // that fewer waves share a CU: 600 facets FP64, 3e4 photons 34 -> 27 us,
+    // 1e5 37 -> 32 us; with mirror scatter and tube 45 -> 34, 49 -> 42 us.
+    if (grid < cus) {
+        const int64_t chunks = (photons->n + 63) / 64;
+        grid = chunks < cus ? chunks : cus;
     }
     if (precision == MX_PREC_FP64 && ext)
         hipLaunchKernelGGL((mx_trace_kernel<64, MX_BLOCK_EXT, true>), dim3((unsigned)grid), dim3(block), lds, st,
@@ -2887,7 +2894,7 @@ extern "C" int mx_trace_split(const MxTables *tables, const MxPhotons *photons, 
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) cus = 0;
     if (cus <= 0) cus = 256;
     int per_cu = (flags >> 8) & 0xff;
-    if (per_cu <= 0) per_cu = precision == MX_PREC_FP64 ? MX_DEFAULT_WG_PER_CU64 : MX_DEFAULT_WG_PER_CU32;
+    if (per_cu <= 0) per_cu = MX_DEFAULT_WG_PER_CU;
     hipStream_t st = (hipStream_t)stream;
     // the queue counters start at zero (a fill kernel, so that the call can
     // be captured in a graph)
