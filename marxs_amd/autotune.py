@@ -58,7 +58,7 @@ def tune_trace(ci, dp, uniforms, precision=32, candidates=(1, 2, 3, 4), reps=5, 
 def _batched_candidates(bt):
     from .batch import BLOCK, BLOCK_EXT
     bs = BLOCK_EXT if bt.ext_stages else BLOCK[bt.precision]
-    out = []
+    out = [{'tile_photons': None, 'scale_by_cost': False, 'order': 'cost', 'wg_per_cu': 1}]
     for mult in (1, 2, 4, 8):
         for scaled in (False, True):
             out.append({'tile_photons': bs * mult, 'scale_by_cost': scaled, 'order': 'cost',
