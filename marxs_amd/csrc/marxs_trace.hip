@@ -173,6 +173,12 @@ __device__ __forceinline__ float dotf(f3 a, f3 b) {
 #pragma clang fp contract(fast)
     return a.x * b.x + a.y * b.y + a.z * b.z;
 }
+// The same fused in a fixed order: left to the compiler, which of the first two
+// products is rounded can differ from one kernel to the next, and kernels that
+// decide on the same rays have to agree.
+__device__ __forceinline__ float dotf_fused(f3 a, f3 b) {
+    return __builtin_fmaf(a.z, b.z, __builtin_fmaf(a.y, b.y, a.x * b.x));
+}
 __device__ __forceinline__ f3 subf(f3 a, f3 b) { return mkf(a.x - b.x, a.y - b.y, a.z - b.z); }
 __device__ __forceinline__ f3 crossf(f3 a, f3 b) {
 #pragma clang fp contract(fast)
@@ -242,6 +248,12 @@ __device__ __forceinline__ f3 ptrans32(f3 d1, f3 d2, f3 pol) {
 // loads even though the kernel writes other global memory.
 template <typename T> using cptr = const __attribute__((address_space(4))) T *;
 template <typename T> __device__ __forceinline__ cptr<T> cp(const T *p) { return (cptr<T>)p; }
+
+// Waits here for the load that x comes from.  Loads and stores share one
+// counter that counts down in order; where a branch that loads joins one that
+// does not, the compiler waits for the counter to reach zero, and with it for
+// all the stores issued since, on both paths.
+template <typename V> __device__ __forceinline__ void arrived(V &x) { asm volatile("" : "+v"(x)); }
 
 // Status counters of a workgroup, in LDS (indices MX_ST_*).  An event is
 // counted once per wave: the first active lane adds the number of active
@@ -645,6 +657,10 @@ struct Ray {
     double prob, energy;
     double u_first;      // prefetched first grating draw
     int64_t i;           // photon index (-1: no photon)
+    // the id column the last array stage wrote for every photon (-1: none) and
+    // whether this photon's entry is negative (the extended kernels)
+    int id_col = -1;
+    bool no_id = false;
 };
 
 // Uniform slot of the k-th interaction of a photon inside one stage.
@@ -691,7 +707,14 @@ __device__ __forceinline__ void thin_lens64(d3 c, double f, d3 q, d3 &d, d3 &pol
 __device__ __noinline__ double acos_call(double x) { return acos(x); }
 __device__ __noinline__ double asin_call(double x) { return asin(x); }
 __device__ __noinline__ double sin_call(double x) { return sin(x); }
-__device__ __noinline__ double cos_call(double x) { return cos(x); }
+// sin and cos of one angle: the same bits as sin(x) and cos(x), with one range
+// reduction and one pair of polynomials instead of two.
+__device__ __noinline__ double2 sincos_call(double x) {
+    double s, c;
+    sincos(x, &s, &c);
+    return make_double2(s, c);
+}
+__device__ __noinline__ double fmod_call(double x, double y) { return fmod(x, y); }
 __device__ __noinline__ double pow_call(double x, double y) { return pow(x, y); }
 __device__ __noinline__ double atan2_call(double y, double x) { return atan2(y, x); }
 // Inverse of the standard normal CDF (the scatter's normal deviate from a
@@ -950,7 +973,8 @@ __device__ __forceinline__ double l1_transmission(const MxTables &T, const unsig
 __device__ __forceinline__ d3 axangle_t(d3 ax, double ang, d3 v) {
     ax = unit3(ax);
     const double x = ax.x, y = ax.y, z = ax.z;
-    const double c = cos_call(ang), s = sin_call(ang), C = 1 - c;
+    const double2 sc = sincos_call(ang);
+    const double c = sc.y, s = sc.x, C = 1 - c;
     const double xs = x * s, ys = y * s, zs = z * s;
     const double xC = x * C, yC = y * C, zC = z * C;
     const double xyC = x * yC, yzC = y * zC, zxC = z * xC;
@@ -960,6 +984,35 @@ __device__ __forceinline__ d3 axangle_t(d3 ax, double ang, d3 v) {
     return mk(m00 * v.x + m10 * v.y + m20 * v.z,
               m01 * v.x + m11 * v.y + m21 * v.z,
               m02 * v.x + m12 * v.y + m22 * v.z);
+}
+
+// What a radial scatter layer reads of its stack record: the widths (words 13
+// and 16) and the centre (17-19).  In a stage of one element (a mirror's
+// scatter) the record is the same in every lane: scalar loads, which do not
+// wait for the stores of the stages before.
+struct Radial {
+    double s_in, s_perp;
+    d3 c;
+};
+__device__ __forceinline__ Radial radial_record(const MxTables &T, const cptr<int> si, const int *ei) {
+    Radial r;
+    if (si[1] == 1) {
+        const cptr<double> sr = cp(T.sel_d) + cp(T.elem_i)[(size_t)si[2] * MX_EI + 6];
+        r.s_in = sr[13];
+        r.s_perp = sr[16];
+        r.c = ld3(sr + 17);
+    } else {
+        const cptr<double> sr = cp(T.sel_d) + ei[6];
+        r.s_in = sr[13];
+        r.s_perp = sr[16];
+        r.c = ld3(sr + 17);
+        arrived(r.s_in);
+        arrived(r.s_perp);
+        arrived(r.c.x);
+        arrived(r.c.y);
+        arrived(r.c.z);
+    }
+    return r;
 }
 
 // The draws of one stack interaction (slots 5 k + j, j = 0 membrane order,
@@ -972,9 +1025,8 @@ struct StackDraws {
     double u[MX_STACK_DRAWS];
     bool scat;   // the stack has a scatter layer
 };
-template <typename SRP>
 __device__ __forceinline__ StackDraws stack_draws(const MxTables &T, const MxPhotons &P, const Ray &R,
-                                                  const cptr<int> si, int prog, SRP sr, int k0, int64_t i,
+                                                  const cptr<int> si, int prog, const int *ei, int k0, int64_t i,
                                                   const Counters &cnt) {
     unsigned ops = 0;
     for (int k = 0; k < (prog & 15); ++k) ops |= 1u << ((prog >> (4 + 3 * k)) & 7);
@@ -990,8 +1042,9 @@ __device__ __forceinline__ StackDraws stack_draws(const MxTables &T, const MxPho
         D.u[3] = draw(T, P, R, si[4], si[5], k0 + 3, i, cnt);
         D.u[4] = draw(T, P, R, si[4], si[5], k0 + 4, i, cnt);
     } else if (ops & (1u << MX_OP_RADIAL)) {
-        if (sr[13] != 0.0) D.u[3] = draw(T, P, R, si[4], si[5], k0 + 3, i, cnt);
-        if (sr[16] != 0.0) D.u[4] = draw(T, P, R, si[4], si[5], k0 + 4, i, cnt);
+        const Radial rr = radial_record(T, si, ei);
+        if (rr.s_in != 0.0) D.u[3] = draw(T, P, R, si[4], si[5], k0 + 3, i, cnt);
+        if (rr.s_perp != 0.0) D.u[4] = draw(T, P, R, si[4], si[5], k0 + 4, i, cnt);
     }
     return D;
 }
@@ -1036,7 +1089,7 @@ __device__ __forceinline__ void stack_layers(const MxTables &T, const MxPhotons 
     // the quality factor's order: the membrane's, or (no grating layer before
     // it) the photon's order column stage_i[49]
     int m_last = si[49] >= 0 ? P.icol[si[49]][i] : MX_ORDER_NONE;
-    const StackDraws D = stack_draws(T, P, R, si, prog, sr, k0, i, cnt);
+    const StackDraws D = stack_draws(T, P, R, si, prog, ei, k0, i, cnt);
     const int nops = prog & 15;
     for (int k = 0; k < nops; ++k) {
         const int op = (prog >> (4 + 3 * k)) & 7;
@@ -1108,16 +1161,17 @@ __device__ __forceinline__ void stack_layers(const MxTables &T, const MxPhotons 
             d = nd;
             put_f(P, si[46], i, ang);
         } else if (op == MX_OP_RADIAL) {
-            const d3 radial = sub3(R.p, ld3(sr + 17));
+            const Radial rr = radial_record(T, si, ei);
+            const d3 radial = sub3(R.p, rr.c);
             const d3 perpplane = cross3(d, radial);
             d3 nd = d;
             double a_in = 0.0, a_perp = 0.0;
-            if (sr[13] != 0.0) {
-                a_in = inv_normal_cdf(D.scat ? draw(T, P, R, si[4], si[5], k0 + 3, i, cnt) : D.u[3]) * sr[13];
+            if (rr.s_in != 0.0) {
+                a_in = inv_normal_cdf(D.scat ? draw(T, P, R, si[4], si[5], k0 + 3, i, cnt) : D.u[3]) * rr.s_in;
                 nd = axangle_t(perpplane, a_in, d);
             }
-            if (sr[16] != 0.0) {
-                a_perp = inv_normal_cdf(D.scat ? draw(T, P, R, si[4], si[5], k0 + 4, i, cnt) : D.u[4]) * sr[16];
+            if (rr.s_perp != 0.0) {
+                a_perp = inv_normal_cdf(D.scat ? draw(T, P, R, si[4], si[5], k0 + 4, i, cnt) : D.u[4]) * rr.s_perp;
                 nd = axangle_t(radial, a_perp, nd);
             }
             pol = ptrans64(d, nd, pol);
@@ -1189,7 +1243,7 @@ __device__ __forceinline__ void stack_layers32(const MxTables &T, const MxPhoton
     const double energy = R.energy;
     const int k0 = MX_STACK_DRAWS * nhit;
     int m_last = si[49] >= 0 ? P.icol[si[49]][i] : MX_ORDER_NONE;
-    const StackDraws D = stack_draws(T, P, R, si, prog, sr, k0, i, cnt);
+    const StackDraws D = stack_draws(T, P, R, si, prog, ei_, k0, i, cnt);
     const int nops = prog & 15;
     for (int k = 0; k < nops; ++k) {
         const int op = (prog >> (4 + 3 * k)) & 7;
@@ -1304,18 +1358,19 @@ __device__ __forceinline__ void stack_layers32(const MxTables &T, const MxPhoton
             R.df = nd;
             put_f(P, si[46], i, (double)ang);
         } else if (op == MX_OP_RADIAL) {
-            const f3 radial = tof(sub3(R.p, ld3(sr + 17)));
+            const Radial rr = radial_record(T, si, ei_);
+            const f3 radial = tof(sub3(R.p, rr.c));
             const f3 perpplane = crossf(R.df, radial);
             f3 nd = R.df;
             float a_in = 0.0f, a_perp = 0.0f;
-            if (sr[13] != 0.0) {
+            if (rr.s_in != 0.0) {
                 a_in = inv_normal_cdf32(D.scat ? draw(T, P, R, si[4], si[5], k0 + 3, i, cnt) : D.u[3]) *
-                       (float)sr[13];
+                       (float)rr.s_in;
                 nd = axangle_t32(perpplane, a_in, R.df);
             }
-            if (sr[16] != 0.0) {
+            if (rr.s_perp != 0.0) {
                 a_perp = inv_normal_cdf32(D.scat ? draw(T, P, R, si[4], si[5], k0 + 4, i, cnt) : D.u[4]) *
-                         (float)sr[16];
+                         (float)rr.s_perp;
                 nd = axangle_t32(radial, a_perp, nd);
             }
             R.polf = ptrans32(R.df, nd, R.polf);
@@ -1330,8 +1385,12 @@ __device__ __forceinline__ void stack_layers32(const MxTables &T, const MxPhoton
 
 // ------------------------------------------------------------ tube stages
 // numpy's floor modulo (the sign of the divisor), as Python's % on floats.
+// fmod(a, b) is a for |a| < b, and |a| - b (exact) with the sign of a for
+// b <= |a| < 2 b: one subtraction where the library reduces bit by bit.
 __device__ __forceinline__ double pymod(double a, double b) {
-    double m = fmod(a, b);
+    const double x = fabs(a);
+    double m = a;
+    if (!(x < b)) m = x < 2 * b ? copysign(x - b, a) : fmod_call(a, b);
     if (m != 0.0) {
         if ((b < 0.0) != (m < 0.0)) m += b;
     } else {
@@ -1349,7 +1408,8 @@ __device__ __forceinline__ bool angle_between(double ang, double b1, double b2) 
 }
 
 // m (3 rows of a row-major 4x4) applied to (v, w), summed in index order.
-__device__ __forceinline__ d3 aff3(const double *m, d3 v, double w) {
+template <typename MP>
+__device__ __forceinline__ d3 aff3(MP m, d3 v, double w) {
     return mk(((m[0] * v.x + m[1] * v.y) + m[2] * v.z) + m[3] * w,
               ((m[4] * v.x + m[5] * v.y) + m[6] * v.z) + m[7] * w,
               ((m[8] * v.x + m[9] * v.y) + m[10] * v.z) + m[11] * w);
@@ -1361,7 +1421,10 @@ __device__ __forceinline__ d3 aff3(const double *m, d3 v, double w) {
 // of two hits the nearer one counts.  cr: tube record (inverse pose,
 // pose, R, z zoom, limits, pixel size, centre pixel).  Returns the global
 // point, phi and z in global units.
-__device__ __forceinline__ bool tube_hit(const double *cr, d3 p, d3 d, d3 &q, double &phi, double &z) {
+// The azimuth is the expensive test (an arc tangent of about 140 instructions
+// and two modulos), so it is made for the nearer of the roots that pass the
+// others, and for the second one only in lanes where the first fails.
+__device__ __forceinline__ bool tube_hit(cptr<double> cr, d3 p, d3 d, d3 &q, double &phi, double &z) {
     const d3 xyz = aff3(cr, p, 1.0), dl = aff3(cr, d, 0.0);
     const double x = xyz.x, y = xyz.y, rx = dl.x, ry = dl.y;
     const double c = (x * x + y * y) - 1.;
@@ -1372,17 +1435,22 @@ __device__ __forceinline__ bool tube_hit(const double *cr, d3 p, d3 d, d3 &q, do
     const double denom = 2 * a;
     const double root = sqrt(under);
     const double a1 = (-b + root) / denom, a2 = (-b - root) / denom;
-    const double phi1 = atan2_call(y + a1 * ry, x + a1 * rx);
-    const double phi2 = atan2_call(y + a2 * ry, x + a2 * rx);
     const double z1 = xyz.z + a1 * dl.z, z2 = xyz.z + a2 * dl.z;
-    bool h1 = (a1 >= 0.0) && (fabs(z1) <= 1.) && angle_between(phi1, cr[34], cr[35]);
-    bool h2 = (a2 >= 0.0) && (fabs(z2) <= 1.) && angle_between(phi2, cr[34], cr[35]);
-    if (h2 && a2 < a1) h1 = false;
-    if (h1 && a2 >= a1) h2 = false;
-    if (!(h1 || h2)) return false;
-    const double t = h1 ? a1 : a2;
-    phi = h1 ? phi1 : phi2;
-    z = (h1 ? z1 : z2) * cr[33];
+    const bool g1 = (a1 >= 0.0) && (fabs(z1) <= 1.), g2 = (a2 >= 0.0) && (fabs(z2) <= 1.);
+    bool second = g2 && (a2 < a1 || !g1);   // the root tested: a2, or a1
+    bool left = g1 && g2;                   // the other one is left
+    bool hit = g1 || g2;
+    double t = second ? a2 : a1;
+    while (hit) {
+        phi = atan2_call(y + t * ry, x + t * rx);
+        if (angle_between(phi, cr[34], cr[35])) break;
+        hit = left;
+        left = false;
+        second = !second;
+        t = second ? a2 : a1;
+    }
+    if (!hit) return false;
+    z = (second ? z2 : z1) * cr[33];
     q = aff3(cr + 16, mk(x + t * rx, y + t * ry, xyz.z + t * dl.z), 1.0);
     return true;
 }
@@ -1398,8 +1466,10 @@ __device__ __forceinline__ void tube_stage(const MxTables &T, const MxPhotons &P
     const d3 d = PREC == 64 ? R.d : tod(R.df);
     int nhit = 0;
     for (int j = 0; j < n_el; ++j) {
-        const int *ei = T.elem_i + (size_t)(e0 + j) * MX_EI;
-        const double *cr = T.sel_d + ei[6];
+        // the element is the same in every lane: scalar loads, which do not
+        // wait for the stores of the stages before
+        const cptr<int> ei = cp(T.elem_i) + (size_t)(e0 + j) * MX_EI;
+        const cptr<double> cr = cp(T.sel_d) + ei[6];
         d3 q;
         double phi, z;
         if (!tube_hit(cr, R.p, d, q, phi, z)) continue;
@@ -1770,6 +1840,7 @@ __device__ __forceinline__ bool array_stage(const MxTables &T, const MxPhotons &
     const int *ssl_g = T.succ_start + si[34];
     const int *sul_g = T.succ_items + si[35];
     int last = -1, nhit = 0;
+    bool no_id = true;
     for (;;) {
         d3 q;
         double ly, lz;
@@ -1794,7 +1865,7 @@ __device__ __forceinline__ bool array_stage(const MxTables &T, const MxPhotons &
             f3 a = ldf3(sf);
             float da = dotf(R.df, a);
             if (da != 0.0f && da == da) {
-                kadv = fdiv_fast(-dotf(r0, a), da);
+                kadv = fdiv_fast(-dotf_fused(r0, a), da);
                 if (!(fabsf(kadv) < 1e30f)) kadv = 0.0f;
             }
             pr = mkf(r0.x + kadv * R.df.x, r0.y + kadv * R.df.y, r0.z + kadv * R.df.z);
@@ -1859,6 +1930,22 @@ __device__ __forceinline__ bool array_stage(const MxTables &T, const MxPhotons &
             else
                 hit = scan_next<PREC>(rec_l, list, items_g, tb, te, last,
                                       R.p, R.d, pr, R.df, kmin32, q, ly, lz, kf, cnt);
+        } else if (EXT && n_el == 1 && !list) {
+            // one element: its record is the same in every lane (scalar loads)
+            if (cnt.tests) count(cnt, MX_ST_TESTS);
+            bool on;
+            if (PREC == 64) {
+                const cptr<double> e1 = cp(T.elem_t) + (size_t)e0 * MX_ET;
+                on = plane_math64(ld3(e1), ld3(e1 + 3), ld3(e1 + 6), ld3(e1 + 9), e1[12], e1[13], R.p, R.d, q, ly, lz);
+            } else {
+                const cptr<float> e1 = cp(T.elem_t32) + (size_t)e0 * MX_ET;
+                float yy, zz;
+                on = plane_math32(ldf3(e1), ldf3(e1 + 3), ldf3(e1 + 6), ldf3(e1 + 9), e1[12], e1[13], pr, R.df, kmin32,
+                                  kf, yy, zz);
+                ly = yy;
+                lz = zz;
+            }
+            hit = on ? 0 : -1;
         } else if (PREC == 64) {
             hit = scan_next<PREC>(T.elem_t + (size_t)e0 * MX_ET, list, items_g,
                                   tb, te, last, R.p, R.d, pr, R.df, kmin32, q, ly, lz, kf, cnt);
@@ -1944,7 +2031,7 @@ __device__ __forceinline__ bool array_stage(const MxTables &T, const MxPhotons &
             put_i(P, si[13], i, m);
             put_f(P, si[14], i, blaze);
         } else if (EXT && kind == MX_STAGE_STACK) {
-            id = ei[0];
+            id = n_el == 1 ? cp(T.elem_i)[(size_t)e0 * MX_EI] : ei[0];
             if (PREC == 32) {
                 const float *er = L ? (const float *)rec_l + (size_t)hit * MX_ET : T.elem_t32 + eg * MX_ET;
                 const float *pl = (L && si[22] >= 0) ? (const float *)(lds + si[22]) + (size_t)hit * 16 : nullptr;
@@ -1977,12 +2064,19 @@ __device__ __forceinline__ bool array_stage(const MxTables &T, const MxPhotons &
         put_f(P, si[10], i, ly);
         put_f(P, si[11], i, lz);
         put_i(P, si[12], i, id);
+        no_id = id < 0;
         R.p = q;
         last = hit;
         ++nhit;
         if (last >= n_el - 1) break;
     }
     if (nhit == 0) put_defaults(P, si, i);
+    if (EXT) {
+        // every photon has an entry when the stage creates the column (-1
+        // where it met no element)
+        R.id_col = (si[19] & 4) ? si[12] : -1;
+        R.no_id = no_id;
+    }
     return false;
 }
 
@@ -2054,6 +2148,7 @@ __device__ __forceinline__ void run_stage(const MxTables &T, const MxPhotons &P,
     {
         const cptr<int> si = cp(T.stage_i) + (size_t)s * MX_SI;
         const int kind = si[0], e0 = si[2];
+        if (EXT && kind != MX_STAGE_CATSUPPORT) R.id_col = -1;
 
         if (kind == MX_STAGE_APERTURE_CIRCLE || kind == MX_STAGE_APERTURE_RECT) {
             const double u0 = draw(T, P, R, si[4], si[5], 0, i, cnt);
@@ -2066,7 +2161,14 @@ __device__ __forceinline__ void run_stage(const MxTables &T, const MxPhotons &P,
             // the facet frame absorbs photons that met no facet; si[6] is
             // the facet id column, written by an earlier stage of this trace
             const int c = si[6];
-            if (c < 0 || P.icol[c][i] < 0) R.prob = 0.0;
+            bool off = true;
+            if (c >= 0) {
+                // written by the array stage just before: not read back, which
+                // would wait for its stores and then for the load
+                if (EXT && R.id_col == c) off = R.no_id;
+                else off = P.icol[c][i] < 0;
+            }
+            if (off) R.prob = 0.0;
             return;
         }
         if (EXT && kind == MX_STAGE_CYLINDER) {
@@ -2167,7 +2269,7 @@ __device__ __forceinline__ bool stage_may_hit(const MxTables &T, const int s, co
         float da = dotf(R.df, a);
         float kadv = 0.0f;
         if (da != 0.0f && da == da) {
-            kadv = fdiv_fast(-dotf(r0, a), da);
+            kadv = fdiv_fast(-dotf_fused(r0, a), da);
             if (!(fabsf(kadv) < 1e30f)) kadv = 0.0f;
         }
         const f3 pr = mkf(r0.x + kadv * R.df.x, r0.y + kadv * R.df.y, r0.z + kadv * R.df.z);
@@ -2311,6 +2413,7 @@ __device__ __forceinline__ void trace_chunk(const MxTables &T, const MxPhotons &
             if (!run && R.i >= 0) put_defaults(P, cp(T.stage_i) + (size_t)s * MX_SI, R.i);
         }
         if (run) run_stage<PREC, EXT>(T, P, s, use_grid, cnt, lds, R);
+        R.id_col = -1;   // rays change lanes between stages
     }
     if (R.i >= 0) finish_ray<PREC>(P, R);
 }
