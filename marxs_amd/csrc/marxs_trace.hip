@@ -87,10 +87,33 @@ __device__ __forceinline__ d3 sub3(d3 a, d3 b) { return mk(a.x - b.x, a.y - b.y,
 __device__ __forceinline__ d3 cross3(d3 a, d3 b) {
     return mk(a.y * b.z - a.z * b.y, a.z * b.x - a.x * b.z, a.x * b.y - a.y * b.x);
 }
+// Several quotients with one divisor.  A double division is eleven
+// instructions: two that scale, a reciprocal with two Newton steps of the
+// divisor alone, and a quotient with one correction from its exact remainder.
+// Divisor does the steps of the divisor once, so that each quotient takes four.
+// The steps are those of `/` without the scaling, and so are the bits unless
+// the numerator, the divisor or the remainder comes near the ends of the
+// exponent range (below 1e-290 or above 1e290); zeros, infinities and NaN are
+// put right by the last instruction as in `/`.  2.5e6 photons, 600 facets with
+// an interpolated efficiency 374 -> 364 us; 1e6 through mirror scatter, facets
+// and tube 299 -> 294 us a call.
+struct Divisor {
+    double d, r;
+    __device__ __forceinline__ explicit Divisor(double d_) : d(d_) {
+        double x = __builtin_amdgcn_rcp(d);
+        x = __builtin_fma(x, __builtin_fma(-d, x, 1.0), x);
+        r = __builtin_fma(x, __builtin_fma(-d, x, 1.0), x);
+    }
+    // x / d
+    __device__ __forceinline__ double of(double x) const {
+        const double q = x * r;
+        return __builtin_amdgcn_div_fixup(__builtin_fma(__builtin_fma(-d, q, x), r, q), d, x);
+    }
+    __device__ __forceinline__ d3 of(d3 v) const { return mk(of(v.x), of(v.y), of(v.z)); }
+};
 // norm_vector (marxs/math/utils.py:150-164): v / sqrt(sum v*v)
 __device__ __forceinline__ d3 unit3(d3 v) {
-    double n = sqrt(v.x * v.x + v.y * v.y + v.z * v.z);
-    return mk(v.x / n, v.y / n, v.z / n);
+    return Divisor(sqrt(v.x * v.x + v.y * v.y + v.z * v.z)).of(v);
 }
 
 // FinitePlane.intersect, marxs/math/geometry.py:233-253
@@ -148,7 +171,7 @@ __device__ __forceinline__ d3 ptrans64(d3 d1, d3 d2, d3 pol) {
         if (sn != sn) return mk(NAN, NAN, NAN);
         return pol;
     }
-    s = mk(s.x / sn, s.y / sn, s.z / sn);
+    s = Divisor(sn).of(s);
     d3 pin = cross3(a, s), pout = cross3(b, s);
     // pmat[j][l] = s_j s_l + pout_j pin_l + b_j a_l ; out_j = sum_l pmat[j][l] pol_l
     double m00 = s.x * s.x + pout.x * pin.x + b.x * a.x;
@@ -1434,7 +1457,8 @@ __device__ __forceinline__ bool tube_hit(cptr<double> cr, d3 p, d3 d, d3 &q, dou
     if (!(under >= 0.0)) return false;
     const double denom = 2 * a;
     const double root = sqrt(under);
-    const double a1 = (-b + root) / denom, a2 = (-b - root) / denom;
+    const Divisor by(denom);
+    const double a1 = by.of(-b + root), a2 = by.of(-b - root);
     const double z1 = xyz.z + a1 * dl.z, z2 = xyz.z + a2 * dl.z;
     const bool g1 = (a1 >= 0.0) && (fabs(z1) <= 1.), g2 = (a2 >= 0.0) && (fabs(z2) <= 1.);
     bool second = g2 && (a2 < a1 || !g1);   // the root tested: a2, or a1
@@ -1474,8 +1498,9 @@ __device__ __forceinline__ void tube_stage(const MxTables &T, const MxPhotons &P
         double phi, z;
         if (!tube_hit(cr, R.p, d, q, phi, z)) continue;
         if (nhit > 0) count(cnt, MX_ST_MULTI_HIT);
-        put_f(P, si[15], i, phi * cr[32] / cr[36] + cr[37]);
-        put_f(P, si[16], i, z / cr[36] + cr[38]);
+        const Divisor size(cr[36]);
+        put_f(P, si[15], i, size.of(phi * cr[32]) + cr[37]);
+        put_f(P, si[16], i, size.of(z) + cr[38]);
         put_f(P, si[10], i, phi);
         put_f(P, si[11], i, z);
         put_i(P, si[12], i, ei[0]);
@@ -1642,8 +1667,9 @@ __device__ __forceinline__ void detector_hit(const MxPhotons &P, SIP si, TP et, 
         dp0 = ly * ip + px[1];
         dp1 = lz * ip + px[2];
     } else {
-        dp0 = ly / px[0] + px[1];
-        dp1 = lz / px[0] + px[2];
+        const Divisor size(px[0]);
+        dp0 = size.of(ly) + px[1];
+        dp1 = size.of(lz) + px[2];
     }
     put_f(P, si[15], i, dp0);
     put_f(P, si[16], i, dp1);

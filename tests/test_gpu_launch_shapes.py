@@ -72,6 +72,7 @@ def test_short_lists_are_the_head_of_a_long_one(cat, prec):
 
 @pytest.mark.parametrize('prec', [64, 32])
 def test_tables_in_lds_or_not(cat, prec):
+    import torch
     from marxs_amd.batch import _tables_with_budget
     n = 30011
     src = _source(n)
@@ -86,7 +87,14 @@ def test_tables_in_lds_or_not(cat, prec):
             cat.dev_tables = _tables_with_budget(cat, budget)
             sizes.add(int(cat.dev_tables.struct.lds_bytes64 if prec == 64 else cat.dev_tables.struct.lds_bytes32))
             got, st2 = _launch(cat, src, u, prec)
-            _same(ref, got)
+            _same(ref, got, skip=('blaze',) if prec == 32 else ())
+            # FP32: the cosine of the blaze angle is rounded in steps of 2^-24
+            # below 1, and code that reads its tables from elsewhere may fuse
+            # the products in it differently: 4 such steps, times 1 / sine
+            x, y = ref['blaze'].view(torch.float64), got['blaze'].view(torch.float64)
+            ok = ~torch.isnan(x)
+            assert torch.equal(ok, ~torch.isnan(y))
+            assert float(((x - y).abs() * torch.sin(x))[ok].max()) <= (4 * 2. ** -24 if prec == 32 else 0.)
             assert (st == st2).all()
     finally:
         cat.dev_tables = was
