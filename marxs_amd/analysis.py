@@ -21,6 +21,8 @@ loop of ``resolvingpower_per_order``, the detector positions tried by
 ``find_best_detector_position``) keep the photons in HBM between traces and
 run the FP64 kernels.
 """
+import functools
+
 import numpy as np
 import torch
 
@@ -77,6 +79,13 @@ def _orders_i32(col):
     return col.to(torch.int32).contiguous()
 
 
+@functools.lru_cache(maxsize=32)
+def _device_orders(orders, device):
+    """Order numbers (a tuple) on the device, read only.  Copying them there
+    on every call takes 20 us, as much as a small list's sums."""
+    return torch.as_tensor(np.array(orders, dtype=np.int32), device=device)
+
+
 def order_stats(order, prob, orders, value=None, res_filter=False, sigma=3., maxiters=5,
                 select=None, stream=None):
     """Per-order reductions on the GPU (``mx_order_stats``).
@@ -94,7 +103,8 @@ def order_stats(order, prob, orders, value=None, res_filter=False, sigma=3., max
         empty = np.zeros(0)
         return {'prob_sum': empty, 'count': np.zeros(0, np.int64), 'mean': empty,
                 'median': empty, 'std': empty, 'n_kept': np.zeros(0, np.int64)}
-    if len(np.unique(orders)) != len(orders):
+    numbers = tuple(orders.tolist())
+    if len(set(numbers)) != len(numbers):
         raise ValueError('order numbers must be distinct')
     if len(orders) > _lib.MX_MAX_ORDERS:
         # the kernels take at most MX_MAX_ORDERS orders per call
@@ -118,7 +128,7 @@ def order_stats(order, prob, orders, value=None, res_filter=False, sigma=3., max
             res.update({'mean': np.full(no, np.nan), 'median': np.full(no, np.nan),
                         'std': np.full(no, np.nan), 'n_kept': np.zeros(no, np.int64)})
         return res
-    ords = torch.as_tensor(orders.astype(np.int32), device=dev)
+    ords = _device_orders(tuple(orders.astype(np.int32).tolist()), dev)
     wsb = int(_lib.lib.mx_order_stats_workspace(n, no, int(v is not None)))
     if wsb < 0:
         raise ValueError('order statistics: invalid sizes')
@@ -127,10 +137,6 @@ def order_stats(order, prob, orders, value=None, res_filter=False, sigma=3., max
     keys = ('prob_sum', 'count', 'mean', 'median', 'std', 'n_kept')
     ints = ('count', 'n_kept')
     buf = torch.empty(len(keys) * no, dtype=torch.float64, device=dev)
-    out = {}
-    for j, k in enumerate(keys):
-        part = buf[j * no:(j + 1) * no]
-        out[k] = part.view(torch.int64) if k in ints else part
     a = _lib.MxOrderStats()
     a.n = n
     a.order = o.data_ptr()
@@ -143,8 +149,9 @@ def order_stats(order, prob, orders, value=None, res_filter=False, sigma=3., max
     a.maxiters = int(maxiters)
     a.workspace = ws.data_ptr()
     a.workspace_bytes = wsb
-    for k in ('prob_sum', 'count', 'mean', 'median', 'std', 'n_kept'):
-        setattr(a, k, out[k].data_ptr())
+    base = buf.data_ptr()
+    for j, k in enumerate(keys):
+        setattr(a, k, base + 8 * j * no)
     if stream is None:
         stream = torch.cuda.current_stream(dev).cuda_stream
     _lib.check(_lib.lib.mx_order_stats(a, stream))
@@ -213,6 +220,17 @@ def resolvingpower_from_photonlist(photons, orders, col='proj_x', zeropos=None, 
     return _resolving_power(order, value, orders, zeropos, False, prob)
 
 
+def _average_R_Aeff_1d(r, aeff):
+    """``average_R_Aeff`` of 1-d float arrays with the same sums in the same
+    order (a masked product counts as 0 there), without masked arrays, which
+    take 45 us for 15 orders; all masked or a zero weight sum goes there."""
+    fin = np.isfinite(r)
+    scl = np.where(fin, aeff, 0.).sum()
+    if not fin.any() or not scl != 0. or not np.isfinite(scl):
+        return average_R_Aeff(r, aeff)
+    return np.multiply(np.where(fin, r, 0.), np.where(fin, aeff, 0.)).sum() / scl, aeff.sum()
+
+
 def average_R_Aeff(r, aeff, axis=None):
     """Summed effective area and area-weighted average of the finite
     resolving powers (gratings.py:187-212)."""
@@ -265,7 +283,7 @@ class CaptureResAeff:
             except AnalysisError:
                 res = np.nan * np.ones(len(self.orders))
         disporders = self.orders != 0
-        avggratres, aeffgrat = average_R_Aeff(res[disporders], aeff[disporders])
+        avggratres, aeffgrat = _average_R_Aeff_1d(res[disporders], aeff[disporders])
         aeff = np.asarray(aeff)
         aeff0 = np.sum(aeff[~disporders])
         return {'Aeff0': aeff0, 'Aeffgrat': aeffgrat, 'Aeff': aeff, 'Rgrat': avggratres, 'R': res}
@@ -278,15 +296,16 @@ class CaptureResAeff:
         want = list(dict.fromkeys([int(x) for x in orders] + ([0] if self.zeropos is None else [])))
         r = order_stats(order, prob, want, value=value, res_filter=True)
         idx = {o: i for i, o in enumerate(want)}
-        aeff = np.array([r['prob_sum'][idx[int(o)]] for o in orders]) / n_photons * self.A_geom
+        at = np.array([idx[int(o)] for o in orders], dtype=int)
+        aeff = r['prob_sum'][at] / n_photons * self.A_geom
         zeropos = self.zeropos
         if zeropos is None:
             if r['count'][idx[0]] < 20:
                 return np.nan * np.ones(len(orders)), aeff
             zeropos = r['mean'][idx[0]]
-        ok = np.array([r['count'][idx[int(o)]] > 20 for o in orders])
-        pos = np.where(ok, [r['mean'][idx[int(o)]] for o in orders], np.nan)
-        std = np.where(ok, [r['std'][idx[int(o)]] for o in orders], np.nan)
+        ok = r['count'][at] > 20
+        pos = np.where(ok, r['mean'][at], np.nan)
+        std = np.where(ok, r['std'][at], np.nan)
         with np.errstate(invalid='ignore', divide='ignore'):
             res = np.abs(pos - zeropos) / (std * RES_FWHM)
         return res, aeff

@@ -45,6 +45,15 @@ def _dev(device):
     return torch.device(device)
 
 
+def _row_pointers(t):
+    """Addresses of the rows of a (3, N) column (a tensor each would take
+    2 us)."""
+    if type(t) is torch.Tensor and t.dim() == 2 and t.shape[0] >= 3:
+        p, step = t.data_ptr(), t.stride(0) * t.element_size()
+        return p, p + step, p + 2 * step
+    return t[0].data_ptr(), t[1].data_ptr(), t[2].data_ptr()
+
+
 class DeviceTables:
     """Compiled tables resident on one GPU."""
 
@@ -138,8 +147,10 @@ class DevicePhotons:
     def clone(self):
         c = DevicePhotons.__new__(DevicePhotons)
         c.device, c.n, c.has_pos = self.device, self.n, self.has_pos
-        for a in ('dir', 'pol', 'energy', 'prob', 'pos'):
+        for a in ('dir', 'pol', 'energy', 'prob'):
             setattr(c, a, getattr(self, a).clone())
+        # positions that no trace has set yet are memory as it was allocated
+        c.pos = self.pos.clone() if self.has_pos else torch.empty_like(self.pos)
         c.fcols = {k: v.clone() for k, v in self.fcols.items()}
         c.icols = {k: v.clone() for k, v in self.icols.items()}
         return c
@@ -322,17 +333,16 @@ class CompiledInstrument:
         if t.n_uniform_slots > 0:
             P.uniform_stride = uniforms.stride(0)
             P.uniforms = uniforms.data_ptr()
-        for k in range(3):
-            P.pos[k] = dp.pos[k].data_ptr()
-            P.dir[k] = dp.dir[k].data_ptr()
-            P.pol[k] = dp.pol[k].data_ptr()
+        P.pos[:] = _row_pointers(dp.pos)
+        P.dir[:] = _row_pointers(dp.dir)
+        P.pol[:] = _row_pointers(dp.pol)
         P.energy = (src if src is not None else dp).energy.data_ptr()
         P.prob = dp.prob.data_ptr()
         if src is not None:
-            for k in range(3):
-                P.pos_in[k] = src.pos[k].data_ptr() if src.has_pos else None
-                P.dir_in[k] = src.dir[k].data_ptr()
-                P.pol_in[k] = src.pol[k].data_ptr()
+            if src.has_pos:
+                P.pos_in[:] = _row_pointers(src.pos)
+            P.dir_in[:] = _row_pointers(src.dir)
+            P.pol_in[:] = _row_pointers(src.pol)
             P.prob_in = src.prob.data_ptr()
         for k, name in enumerate(t.fcols):
             P.fcol[k] = dp.fcols[name].data_ptr()
