@@ -134,27 +134,44 @@ __device__ __forceinline__ double wave_sum(double v) {
     return v;
 }
 
-// Photon i through the facet of geometry record G onto detector record C:
+// A photon's columns.
+struct PhotonIn {
+    double pos[3], dir[3], energy;
+    int order;
+};
+__device__ __forceinline__ PhotonIn photon_in(const MxAdjointArgs &A, int64_t i) {
+    PhotonIn p;
+    for (int k = 0; k < 3; ++k) {
+        p.pos[k] = A.pos[k][i];
+        p.dir[k] = A.dir[k][i];
+    }
+    p.energy = A.energy[i];
+    p.order = A.order[i];
+    return p;
+}
+
+// A photon through the facet of geometry record G onto detector record C:
 // returns its coordinate y, and with bw the seed's derivatives g (seed
 // yb0 + yb1 (y - c_f . u + yoff)).
 template <int PREC>
-__device__ __forceinline__ double photon_replay(const MxAdjointArgs &A, const double *G, const double *C, int64_t i,
-                                                bool bw, double yb0, double yb1, double yoff, double *g) {
+__device__ __forceinline__ double photon_replay(const MxAdjointArgs &A, const double *G, const double *C,
+                                                const PhotonIn &in, bool bw, double yb0, double yb1, double yoff,
+                                                double *g) {
     const double cu = A.coord == 0 ? G[0] : (A.coord == 1 ? G[1] : G[2]);
     const double ang = G[13];
     double sgd, cgd;
     sincos(-ang, &sgd, &cgd);
     const int sign_mode = (int)G[14];
     const double trans = G[15] != 0.0 ? 1.0 : -1.0;
-    const double wave = AJ_E2W / A.energy[i];
-    const int m = A.order[i];
+    const double wave = AJ_E2W / in.energy;
+    const int m = in.order;
     double y;
     // relative positions in FP64 (exact origin subtraction)
-    const double r0x = A.pos[0][i] - G[0], r0y = A.pos[1][i] - G[1], r0z = A.pos[2][i] - G[2];
+    const double r0x = in.pos[0] - G[0], r0y = in.pos[1] - G[1], r0z = in.pos[2] - G[2];
     const double rcx = C[0] - G[0], rcy = C[1] - G[1], rcz = C[2] - G[2];
     if (PREC == 64) {
         double gg[AJ_NG];
-        y = photon_adjoint<double>(v3(r0x, r0y, r0z), v3(A.dir[0][i], A.dir[1][i], A.dir[2][i]),
+        y = photon_adjoint<double>(v3(r0x, r0y, r0z), v3(in.dir[0], in.dir[1], in.dir[2]),
                                    v3(rcx, rcy, rcz), ld<double>(C + 3),
                                    v3((double)(A.coord == 0), (double)(A.coord == 1), (double)(A.coord == 2)),
                                    ld<double>(G + 3), ld<double>(G + 6), ld<double>(G + 9), G[12],
@@ -163,7 +180,7 @@ __device__ __forceinline__ double photon_replay(const MxAdjointArgs &A, const do
     } else {
         float gf[AJ_NG];
         y = (double)photon_adjoint<float>(v3((float)r0x, (float)r0y, (float)r0z),
-                                          v3((float)A.dir[0][i], (float)A.dir[1][i], (float)A.dir[2][i]),
+                                          v3((float)in.dir[0], (float)in.dir[1], (float)in.dir[2]),
                                           v3((float)rcx, (float)rcy, (float)rcz), ld<float>(C + 3),
                                           v3((float)(A.coord == 0), (float)(A.coord == 1), (float)(A.coord == 2)),
                                           ld<float>(G + 3), ld<float>(G + 6), ld<float>(G + 9), (float)G[12],
@@ -221,7 +238,7 @@ __device__ __forceinline__ void adjoint_photons(const MxAdjointArgs &A, const do
             }
         }
         double g[AJ_NG];
-        const double y = photon_replay<PREC>(A, G, C, i, bw, yb0, yb1, yoff, g);
+        const double y = photon_replay<PREC>(A, G, C, photon_in(A, i), bw, yb0, yb1, yoff, g);
         if (A.y_out) A.y_out[i] = y;
         const double ys = y - A.y_shift;
         m0 += wgt;
@@ -369,21 +386,41 @@ __device__ __forceinline__ void pose_axes(const MxPoseArgs &A, int f, double v[3
     }
 }
 
+// What both directions need of facet f: the axes with 1 / length, (dRe_a
+// Rpost)[:, k] for the three angles a, and zoom_k.
+struct PoseParts {
+    double v[3][3], inv[3], col[3][3][3], z[3];
+};
+__device__ __forceinline__ void pose_parts(const MxPoseArgs &A, int f, PoseParts &p) {
+    double dRe[3][9];
+    pose_axes(A, f, p.v, p.inv, dRe);
+    const double *Rp = A.rpost + (size_t)f * 9;
+    for (int k = 0; k < 3; ++k) {
+        p.z[k] = A.zoom[(size_t)f * 3 + k];
+        for (int a = 0; a < 3; ++a)
+            for (int i = 0; i < 3; ++i)
+                p.col[k][a][i] = dRe[a][3 * i] * Rp[k] + dRe[a][3 * i + 1] * Rp[3 + k] + dRe[a][3 * i + 2] * Rp[6 + k];
+    }
+}
+
 // Geometry record of facet f (centre, e_x, e_y, e_z, period, groove angle,
 // sign mode, transmission).
-__device__ __forceinline__ void pose_forward(const MxPoseArgs &A, int f, double *g) {
-    double v[3][3], inv[3], dRe[3][9];
-    pose_axes(A, f, v, inv, dRe);
+__device__ __forceinline__ void pose_geometry(const MxPoseArgs &A, int f, const PoseParts &p, double *g) {
     const double *th = A.theta + (size_t)f * 6;
     const double *G = A.gu;
     const double t[3] = {th[0] + A.t0[3 * f], th[1] + A.t0[3 * f + 1], th[2] + A.t0[3 * f + 2]};
     for (int i = 0; i < 3; ++i) g[i] = G[4 * i] * t[0] + G[4 * i + 1] * t[1] + G[4 * i + 2] * t[2] + G[4 * i + 3];
     for (int k = 0; k < 3; ++k)
-        for (int i = 0; i < 3; ++i) g[3 + 3 * k + i] = v[k][i] * inv[k];
+        for (int i = 0; i < 3; ++i) g[3 + 3 * k + i] = p.v[k][i] * p.inv[k];
     g[12] = A.period[f];
     g[13] = A.extra[3 * f];
     g[14] = A.extra[3 * f + 1];
     g[15] = A.extra[3 * f + 2];
+}
+__device__ __forceinline__ void pose_forward(const MxPoseArgs &A, int f, double *g) {
+    PoseParts p;
+    pose_parts(A, f, p);
+    pose_geometry(A, f, p, g);
 }
 
 // dL/dg of facet f from the single-pass sums S (A then B) and the moments.
@@ -402,34 +439,30 @@ __device__ __forceinline__ double loss_from_moments(const double mom[3], double 
 }
 
 // The 13 gradients gg of facet f mapped to d/d theta (6) and d/d period.
-__device__ __forceinline__ void pose_backward(const MxPoseArgs &A, int f, const double *gg, double *out) {
-    double v[3][3], inv[3], dRe[3][9];
-    pose_axes(A, f, v, inv, dRe);
+__device__ __forceinline__ void pose_chain(const MxPoseArgs &A, int f, const PoseParts &p, const double *gg, double *out) {
     const double *G = A.gu;
-    const double *Rp = A.rpost + (size_t)f * 9;
-    const double *z = A.zoom + (size_t)f * 3;
     for (int j = 0; j < 3; ++j) out[j] = G[j] * gg[0] + G[4 + j] * gg[1] + G[8 + j] * gg[2];   // G^T g_c
     double ga[3] = {0, 0, 0};
     for (int k = 0; k < 3; ++k) {
-        const double e[3] = {v[k][0] * inv[k], v[k][1] * inv[k], v[k][2] * inv[k]};
+        const double e[3] = {p.v[k][0] * p.inv[k], p.v[k][1] * p.inv[k], p.v[k][2] * p.inv[k]};
         const double *ge = gg + 3 + 3 * k;
         const double eg = e[0] * ge[0] + e[1] * ge[1] + e[2] * ge[2];
         double gv[3];
-        for (int i = 0; i < 3; ++i) gv[i] = (ge[i] - e[i] * eg) * inv[k];
+        for (int i = 0; i < 3; ++i) gv[i] = (ge[i] - e[i] * eg) * p.inv[k];
         double h[3];   // G^T gv zoom_k
-        for (int j = 0; j < 3; ++j) h[j] = (G[j] * gv[0] + G[4 + j] * gv[1] + G[8 + j] * gv[2]) * z[k];
-        for (int a = 0; a < 3; ++a) {
-            // (dRe_a Rpost)[:, k]
-            double col[3];
-            for (int i = 0; i < 3; ++i)
-                col[i] = dRe[a][3 * i] * Rp[k] + dRe[a][3 * i + 1] * Rp[3 + k] + dRe[a][3 * i + 2] * Rp[6 + k];
-            ga[a] += h[0] * col[0] + h[1] * col[1] + h[2] * col[2];
-        }
+        for (int j = 0; j < 3; ++j) h[j] = (G[j] * gv[0] + G[4 + j] * gv[1] + G[8 + j] * gv[2]) * p.z[k];
+        for (int a = 0; a < 3; ++a)
+            ga[a] += h[0] * p.col[k][a][0] + h[1] * p.col[k][a][1] + h[2] * p.col[k][a][2];
     }
     out[3] = ga[0];
     out[4] = ga[1];
     out[5] = ga[2];
     out[6] = gg[12];
+}
+__device__ __forceinline__ void pose_backward(const MxPoseArgs &A, int f, const double *gg, double *out) {
+    PoseParts p;
+    pose_parts(A, f, p);
+    pose_chain(A, f, p, gg, out);
 }
 
 __global__ void mx_facet_pose_kernel(MxPoseArgs A) {
@@ -491,8 +524,8 @@ extern "C" int mx_facet_pose(const MxPoseArgs *a, void *stream) {
 // adds its tasks and applies the chain rule.  The call without that order
 // (fill, frames, replay, chain rule: 4 kernels) adds every photon's 26 values
 // with atomics, in LDS up to 315 facets and in global memory beyond.  Kernel
-// times, us: 200 facets, 2.1e4 photons FP32 31 -> 18; 600 facets, 9.1e4
-// photons FP64 178 -> 27.  Bound by latency: the chain of one photon's replay
+// times, us: 200 facets, 2.1e4 photons FP32 31 -> 14; 600 facets, 9.1e4
+// photons FP64 178 -> 18.  Bound by latency: the chain of one photon's replay
 // (two planes, the grating equation and its adjoint) and of the facet's frame.
 #define AJ_TASK 128             // work-items per task
 #define AJ_SUMS (2 * AJ_NG + 3) // A, B, moments
@@ -513,33 +546,53 @@ __device__ __forceinline__ double wave_total(double v) {
     return v;
 }
 
+// Moments of the tasks, then their sums A and B, in S.part.
+__device__ __forceinline__ double *task_moments(const MxAdjointStep &S, int k) { return S.part + (size_t)k * S.n_tasks; }
+__device__ __forceinline__ double *task_sums(const MxAdjointStep &S, int64_t j) {
+    return S.part + 3 * (size_t)S.n_tasks + (size_t)j * (2 * AJ_NG);
+}
+static_assert(AJ_SUMS <= MX_AJ_PART, "a task's sums and moments");
+
+// The first photon of each work-item is loaded before the facet's frame is
+// formed, so that the loads are under way during that chain (8.7 -> 8.3 us for
+// 200 facets; 11.4 either way for 600).
 template <int PREC>
 __global__ __launch_bounds__(AJ_TASK) void mx_adjoint_task_kernel(MxAdjointStep S) {
     __shared__ double red[AJ_TASK / 64][AJ_SUMS];
     const int32_t *task = S.task + 3 * (size_t)blockIdx.x;
     const int f = task[0], b = task[1], e = task[2];
     if (b >= e) return;
+    const MxAdjointArgs &A = S.photons;
+    int i = b + (int)threadIdx.x;
+    // a work-item without a photon loads the task's last one
+    const int i0 = i < e ? i : e - 1;
+    PhotonIn in = photon_in(A, i0);
+    int c = A.ccd[i0];
+    double wgt = A.weight ? A.weight[i0] : 1.0;
     double G[MX_AJ_GEOM];
     pose_forward(S.pose, f, G);
-    const MxAdjointArgs &A = S.photons;
     double s[AJ_SUMS];
 #pragma unroll
     for (int k = 0; k < AJ_SUMS; ++k) s[k] = 0.0;
-    for (int i = b + (int)threadIdx.x; i < e; i += AJ_TASK) {
-        const int c = A.ccd[i];
-        const double wgt = A.weight ? A.weight[i] : 1.0;
-        if (c < 0 || c >= A.n_ccd || !(wgt != 0.0)) continue;
-        double g[AJ_NG];
-        const double y = photon_replay<PREC>(A, G, A.ccd_t + (size_t)c * MX_ET, i, true, wgt, 0.0, 0.0, g);
-        const double ys = y - A.y_shift;
+    while (i < e) {
+        if (c >= 0 && c < A.n_ccd && wgt != 0.0) {
+            double g[AJ_NG];
+            const double y = photon_replay<PREC>(A, G, A.ccd_t + (size_t)c * MX_ET, in, true, wgt, 0.0, 0.0, g);
+            const double ys = y - A.y_shift;
 #pragma unroll
-        for (int k = 0; k < AJ_NG; ++k) {
-            s[k] += g[k];
-            s[AJ_NG + k] += ys * g[k];
+            for (int k = 0; k < AJ_NG; ++k) {
+                s[k] += g[k];
+                s[AJ_NG + k] += ys * g[k];
+            }
+            s[2 * AJ_NG] += wgt;
+            s[2 * AJ_NG + 1] += wgt * ys;
+            s[2 * AJ_NG + 2] += wgt * ys * ys;
         }
-        s[2 * AJ_NG] += wgt;
-        s[2 * AJ_NG + 1] += wgt * ys;
-        s[2 * AJ_NG + 2] += wgt * ys * ys;
+        i += AJ_TASK;
+        if (i >= e) break;
+        in = photon_in(A, i);
+        c = A.ccd[i];
+        wgt = A.weight ? A.weight[i] : 1.0;
     }
 #pragma unroll
     for (int k = 0; k < AJ_SUMS; ++k) {
@@ -548,47 +601,60 @@ __global__ __launch_bounds__(AJ_TASK) void mx_adjoint_task_kernel(MxAdjointStep 
     }
     __syncthreads();
     if (threadIdx.x < AJ_SUMS) {
+        const int k = (int)threadIdx.x;
         double x = 0.0;
-        for (int w = 0; w < AJ_TASK / 64; ++w) x += red[w][threadIdx.x];
-        S.part[(size_t)blockIdx.x * MX_AJ_PART + threadIdx.x] = x;
+        for (int w = 0; w < AJ_TASK / 64; ++w) x += red[w][k];
+        if (k < 2 * AJ_NG) task_sums(S, blockIdx.x)[k] = x;
+        else task_moments(S, k - 2 * AJ_NG)[blockIdx.x] = x;
     }
 }
 
-// One wave per facet.  Every wave adds up the moments of all tasks for itself.
-__global__ __launch_bounds__(64) void mx_adjoint_finish_kernel(MxAdjointStep S) {
+// Two waves per facet: the first adds the sums of the facet's tasks and, for
+// itself, the moments of all tasks, while the second forms the facet's frame
+// and its derivatives.  Bound by latency: one wave doing both, with the moments
+// 256 bytes apart, took 9.9 us for 200 facets and 16.5 us for 600, this 6.0 and
+// 7.0.
+__global__ __launch_bounds__(128) void mx_adjoint_finish_kernel(MxAdjointStep S) {
     __shared__ double sums[2 * AJ_NG];
-    const int f = blockIdx.x, lane = threadIdx.x;
+    __shared__ PoseParts parts;
+    const int f = blockIdx.x, lane = threadIdx.x & 63;
     const MxPoseArgs &P = S.pose;
-    const int n_tasks = S.task_first[P.n_facet];
     double m[3] = {0.0, 0.0, 0.0};
+    if (threadIdx.x < 64) {
+        const int n_tasks = S.task_first[P.n_facet], j0 = S.task_first[f], j1 = S.task_first[f + 1];
+        double x = 0.0;
+        if (lane < 2 * AJ_NG)
 #pragma unroll 4
-    for (int j = lane; j < n_tasks; j += 64) {
-        const double *q = S.part + (size_t)j * MX_AJ_PART + 2 * AJ_NG;
-        m[0] += q[0];
-        m[1] += q[1];
-        m[2] += q[2];
-    }
-    double x = 0.0;
-    if (lane < 2 * AJ_NG)
-#pragma unroll 4
-        for (int j = S.task_first[f]; j < S.task_first[f + 1]; ++j) x += S.part[(size_t)j * MX_AJ_PART + lane];
-    if (lane < 2 * AJ_NG) sums[lane] = x;
+            for (int j = j0; j < j1; ++j) x += task_sums(S, j)[lane];
+#pragma unroll 8
+        for (int j = lane; j < n_tasks; j += 64)
+            for (int k = 0; k < 3; ++k) m[k] += task_moments(S, k)[j];
+        if (lane < 2 * AJ_NG) sums[lane] = x;
 #pragma unroll
-    for (int k = 0; k < 3; ++k) m[k] = __shfl(wave_total(m[k]), 63);
+        for (int k = 0; k < 3; ++k) m[k] = __shfl(wave_total(m[k]), 63);
+    } else {
+        PoseParts p;
+        pose_parts(P, f, p);
+        double geom[MX_AJ_GEOM];
+        pose_geometry(P, f, p, geom);
+        if (lane == 0) {
+            parts = p;
+            for (int k = 0; k < MX_AJ_GEOM; ++k) P.geom[(size_t)f * MX_AJ_GEOM + k] = geom[k];
+            if (S.theta_out)
+                for (int k = 0; k < 6; ++k) S.theta_out[(size_t)f * 6 + k] = P.theta[(size_t)f * 6 + k];
+            if (S.period_out) S.period_out[f] = P.period[f];
+        }
+    }
     __syncthreads();
-    double gg[MX_AJ_NGRAD], out[7], geom[MX_AJ_GEOM];
+    if (threadIdx.x >= 64) return;
+    double gg[MX_AJ_NGRAD], out[7];
     sums_to_grad(sums, m, gg);
-    pose_backward(P, f, gg, out);
-    pose_forward(P, f, geom);
+    pose_chain(P, f, parts, gg, out);
     if (lane == 0) {
-        for (int k = 0; k < MX_AJ_GEOM; ++k) P.geom[(size_t)f * MX_AJ_GEOM + k] = geom[k];
         for (int k = 0; k < 7; ++k) P.grad7[(size_t)f * 7 + k] = out[k];
         if (S.grad_theta)
             for (int k = 0; k < 6; ++k) S.grad_theta[(size_t)f * 6 + k] = out[k];
         if (S.grad_period) S.grad_period[f] = out[6];
-        if (S.theta_out)
-            for (int k = 0; k < 6; ++k) S.theta_out[(size_t)f * 6 + k] = P.theta[(size_t)f * 6 + k];
-        if (S.period_out) S.period_out[f] = P.period[f];
         if (f == 0) {
             const double loss = loss_from_moments(m, P.y_shift);
             P.loss[0] = loss;
@@ -695,7 +761,7 @@ extern "C" int mx_adjoint_step(const MxAdjointStep *s, void *stream) {
         hipLaunchKernelGGL(mx_adjoint_task_kernel<64>, dim3((unsigned)s->n_tasks), dim3(AJ_TASK), 0, st, *s);
     else if (s->n_tasks > 0)
         hipLaunchKernelGGL(mx_adjoint_task_kernel<32>, dim3((unsigned)s->n_tasks), dim3(AJ_TASK), 0, st, *s);
-    hipLaunchKernelGGL(mx_adjoint_finish_kernel, dim3((unsigned)p.n_facet), dim3(64), 0, st, *s);
+    hipLaunchKernelGGL(mx_adjoint_finish_kernel, dim3((unsigned)p.n_facet), dim3(128), 0, st, *s);
     hipError_t err = hipGetLastError();
     if (err != hipSuccess) {
         char buf[256];
