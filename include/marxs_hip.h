@@ -445,6 +445,15 @@ int mx_order_stats_static(const MxOrderStats *args, void *stream);
  * utility for the callers of this library. */
 int mx_fill_i32(int32_t *dst, int64_t n, int32_t v, void *stream);
 
+/* Rows [n][4] = x, y, z, w (16-byte aligned) from three columns, and three
+ * columns from the first values of rows [n][width], width >= 3 (homogeneous
+ * coordinates of a photon table, marxs/optics/base.py:149-211).  Asynchronous
+ * on the stream. */
+int mx_pack_rows(const double *x, const double *y, const double *z, double w, double *rows, int64_t n,
+                 void *stream);
+int mx_unpack_rows(const double *rows, int64_t width, double *x, double *y, double *z, int64_t n,
+                   void *stream);
+
 /* ABI version (MX_ABI_VERSION) and the calling thread's last error text. */
 int mx_abi_version(void);
 const char *mx_last_error(void);

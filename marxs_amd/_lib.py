@@ -114,6 +114,10 @@ def _load():
                                    ctypes.c_void_p, ctypes.c_void_p]
     lib.mx_fill_i32.restype = ctypes.c_int
     lib.mx_fill_i32.argtypes = [P, ctypes.c_int64, ctypes.c_int32, P]
+    lib.mx_pack_rows.restype = ctypes.c_int
+    lib.mx_pack_rows.argtypes = [P, P, P, ctypes.c_double, P, ctypes.c_int64, P]
+    lib.mx_unpack_rows.restype = ctypes.c_int
+    lib.mx_unpack_rows.argtypes = [P, ctypes.c_int64, P, P, P, ctypes.c_int64, P]
     lib.mx_trace_batched.restype = ctypes.c_int
     lib.mx_trace_batched.argtypes = [ctypes.POINTER(MxBatch), ctypes.c_int32, ctypes.c_int32, P]
     lib.mx_adjoint.restype = ctypes.c_int

@@ -3140,3 +3140,53 @@ extern "C" int mx_fill_i32(int32_t *dst, int64_t n, int32_t v, void *stream) {
     hipLaunchKernelGGL(mx_fill_i32_kernel, dim3((unsigned)nblk), dim3(block), 0, (hipStream_t)stream, dst, n, v);
     return hipGetLastError() == hipSuccess ? 0 : 2;
 }
+
+// Rows of a photon table (homogeneous coordinates, [n][width]) from and to the
+// trace's columns.  On the host each turned 1e5 rows in 0.2 to 0.4 ms, most of
+// a table call beside its copies; here it is one pass over memory that takes a
+// few us, and the copies are of rows: table call of 1e5 photons 4.9 -> 2.8 ms.
+__global__ __launch_bounds__(256) void mx_pack_rows_kernel(const double *x, const double *y, const double *z, double w,
+                                                            double2 *rows, int64_t n) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    rows[2 * i] = make_double2(x[i], y[i]);
+    rows[2 * i + 1] = make_double2(z[i], w);
+}
+
+__global__ __launch_bounds__(256) void mx_unpack_rows_kernel(const double *rows, int64_t width, double *x, double *y,
+                                                              double *z, int64_t n) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    const double *r = rows + i * width;
+    x[i] = r[0];
+    y[i] = r[1];
+    z[i] = r[2];
+}
+
+static int rows_launched(const char *what) {
+    if (hipGetLastError() == hipSuccess) return 0;
+    set_error(what);
+    return 2;
+}
+
+extern "C" int mx_pack_rows(const double *x, const double *y, const double *z, double w, double *rows, int64_t n,
+                            void *stream) {
+    if (n < 0 || n > ((int64_t)1 << 38)) { set_error("rows: number out of range"); return 1; }
+    if (n == 0) return 0;
+    if (!x || !y || !z || !rows) { set_error("rows: a pointer is NULL"); return 1; }
+    if ((uintptr_t)rows & 15) { set_error("rows: not 16-byte aligned"); return 1; }
+    hipLaunchKernelGGL(mx_pack_rows_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, (hipStream_t)stream, x, y, z,
+                       w, (double2 *)rows, n);
+    return rows_launched("rows: pack launch failed");
+}
+
+extern "C" int mx_unpack_rows(const double *rows, int64_t width, double *x, double *y, double *z, int64_t n,
+                              void *stream) {
+    if (n < 0 || n > ((int64_t)1 << 38)) { set_error("rows: number out of range"); return 1; }
+    if (width < 3) { set_error("rows: fewer than 3 values"); return 1; }
+    if (n == 0) return 0;
+    if (!x || !y || !z || !rows) { set_error("rows: a pointer is NULL"); return 1; }
+    hipLaunchKernelGGL(mx_unpack_rows_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, (hipStream_t)stream, rows,
+                       width, x, y, z, n);
+    return rows_launched("rows: unpack launch failed");
+}

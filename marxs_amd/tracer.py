@@ -104,6 +104,32 @@ class DeviceTables:
         return self._make_struct(si)
 
 
+def _columns_of(rows, device):
+    """(3, N) device columns from host rows (N, >= 3), turned on the device."""
+    n = rows.shape[0]
+    out = torch.empty((3, n), dtype=torch.float64, device=device)
+    with torch.cuda.device(device):
+        r = torch.as_tensor(rows, device=device)
+        _lib.check(_lib.lib.mx_unpack_rows(r.data_ptr(), rows.shape[1], *_row_pointers(out), n,
+                                           torch.cuda.current_stream(device).cuda_stream))
+    return out
+
+
+def _rows_of(t, w):
+    """Host rows (N, 4) of a (3, N) float64 device column, the last value w."""
+    if not (t.is_cuda and t.dtype == torch.float64 and t.dim() == 2 and t.shape[0] == 3 and t.stride(1) == 1):
+        out = np.empty((t.shape[1], 4))
+        out[:, :3] = t.cpu().numpy().T
+        out[:, 3] = w
+        return out
+    n = t.shape[1]
+    rows = torch.empty((n, 4), dtype=torch.float64, device=t.device)
+    with torch.cuda.device(t.device):
+        _lib.check(_lib.lib.mx_pack_rows(*_row_pointers(t), w, rows.data_ptr(), n,
+                                         torch.cuda.current_stream(t.device).cuda_stream))
+        return rows.cpu().numpy()
+
+
 class DevicePhotons:
     """Structure-of-arrays photon columns on the GPU (float64).
 
@@ -136,12 +162,18 @@ class DevicePhotons:
 
     @classmethod
     def from_table(cls, photons, device=None):
-        def col(name, k=3):
-            return np.ascontiguousarray(np.asarray(photons[name], dtype=float)[:, :k].T)
+        dev = _dev(device)
+
+        def col(name):
+            rows = np.asarray(photons[name], dtype=float)
+            if dev.type == 'cuda' and rows.ndim == 2 and rows.shape[1] >= 3:
+                return _columns_of(np.require(rows, requirements=['C', 'W']), dev)
+            return np.ascontiguousarray(rows[:, :3].T)
         pos = col('pos') if 'pos' in photons.colnames else None
         self = cls(col('dir'), col('polarization'),
                    np.asarray(photons['energy'], dtype=float),
-                   np.asarray(photons['probability'], dtype=float), pos=pos, device=device)
+                   np.asarray(photons['probability'], dtype=float), pos=pos, device=device,
+                   copy=dev.type != 'cuda')     # there every column is a new tensor
         return self
 
     def clone(self):
@@ -419,16 +451,9 @@ def write_back(dp, photons, tables, existing=()):
     when an element has interacting photons, a new output column in which no
     photon was written (all NaN / -1) is not added to the table.
     """
-    n = dp.n
-
-    def h(t, w):
-        out = np.empty((n, 4))
-        out[:, :3] = t.cpu().numpy().T
-        out[:, 3] = w
-        return out
-    photons['pos'] = h(dp.pos, 1.)
-    photons['dir'] = h(dp.dir, 0.)
-    photons['polarization'] = h(dp.pol, 0.)
+    photons['pos'] = _rows_of(dp.pos, 1.)
+    photons['dir'] = _rows_of(dp.dir, 0.)
+    photons['polarization'] = _rows_of(dp.pol, 0.)
     photons['probability'] = dp.prob.cpu().numpy()
     for name in tables.fcols:
         v = dp.fcols[name].cpu().numpy()
