@@ -692,7 +692,8 @@ def compile_tree(tree, n_draws=2, grid=True, grid_min_elements=4, **grid_kw):
 # 1024 (FP32) or 768 (FP64) work-items per CU; the kernel's own LDS is a few
 # hundred bytes).
 LDS_BUDGET32 = 158 * 1024
-LDS_BUDGET64 = 150 * 1024
+# (FP64: the split trace's second kernel holds another 2 KiB)
+LDS_BUDGET64 = 157 * 1024
 # The loose tier's cell lists (read only by rays more oblique than the tight
 # tier allows) are staged last and only while the image leaves this much of
 # the 160 KiB free for the regrouping kernels' ray exchange buffer (about 600
@@ -743,7 +744,7 @@ def _build_lds(tables, budget32=None, budget64=None):
 
     Selector tables first (energies, cumulative probabilities and totals as
     float64, then int32 orders), then per array stage of two or more
-    elements, while it fits: element test records (16 x f32 / f64), for FP32
+    elements, while it fits: element test records (16 x f32 / 14 x f64), for FP32
     also the interaction parameter records, then the culling grid as uint16
     cell offsets and uint16 element indices (tight tier) and the successor
     blocks of both tiers; then the L1 transmission tables of stack stages
@@ -845,7 +846,9 @@ def _build_lds(tables, budget32=None, budget64=None):
             n = len(st.elements)
             if st.kind not in PLANE_ARRAYS or n < 2:
                 continue
-            recs = (tables.elem_t32 if prec == 32 else tables.elem_t)[st.elem0:st.elem0 + n]
+            # FP32 records keep their 16 words (four 16-byte loads), FP64
+            # records the 14 in use
+            recs = (tables.elem_t32 if prec == 32 else tables.elem_t[:, :14])[st.elem0:st.elem0 + n]
             params = (_param_records32(tables, st)
                       if (prec == 32 and st.kind in (STAGE_GRATING, STAGE_STACK)) else None)
             g = st.grid

@@ -39,6 +39,12 @@
 #define MX_E2W 1.2398419292004202e-06   /* keV -> mm, marxs/__init__.py:14 */
 #define MX_E2W_F 1.2398419292004202e-06f
 #define MX_ORDER_NONE (-2147483647 - 1)
+#define MX_LT64 14              /* words of an FP64 test record in LDS: those in
+                                   use of the 16 in global memory.  With them 800
+                                   facets and an interpolated efficiency fit
+                                   (1e6 photons 181 -> 167 us); seven 16-byte words
+                                   also begin in different banks for different
+                                   elements, which measured nothing here     */
 #define MX_DR 18                /* float64 words of a detector record in LDS */
 #ifndef MX_BLOCK32
 #define MX_BLOCK32 1024         /* one workgroup per CU holds the LDS image   */
@@ -1523,11 +1529,11 @@ __device__ __forceinline__ void tube_stage(const MxTables &T, const MxPhotons &P
 #ifndef MX_SCAN_PREFETCH
 #define MX_SCAN_PREFETCH 1
 #endif
-template <int PREC, typename ETP, typename ITP>
+template <int PREC, bool L, typename ETP, typename ITP>
 __device__ __forceinline__ int scan_next(ETP et, bool list, ITP items, int tb, int te,
                                          int last, d3 p, d3 d, f3 pr, f3 df, float kmin32,
                                          d3 &q, double &ly, double &lz, float &kf, const Counters &cnt) {
-    constexpr int G = MX_SCAN_GROUP;
+    constexpr int G = MX_SCAN_GROUP, W = L && PREC == 64 ? MX_LT64 : MX_ET;
 #if MX_SCAN_PREFETCH
     if (G == 1 && list && PREC == 64) {
         // the next candidate's index is read while the current one is
@@ -1542,13 +1548,13 @@ __device__ __forceinline__ int scan_next(ETP et, bool list, ITP items, int tb, i
             if (PREC == 64) {
                 d3 qq;
                 double yy, zz;
-                if (plane_test64((const double *)et + (size_t)j * MX_ET, p, d, qq, yy, zz) && j0 > last) {
+                if (plane_test64((const double *)et + (size_t)j * W, p, d, qq, yy, zz) && j0 > last) {
                     q = qq; ly = yy; lz = zz;
                     return j0;
                 }
             } else {
                 float kk, yy, zz;
-                if (plane_test32((const float *)et + (size_t)j * MX_ET, pr, df, kmin32, kk, yy, zz) && j0 > last) {
+                if (plane_test32((const float *)et + (size_t)j * W, pr, df, kmin32, kk, yy, zz) && j0 > last) {
                     kf = kk; ly = yy; lz = zz;
                     return j0;
                 }
@@ -1573,7 +1579,7 @@ __device__ __forceinline__ int scan_next(ETP et, bool list, ITP items, int tb, i
 #pragma unroll
             for (int g = 0; g < G; ++g) {
                 const int j = jj[g] > last ? jj[g] : 0;
-                hh[g] = plane_test64((const double *)et + (size_t)j * MX_ET, p, d, qq[g], yy[g], zz[g])
+                hh[g] = plane_test64((const double *)et + (size_t)j * W, p, d, qq[g], yy[g], zz[g])
                         && jj[g] > last;
             }
 #pragma unroll
@@ -1584,7 +1590,7 @@ __device__ __forceinline__ int scan_next(ETP et, bool list, ITP items, int tb, i
 #pragma unroll
             for (int g = 0; g < G; ++g) {
                 const int j = jj[g] > last ? jj[g] : 0;
-                hh[g] = plane_test32((const float *)et + (size_t)j * MX_ET, pr, df, kmin32, kk[g], yy[g], zz[g])
+                hh[g] = plane_test32((const float *)et + (size_t)j * W, pr, df, kmin32, kk[g], yy[g], zz[g])
                         && jj[g] > last;
             }
 #pragma unroll
@@ -1950,11 +1956,11 @@ __device__ __forceinline__ bool array_stage(const MxTables &T, const MxPhotons &
         const int *items_g = mode == 3 ? su_g : (mode == 5 ? sul_g : T.cell_items);
         if (L) {
             if (lds_lists && (lds_loose || mode != 4))
-                hit = scan_next<PREC>(rec_l, list,
+                hit = scan_next<PREC, true>(rec_l, list,
                                       mode == 3 ? su_l + su_o : (mode == 5 ? sul_l + su_o : (mode == 4 ? itl_l : it_l)),
                                       tb, te, last, R.p, R.d, pr, R.df, kmin32, q, ly, lz, kf, cnt);
             else
-                hit = scan_next<PREC>(rec_l, list, items_g, tb, te, last,
+                hit = scan_next<PREC, true>(rec_l, list, items_g, tb, te, last,
                                       R.p, R.d, pr, R.df, kmin32, q, ly, lz, kf, cnt);
         } else if (EXT && n_el == 1 && !list) {
             // one element: its record is the same in every lane (scalar loads)
@@ -1973,10 +1979,10 @@ __device__ __forceinline__ bool array_stage(const MxTables &T, const MxPhotons &
             }
             hit = on ? 0 : -1;
         } else if (PREC == 64) {
-            hit = scan_next<PREC>(T.elem_t + (size_t)e0 * MX_ET, list, items_g,
+            hit = scan_next<PREC, false>(T.elem_t + (size_t)e0 * MX_ET, list, items_g,
                                   tb, te, last, R.p, R.d, pr, R.df, kmin32, q, ly, lz, kf, cnt);
         } else {
-            hit = scan_next<PREC>(T.elem_t32 + (size_t)e0 * MX_ET, list, items_g,
+            hit = scan_next<PREC, false>(T.elem_t32 + (size_t)e0 * MX_ET, list, items_g,
                                   tb, te, last, R.p, R.d, pr, R.df, kmin32, q, ly, lz, kf, cnt);
         }
         if (hit < 0) break;
@@ -1993,7 +1999,7 @@ __device__ __forceinline__ bool array_stage(const MxTables &T, const MxPhotons &
 
         // ---- interaction with element `hit`
         const size_t eg = (size_t)(e0 + hit);
-        const double *et = (L && PREC == 64) ? (const double *)rec_l + (size_t)hit * MX_ET : T.elem_t + eg * MX_ET;
+        const double *et = (L && PREC == 64) ? (const double *)rec_l + (size_t)hit * MX_LT64 : T.elem_t + eg * MX_ET;
         const double *ep = T.elem_p + eg * MX_EP;
         const int *ei = T.elem_i + eg * MX_EI;
         int id;
