@@ -1400,6 +1400,14 @@ extern "C" int mx_order_stats_static(const MxOrderStats *a, void *stream) {
     if (a->n_orders < 1 || a->n_orders > MX_MAX_ORDERS) { mx_set_error("order stats: n_orders outside [1, 64]"); return 1; }
     OsPlan L;
     os_plan(a->n, a->n_orders, a->value != nullptr, L);
+    // sums alone: the workspace grows with the number of orders, so that many
+    // orders of a list of several 1e8 photons take a few calls, one after
+    // another on the stream
+    int per = a->n_orders;
+    while (!a->value && per > 1 && (int64_t)L.total > (int64_t)MX_OS_STATIC_BYTES) {
+        per = (per + 1) / 2;
+        os_plan(a->n, per, false, L);
+    }
     if ((int64_t)L.total > (int64_t)MX_OS_STATIC_BYTES) {
         char buf[256];
         snprintf(buf, sizeof(buf),
@@ -1414,5 +1422,14 @@ extern "C" int mx_order_stats_static(const MxOrderStats *a, void *stream) {
     MxOrderStats b = *a;
     b.workspace = ws;
     b.workspace_bytes = (int64_t)MX_OS_STATIC_BYTES;
-    return mx_order_stats(&b, stream);
+    if (per == a->n_orders || !a->orders || !a->prob_sum || !a->count) return mx_order_stats(&b, stream);
+    for (int k = 0; k < a->n_orders; k += per) {
+        b.n_orders = a->n_orders - k < per ? a->n_orders - k : per;
+        b.orders = a->orders + k;
+        b.prob_sum = a->prob_sum + k;
+        b.count = a->count + k;
+        const int rc = mx_order_stats(&b, stream);
+        if (rc) return rc;
+    }
+    return 0;
 }
