@@ -9,8 +9,10 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize('n', [1, 2, 255, 256, 257, 100003])
 @pytest.mark.parametrize('width', [3, 4, 6])
-def test_columns_and_back(gpu, n, width):
+def test_columns_and_back(gpu, n, width, monkeypatch):
+    from marxs_amd import tracer
     from marxs_amd.tracer import _columns_of, _rows_of
+    monkeypatch.setattr(tracer, 'ROWS_ON_DEVICE', 0)
     rows = np.random.default_rng(n).normal(size=(n, width))
     rows[0, :2] = [np.nan, -0.]
     cols = _columns_of(rows, gpu)
@@ -21,11 +23,12 @@ def test_columns_and_back(gpu, n, width):
 
 
 @pytest.mark.parametrize('kind', ['fortran', 'readonly', 'float32', 'reversed', 'empty'])
-def test_table_forms(gpu, kind):
+@pytest.mark.parametrize('rows', [77, 8191, 8192])
+def test_table_forms(gpu, kind, rows):
     import warnings
     import marxs_amd as mx
     from marxs_amd.tracer import DevicePhotons
-    n = 0 if kind == 'empty' else 77
+    n = 0 if kind == 'empty' else rows
     rng = np.random.default_rng(5)
     d = rng.normal(size=(n, 4))
     if kind == 'fortran':
