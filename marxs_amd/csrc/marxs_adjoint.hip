@@ -746,8 +746,11 @@ extern "C" int mx_adjoint_step(const MxAdjointStep *s, void *stream) {
         mx_set_error("adjoint step: a required pose pointer is NULL");
         return 1;
     }
-    if (s->n_tasks > 0 && (!a.pos[0] || !a.pos[1] || !a.pos[2] || !a.dir[0] || !a.dir[1] || !a.dir[2] || !a.energy ||
-                           !a.order || !a.ccd || !a.ccd_t || !s->task || !s->part)) {
+    // without photons every task is empty, and a column of no length may have
+    // no address
+    const unsigned tasks = a.n > 0 ? (unsigned)s->n_tasks : 0;
+    if (tasks > 0 && (!a.pos[0] || !a.pos[1] || !a.pos[2] || !a.dir[0] || !a.dir[1] || !a.dir[2] || !a.energy ||
+                      !a.order || !a.ccd || !a.ccd_t || !s->task || !s->part)) {
         mx_set_error("adjoint step: a required photon pointer is NULL");
         return 1;
     }
@@ -757,10 +760,10 @@ extern "C" int mx_adjoint_step(const MxAdjointStep *s, void *stream) {
         return 1;
     }
     hipStream_t st = (hipStream_t)stream;
-    if (s->n_tasks > 0 && a.precision == MX_PREC_FP64)
-        hipLaunchKernelGGL(mx_adjoint_task_kernel<64>, dim3((unsigned)s->n_tasks), dim3(AJ_TASK), 0, st, *s);
-    else if (s->n_tasks > 0)
-        hipLaunchKernelGGL(mx_adjoint_task_kernel<32>, dim3((unsigned)s->n_tasks), dim3(AJ_TASK), 0, st, *s);
+    if (tasks > 0 && a.precision == MX_PREC_FP64)
+        hipLaunchKernelGGL(mx_adjoint_task_kernel<64>, dim3(tasks), dim3(AJ_TASK), 0, st, *s);
+    else if (tasks > 0)
+        hipLaunchKernelGGL(mx_adjoint_task_kernel<32>, dim3(tasks), dim3(AJ_TASK), 0, st, *s);
     hipLaunchKernelGGL(mx_adjoint_finish_kernel, dim3((unsigned)p.n_facet), dim3(128), 0, st, *s);
     hipError_t err = hipGetLastError();
     if (err != hipSuccess) {
