@@ -160,6 +160,7 @@ class DevicePhotons:
         self.prob = col(prob)
         if pos is None:
             self.pos = torch.empty((3, self.n), **f)
+            self._pos_unset = True
             self.has_pos = False
         else:
             self.pos = col(pos)
@@ -183,13 +184,35 @@ class DevicePhotons:
                    copy=dev.type != 'cuda')     # there every column is a new tensor
         return self
 
+    # Positions that nobody has asked for are memory as it was allocated, and a
+    # clone need not copy them.  Whoever has the tensor may write to it (a
+    # kernel, a graph, the caller), so from then on they count as set, also in
+    # copies that share it.
+    @property
+    def pos(self):
+        self._pos_unset = False
+        return self._pos
+
+    @pos.setter
+    def pos(self, value):
+        self._pos = value
+        self._pos_unset = False
+
+    def __getstate__(self):
+        self._pos_unset = False
+        return {'pos' if k == '_pos' else k: v for k, v in self.__dict__.items() if k != '_pos_unset'}
+
+    def __setstate__(self, state):
+        for k, v in state.items():
+            setattr(self, k, v)
+
     def clone(self):
         c = DevicePhotons.__new__(DevicePhotons)
         c.device, c.n, c.has_pos = self.device, self.n, self.has_pos
         for a in ('dir', 'pol', 'energy', 'prob'):
             setattr(c, a, getattr(self, a).clone())
-        # positions that no trace has set yet are memory as it was allocated
-        c.pos = self.pos.clone() if self.has_pos else torch.empty_like(self.pos)
+        c.pos = torch.empty_like(self._pos) if self._pos_unset else self._pos.clone()
+        c._pos_unset = self._pos_unset
         c.fcols = {k: v.clone() for k, v in self.fcols.items()}
         c.icols = {k: v.clone() for k, v in self.icols.items()}
         return c
