@@ -374,6 +374,7 @@ typedef struct MxAdjointStep {
     double *theta_out;         /* [n_facet][6] copy of pose.theta, may be NULL */
     double *period_out;        /* [n_facet] copy of pose.period, may be NULL */
     double *moments_out;       /* [3] sum w, sum w (y - y_shift), sum w (y - y_shift)^2, may be NULL */
+    double *sums_out;          /* [n_facet][2 * 13] A and B of each facet, as MX_AJ_SUMS leaves them, may be NULL */
     int32_t n_tasks;           /* task_first[n_facet] at least */
     int32_t reserved;
 } MxAdjointStep;

@@ -73,7 +73,7 @@ class MxAdjointStep(ctypes.Structure):
     _fields_ = [('photons', MxAdjointArgs), ('pose', MxPoseArgs), ('task', P), ('task_first', P),
                 ('part', P), ('grad_theta', P), ('grad_period', P), ('loss_out', P),
                 ('theta_out', P), ('period_out', P), ('moments_out', P),
-                ('n_tasks', ctypes.c_int32), ('reserved', ctypes.c_int32)]
+                ('sums_out', P), ('n_tasks', ctypes.c_int32), ('reserved', ctypes.c_int32)]
 
 
 class MxOrderStats(ctypes.Structure):

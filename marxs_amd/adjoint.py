@@ -279,7 +279,7 @@ class AdjointProblem:
             s.photons = self._args(pb['geom'], precision, src=pb['src'])
             s.pose = self._pose_args(2)
             s.task, s.task_first, s.part = (pb[k].data_ptr() for k in ('task', 'task_first', 'part'))
-            s.moments_out = pb['moments'].data_ptr()
+            s.moments_out, s.sums_out = pb['moments'].data_ptr(), pb['sums'].data_ptr()
             s.n_tasks = pb['task'].shape[0]
             pb['step'][precision] = s
         s = _lib.MxAdjointStep.from_buffer_copy(s)
@@ -323,7 +323,7 @@ class AdjointProblem:
         the chain rule back to the poses with dL/dg = A / W + (B - a A) / (W
         sigma) (L = mu + sigma, dL/dy_i = w_i / W (1 + (y_i - mu) / sigma)).
         Results: ``buffers['loss']`` and ``buffers['grad7']`` (d/d theta, d/d
-        period)."""
+        period); ``buffers['sums']`` (A, B per facet) and ``buffers['moments']``."""
         s = self._step_args(precision)
         pb = self._pb
         s.pose.theta, s.pose.period = pb['theta'].data_ptr(), pb['period'].data_ptr()

@@ -629,7 +629,10 @@ __global__ __launch_bounds__(128) void mx_adjoint_finish_kernel(MxAdjointStep S)
 #pragma unroll 8
         for (int j = lane; j < n_tasks; j += 64)
             for (int k = 0; k < 3; ++k) m[k] += task_moments(S, k)[j];
-        if (lane < 2 * AJ_NG) sums[lane] = x;
+        if (lane < 2 * AJ_NG) {
+            sums[lane] = x;
+            if (S.sums_out) S.sums_out[(size_t)f * (2 * AJ_NG) + lane] = x;
+        }
 #pragma unroll
         for (int k = 0; k < 3; ++k) m[k] = __shfl(wave_total(m[k]), 63);
     } else {
