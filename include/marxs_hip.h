@@ -356,7 +356,8 @@ int mx_facet_pose(const MxPoseArgs *args, void *stream);
  * ordered by facet: the results of mx_facet_pose mode 0, mx_adjoint with
  * MX_AJ_SUMS and mx_facet_pose mode 2, up to the order of the sums, which is
  * fixed.  A task is a run of photons of one facet: task[3 j] its facet,
- * [task[3 j + 1], task[3 j + 2]) its photons (an empty run: no task); the
+ * [task[3 j + 1], task[3 j + 2]) its photons (an empty run, or one with a
+ * facet or photons that there are not, counts nothing); the
  * tasks of facet f are task_first[f] .. task_first[f + 1] - 1, and a photon
  * in no task does not count.  photons: n, pos, dir, energy, weight, order,
  * ccd, ccd_t, y_shift, n_ccd, coord and precision are read.  pose: everything

@@ -250,6 +250,8 @@ class AdjointProblem:
                      'facet': self.facet[idx].contiguous(), 'order': self.order[idx].contiguous(),
                      'ccd': self.ccd[idx].contiguous()}
         self._tasks(pb, facet.contiguous())
+        # the buffers are read on whatever stream a later call launches on
+        torch.cuda.current_stream(self.device).synchronize()
         self._pb = pb
         return pb
 

@@ -561,8 +561,16 @@ __global__ __launch_bounds__(AJ_TASK) void mx_adjoint_task_kernel(MxAdjointStep 
     __shared__ double red[AJ_TASK / 64][AJ_SUMS];
     const int32_t *task = S.task + 3 * (size_t)blockIdx.x;
     const int f = task[0], b = task[1], e = task[2];
-    if (b >= e) return;
     const MxAdjointArgs &A = S.photons;
+    auto put = [&](int k, double x) {
+        if (k < 2 * AJ_NG) task_sums(S, blockIdx.x)[k] = x;
+        else task_moments(S, k - 2 * AJ_NG)[blockIdx.x] = x;
+    };
+    if (b >= e || b < 0 || e > A.n || f < 0 || f >= S.pose.n_facet) {
+        // an empty task, or one that is not of these photons and facets
+        if (threadIdx.x < AJ_SUMS) put((int)threadIdx.x, 0.0);
+        return;
+    }
     int i = b + (int)threadIdx.x;
     // a work-item without a photon loads the task's last one
     const int i0 = i < e ? i : e - 1;
@@ -604,8 +612,7 @@ __global__ __launch_bounds__(AJ_TASK) void mx_adjoint_task_kernel(MxAdjointStep 
         const int k = (int)threadIdx.x;
         double x = 0.0;
         for (int w = 0; w < AJ_TASK / 64; ++w) x += red[w][k];
-        if (k < 2 * AJ_NG) task_sums(S, blockIdx.x)[k] = x;
-        else task_moments(S, k - 2 * AJ_NG)[blockIdx.x] = x;
+        put(k, x);
     }
 }
 
@@ -621,7 +628,9 @@ __global__ __launch_bounds__(128) void mx_adjoint_finish_kernel(MxAdjointStep S)
     const MxPoseArgs &P = S.pose;
     double m[3] = {0.0, 0.0, 0.0};
     if (threadIdx.x < 64) {
-        const int n_tasks = S.task_first[P.n_facet], j0 = S.task_first[f], j1 = S.task_first[f + 1];
+        const int all = S.task_first[P.n_facet], first = S.task_first[f], end = S.task_first[f + 1];
+        const int n_tasks = all < S.n_tasks ? all : S.n_tasks;
+        const int j0 = first > 0 ? first : 0, j1 = end < n_tasks ? end : n_tasks;
         double x = 0.0;
         if (lane < 2 * AJ_NG)
 #pragma unroll 4

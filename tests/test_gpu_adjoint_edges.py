@@ -57,3 +57,47 @@ def test_sums_are_in_the_buffers(gpu, precision, call):
     assert bool((torch.abs(pb['sums'] - want) <= 1e-12 * torch.abs(want).max(0).values).all())
     assert abs(float(pb['moments'][0] / moments[0]) - 1.) <= 1e-14
     assert abs(float(pb['moments'][2] / moments[2]) - 1.) <= 1e-12
+
+
+@pytest.mark.parametrize('precision', [64, 32])
+def test_tasks_outside_the_lists(gpu, precision):
+    """A task whose facet or photons there are not counts nothing: the result
+    is that of a list in which it is empty, bit for bit."""
+    import torch
+    prob = _problem(gpu, 50, np.full(50, 300), 7)
+    task, src = prob.buffers['task'], prob.buffers['src']
+    kept, n = task.clone(), src['n']
+    bad = {3: (-1, 0, 100), 10: (50, 0, 100), 20: (2 ** 31 - 1, 5, 6), 30: (7, -1, 100), 40: (7, n - 1, n + 1),
+           50: (7, n, n + 128), 60: (7, -2 ** 31, 2 ** 31 - 1), 70: (7, 100, 99)}
+    got = []
+    for rows in ({j: (0, 0, 0) for j in bad}, bad):
+        task.copy_(kept)
+        for j, row in rows.items():
+            task[j] = torch.tensor(row, dtype=torch.int32)
+        prob.buffers['part'].fill_(float('nan'))
+        got.append(prob.loss_and_grad(prob.theta0, prob.period0, precision))
+    for a, b in zip(*got):
+        assert torch.equal(a, b) and bool(torch.isfinite(a).all())
+
+
+def test_buffers_are_complete_when_they_are_handed_out(gpu, monkeypatch):
+    """Building the buffers waits for the kernels that fill them (delayed
+    here), so that a launch on another stream finds them filled."""
+    import torch
+    from marxs_amd.adjoint import AdjointProblem
+    prob = _problem(gpu, 50, np.full(50, 20), 8)
+    tasks = AdjointProblem._tasks
+
+    def delayed(self, *args):
+        torch.cuda._sleep(20_000_000)
+        return tasks(self, *args)
+    monkeypatch.setattr(AdjointProblem, '_tasks', delayed)
+    prob._pose_buffers()
+    assert torch.cuda.current_stream().query()
+    other = torch.cuda.Stream()
+    prob.buffers['theta'].copy_(prob.theta0)
+    prob.buffers['period'].copy_(prob.period0)
+    other.wait_stream(torch.cuda.current_stream())
+    prob.launch_loss_and_grad(64, other.cuda_stream)
+    torch.cuda.synchronize()
+    assert float(prob.buffers['loss']) == float(prob.loss_and_grad(prob.theta0, prob.period0, 64)[0])
