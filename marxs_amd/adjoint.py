@@ -231,7 +231,9 @@ class AdjointProblem:
         pb['sums'] = pb['accum'][:F * 26].view(F, 26)
         pb['moments'] = pb['accum'][F * 26:]
         # shift of the moments: the weighted mean coordinate at the base pose
-        pose = _lib.MxPoseArgs(n_facet=F, mode=0, theta=self.theta0.data_ptr(), period=self.period0.data_ptr(),
+        theta0, period0 = (x.to(**f64).contiguous() for x in (self.theta0[:, :6].detach().expand(F, 6),
+                                                              self.period0.detach().expand(F)))
+        pose = _lib.MxPoseArgs(n_facet=F, mode=0, theta=theta0.data_ptr(), period=period0.data_ptr(),
                                **{k: pb[k].data_ptr() for k in ('gu', 't0', 'rpost', 'zoom', 'extra', 'geom')})
         _lib.check(_lib.lib.mx_facet_pose(ctypes.byref(pose), ctypes.c_void_p(
             torch.cuda.current_stream(self.device).cuda_stream)))

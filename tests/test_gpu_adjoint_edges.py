@@ -101,3 +101,20 @@ def test_buffers_are_complete_when_they_are_handed_out(gpu, monkeypatch):
     prob.launch_loss_and_grad(64, other.cuda_stream)
     torch.cuda.synchronize()
     assert float(prob.buffers['loss']) == float(prob.loss_and_grad(prob.theta0, prob.period0, 64)[0])
+
+
+def test_base_pose_in_other_layouts(gpu):
+    """The base pose may be a strided view or of single precision: the moments
+    are shifted by the same coordinate."""
+    import torch
+    prob = _problem(gpu, 50, np.full(50, 20), 9)
+    theta0, period0 = prob.theta0.to(torch.float32).to(torch.float64), prob.period0.to(torch.float32).to(torch.float64)
+    wide = torch.full((50, 12), 3., dtype=torch.float64, device=gpu)
+    wide[:, ::2] = theta0
+    shifts = []
+    for theta, period in ((theta0, period0), (wide[:, ::2], period0.repeat_interleave(2)[::2]),
+                          (theta0.to(torch.float32), period0.to(torch.float32))):
+        prob.theta0, prob.period0, prob._pb = theta, period, None
+        prob.buffers
+        shifts.append(prob.y_shift)
+    assert shifts[0] == shifts[1] == shifts[2] and np.isfinite(shifts[0])
