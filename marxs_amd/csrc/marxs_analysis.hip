@@ -805,7 +805,7 @@ __device__ __forceinline__ void kept_moments(const ClipOrder &O, const Kept &K, 
     }
     s1 = wave_add(s1);
     s2 = wave_add(s2);
-    if (K.cut) {
+    if (K.cut || all) {
         s1 += K.c0.s1 + K.c1.s1;
         s2 += K.c0.s2 + K.c1.s2;
     }
@@ -1279,7 +1279,16 @@ __global__ __launch_bounds__(MX_OS_CLIP) void mx_os_clip_kernel(MxOrderStats a, 
             }
             K = Q;
             cen = kept_median(O, K, (int64_t)N, (int64_t)below, S, list, H);
-            kept_moments(O, K, N, K.cut ? c : cen, nlist >= 0 && K.cut, mean, sd);
+            // few values: summed again about their own median, as they may be
+            // a pair one standard deviation from it, which stays or goes with
+            // the last bit (more bits are lost in sums about another point)
+            const bool few = N <= (double)MX_OS_CAND && (K.cut || nlist >= 0);
+            if (few) {
+                double unused;
+                cut_bins(O, K, cen, S, p, list, nlist, unused);
+                p ^= 1;
+            }
+            kept_moments(O, K, N, few || !K.cut ? cen : c, nlist >= 0 && (K.cut || few), mean, sd);
             c = cen;
             if (it == a.maxiters) break;
         }
