@@ -80,9 +80,12 @@ def _orders_i32(col):
 
 
 @functools.lru_cache(maxsize=32)
-def _device_orders(orders, device):
-    """Order numbers (a tuple) on the device, read only.  Copying them there
-    on every call takes 20 us, as much as a small list's sums."""
+def _device_orders(orders, device, stream):
+    """Order numbers (a tuple) on the device, read only, for kernels ordered
+    with torch's current stream, whose handle is ``stream``: the memory of an
+    entry that is dropped goes back to that stream, behind the kernels that
+    read it.  Copying them there on every call takes 20 us, as much as a small
+    list's sums."""
     return torch.as_tensor(np.array(orders, dtype=np.int32), device=device)
 
 
@@ -128,7 +131,8 @@ def order_stats(order, prob, orders, value=None, res_filter=False, sigma=3., max
             res.update({'mean': np.full(no, np.nan), 'median': np.full(no, np.nan),
                         'std': np.full(no, np.nan), 'n_kept': np.zeros(no, np.int64)})
         return res
-    ords = _device_orders(tuple(orders.astype(np.int32).tolist()), dev)
+    current = torch.cuda.current_stream(dev)
+    ords = _device_orders(tuple(orders.astype(np.int32).tolist()), dev, current.cuda_stream)
     wsb = int(_lib.lib.mx_order_stats_workspace(n, no, int(v is not None)))
     if wsb < 0:
         raise ValueError('order statistics: invalid sizes')
@@ -153,8 +157,13 @@ def order_stats(order, prob, orders, value=None, res_filter=False, sigma=3., max
     for j, k in enumerate(keys):
         setattr(a, k, base + 8 * j * no)
     if stream is None:
-        stream = torch.cuda.current_stream(dev).cuda_stream
-    _lib.check(_lib.lib.mx_order_stats(a, stream))
+        _lib.check(_lib.lib.mx_order_stats(a, current.cuda_stream))
+    else:
+        # inputs, workspace and results belong to the current stream
+        other = torch.cuda.ExternalStream(getattr(stream, 'value', stream) or 0, device=dev)
+        other.wait_stream(current)
+        _lib.check(_lib.lib.mx_order_stats(a, stream))
+        current.wait_stream(other)
     host = buf.cpu().numpy()
     res = {}
     for j, k in enumerate(keys):
