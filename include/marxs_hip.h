@@ -33,7 +33,7 @@
 extern "C" {
 #endif
 
-#define MX_ABI_VERSION 21
+#define MX_ABI_VERSION 22
 
 #define MX_MAX_FCOLS 16
 #define MX_MAX_ICOLS 8
@@ -46,6 +46,11 @@ extern "C" {
 #define MX_EP 16   /* double per element, interaction parameters */
 #define MX_EI 8    /* int32 per element */
 #define MX_SELI 12 /* int32 per order selector */
+#define MX_LT64 14 /* double per element, intersection data in lds_image64: the words
+                      in use of the MX_ET in elem_t (lds_image32 holds all MX_ET floats) */
+#define MX_DR 18   /* double per element of a detector stage in both LDS images, at byte
+                      offset stage_i[51] (FP32) / stage_i[52] (FP64), 0 = not there: elem_t
+                      0-11, elem_p 6-9, then as int32 elem_i 0, 4, 5 and one unused */
 
 /* Order-selector rows sel_i[k][0 .. MX_SELI-1].  Offsets count doubles in
  * sel_d (ints in sel_o); LDS offsets count bytes in that precision's LDS
@@ -121,8 +126,8 @@ extern "C" {
                               600-facet workload, see mx_trace_regroup_pairs) */
 /* bits 8..15: workgroups launched per CU (persistent grid; each takes a
  * contiguous share of the photons, which its waves take in chunks of 64);
- * 0 = the library default: 2 for the FP32 kernel, 1 for the FP64 kernel, 1
- * for the extended kernels (stack, tube or lens-reflectivity stages) */
+ * 0 = the library default, 1.  A list too short for one full workgroup per CU
+ * is spread over the CUs in chunks of 64 whatever is asked for. */
 #define MX_FLAG_WG_PER_CU(n) (((n) & 0xff) << 8)
 /* bits 16..23: regroup a workgroup's rays before a stage only when at most
  * n/256 of them can interact with it (1..255; 0 = the library default) */

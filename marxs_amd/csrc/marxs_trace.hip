@@ -39,13 +39,9 @@
 #define MX_E2W 1.2398419292004202e-06   /* keV -> mm, marxs/__init__.py:14 */
 #define MX_E2W_F 1.2398419292004202e-06f
 #define MX_ORDER_NONE (-2147483647 - 1)
-#define MX_LT64 14              /* words of an FP64 test record in LDS: those in
-                                   use of the 16 in global memory.  With them 800
-                                   facets and an interpolated efficiency fit
-                                   (1e6 photons 181 -> 167 us); seven 16-byte words
-                                   also begin in different banks for different
-                                   elements, which measured nothing here     */
-#define MX_DR 18                /* float64 words of a detector record in LDS */
+// (MX_LT64: with 14 of the 16 words 800 facets and an interpolated efficiency
+// fit, 1e6 photons 181 -> 167 us; seven 16-byte words also begin in different
+// banks for different elements, which measured nothing here)
 #ifndef MX_BLOCK32
 #define MX_BLOCK32 1024         /* one workgroup per CU holds the LDS image   */
 #endif
