@@ -559,6 +559,11 @@ static_assert(AJ_SUMS <= MX_AJ_PART, "a task's sums and moments");
 template <int PREC>
 __global__ __launch_bounds__(AJ_TASK) void mx_adjoint_task_kernel(MxAdjointStep S) {
     __shared__ double red[AJ_TASK / 64][AJ_SUMS];
+    // what the task is checked against, read with the address of the list (the
+    // compiler would read it after the task and wait once more)
+    int n = (int)S.photons.n;    // below 2^31: mx_adjoint_step
+    unsigned n_facet = (unsigned)S.pose.n_facet;
+    asm volatile("" : "+s"(n), "+s"(n_facet));
     const int32_t *task = S.task + 3 * (size_t)blockIdx.x;
     const int f = task[0], b = task[1], e = task[2];
     const MxAdjointArgs &A = S.photons;
@@ -566,7 +571,7 @@ __global__ __launch_bounds__(AJ_TASK) void mx_adjoint_task_kernel(MxAdjointStep 
         if (k < 2 * AJ_NG) task_sums(S, blockIdx.x)[k] = x;
         else task_moments(S, k - 2 * AJ_NG)[blockIdx.x] = x;
     };
-    if (b >= e || b < 0 || e > A.n || f < 0 || f >= S.pose.n_facet) {
+    if ((b >= e) | (b < 0) | (e > n) | ((unsigned)f >= n_facet)) {
         // an empty task, or one that is not of these photons and facets
         if (threadIdx.x < AJ_SUMS) put((int)threadIdx.x, 0.0);
         return;
@@ -616,11 +621,41 @@ __global__ __launch_bounds__(AJ_TASK) void mx_adjoint_task_kernel(MxAdjointStep 
     }
 }
 
+// The moments of all tasks, added once by one workgroup instead of by every
+// facet's: that takes another launch, while every facet reading every task
+// takes facets x tasks x 24 B from the caches.  A call FP32 with every facet
+// adding / with this kernel, us: 600 facets, 693 tasks 18.8 / 21.3; 2100, 2428
+// 30.7 / 31.5; 3000, 3468 41.4 / 37.4; 9000, 9140 167 / 81; 22000, 22859
+// 771 / 198.
+#define AJ_MANY 6000000         // facets x tasks from which on it pays
+#define AJ_MOMENTS 1024
+__device__ __forceinline__ double *all_moments(const MxAdjointStep &S) { return S.part + AJ_SUMS * (size_t)S.n_tasks; }
+static_assert(AJ_SUMS + 3 <= MX_AJ_PART, "the moments of all tasks behind those of each");
+__global__ __launch_bounds__(AJ_MOMENTS) void mx_adjoint_moments_kernel(MxAdjointStep S) {
+    __shared__ double red[3][AJ_MOMENTS / 64];
+    const int all = S.task_first[S.pose.n_facet], n_tasks = all < S.n_tasks ? all : S.n_tasks;
+    double m[3] = {0.0, 0.0, 0.0};
+#pragma unroll 4
+    for (int j = threadIdx.x; j < n_tasks; j += AJ_MOMENTS)
+        for (int k = 0; k < 3; ++k) m[k] += task_moments(S, k)[j];
+    for (int k = 0; k < 3; ++k) {
+        const double x = wave_total(m[k]);
+        if ((threadIdx.x & 63) == 63) red[k][threadIdx.x >> 6] = x;
+    }
+    __syncthreads();
+    if (threadIdx.x < 3) {
+        double x = 0.0;
+        for (int w = 0; w < AJ_MOMENTS / 64; ++w) x += red[threadIdx.x][w];
+        all_moments(S)[threadIdx.x] = x;
+    }
+}
+
 // Two waves per facet: the first adds the sums of the facet's tasks and, for
 // itself, the moments of all tasks, while the second forms the facet's frame
 // and its derivatives.  Bound by latency: one wave doing both, with the moments
 // 256 bytes apart, took 9.9 us for 200 facets and 16.5 us for 600, this 6.0 and
-// 7.0.
+// 7.0.  (MANY: the moments are there, from mx_adjoint_moments_kernel.)
+template <bool MANY>
 __global__ __launch_bounds__(128) void mx_adjoint_finish_kernel(MxAdjointStep S) {
     __shared__ double sums[2 * AJ_NG];
     __shared__ PoseParts parts;
@@ -628,22 +663,24 @@ __global__ __launch_bounds__(128) void mx_adjoint_finish_kernel(MxAdjointStep S)
     const MxPoseArgs &P = S.pose;
     double m[3] = {0.0, 0.0, 0.0};
     if (threadIdx.x < 64) {
+        int most = S.n_tasks;
+        asm volatile("" : "+s"(most));
         const int all = S.task_first[P.n_facet], first = S.task_first[f], end = S.task_first[f + 1];
-        const int n_tasks = all < S.n_tasks ? all : S.n_tasks;
-        const int j0 = first > 0 ? first : 0, j1 = end < n_tasks ? end : n_tasks;
+        const int n_tasks = all < most ? all : most, j0 = first > 0 ? first : 0, j1 = end < most ? end : most;
         double x = 0.0;
         if (lane < 2 * AJ_NG)
 #pragma unroll 4
             for (int j = j0; j < j1; ++j) x += task_sums(S, j)[lane];
+        if (MANY) {
+            for (int k = 0; k < 3; ++k) m[k] = all_moments(S)[k];
+        } else {
 #pragma unroll 8
-        for (int j = lane; j < n_tasks; j += 64)
-            for (int k = 0; k < 3; ++k) m[k] += task_moments(S, k)[j];
-        if (lane < 2 * AJ_NG) {
-            sums[lane] = x;
-            if (S.sums_out) S.sums_out[(size_t)f * (2 * AJ_NG) + lane] = x;
-        }
+            for (int j = lane; j < n_tasks; j += 64)
+                for (int k = 0; k < 3; ++k) m[k] += task_moments(S, k)[j];
 #pragma unroll
-        for (int k = 0; k < 3; ++k) m[k] = __shfl(wave_total(m[k]), 63);
+            for (int k = 0; k < 3; ++k) m[k] = __shfl(wave_total(m[k]), 63);
+        }
+        if (lane < 2 * AJ_NG) sums[lane] = x;
     } else {
         PoseParts p;
         pose_parts(P, f, p);
@@ -658,7 +695,11 @@ __global__ __launch_bounds__(128) void mx_adjoint_finish_kernel(MxAdjointStep S)
         }
     }
     __syncthreads();
-    if (threadIdx.x >= 64) return;
+    if (threadIdx.x >= 64) {
+        // (here, as the barrier would wait for the stores)
+        if (S.sums_out && lane < 2 * AJ_NG) S.sums_out[(size_t)f * (2 * AJ_NG) + lane] = sums[lane];
+        return;
+    }
     double gg[MX_AJ_NGRAD], out[7];
     sums_to_grad(sums, m, gg);
     pose_chain(P, f, parts, gg, out);
@@ -776,7 +817,13 @@ extern "C" int mx_adjoint_step(const MxAdjointStep *s, void *stream) {
         hipLaunchKernelGGL(mx_adjoint_task_kernel<64>, dim3(tasks), dim3(AJ_TASK), 0, st, *s);
     else if (tasks > 0)
         hipLaunchKernelGGL(mx_adjoint_task_kernel<32>, dim3(tasks), dim3(AJ_TASK), 0, st, *s);
-    hipLaunchKernelGGL(mx_adjoint_finish_kernel, dim3((unsigned)p.n_facet), dim3(128), 0, st, *s);
+    const bool many = tasks > 0 && (int64_t)p.n_facet * s->n_tasks >= AJ_MANY;
+    if (many) {
+        hipLaunchKernelGGL(mx_adjoint_moments_kernel, dim3(1), dim3(AJ_MOMENTS), 0, st, *s);
+        hipLaunchKernelGGL(mx_adjoint_finish_kernel<true>, dim3((unsigned)p.n_facet), dim3(128), 0, st, *s);
+    } else {
+        hipLaunchKernelGGL(mx_adjoint_finish_kernel<false>, dim3((unsigned)p.n_facet), dim3(128), 0, st, *s);
+    }
     hipError_t err = hipGetLastError();
     if (err != hipSuccess) {
         char buf[256];

@@ -118,3 +118,32 @@ def test_base_pose_in_other_layouts(gpu):
         prob.buffers
         shifts.append(prob.y_shift)
     assert shifts[0] == shifts[1] == shifts[2] and np.isfinite(shifts[0])
+
+
+@pytest.mark.parametrize('precision', [64, 32])
+@pytest.mark.parametrize('facets', [2300, 2400])
+def test_many_facets(gpu, facets, precision, monkeypatch):
+    """Below and above the number of facets and tasks (2300 x 2479, 2400 x
+    2587) from which on the moments are added by a kernel of their own; bounds
+    as for the smaller problems (sums of 10 photons a facet, moments of 24000)."""
+    import torch
+    from marxs_amd import configs
+    whole = configs.cat_rowland_instrument
+
+    def small_facets(n):
+        inst, parts = whole(50)
+        gas = configs._gas_with_n(parts['rowland'], n, [301.5, 562.5], [8., 8.],
+                                  {'zoom': [1, 3., 3.], 'd': 2e-4, 'order_selector': parts['efficiency']})
+        return inst, {**parts, 'gratings': gas}
+    monkeypatch.setattr(configs, 'cat_rowland_instrument', small_facets)
+    prob = _problem(gpu, facets, np.full(facets, 10), facets)
+    assert (facets * prob.buffers['task'].shape[0] >= 6000000) == (facets == 2400)
+    loss, gt, gp = prob.loss_and_grad(prob.theta0, prob.period0, precision)
+    again = prob.loss_and_grad(prob.theta0, prob.period0, precision)
+    assert torch.equal(loss, again[0]) and torch.equal(gt, again[1]) and torch.equal(gp, again[2])
+    moments = prob.buffers['moments'].clone()
+    loss_u, g7, _ = _unordered(prob, prob.theta0, prob.period0, precision)
+    assert abs(loss.item() - loss_u.item()) <= 1e-12 * abs(loss_u.item())
+    assert abs(float(moments[2] / prob.buffers['moments'][2]) - 1.) <= 1e-12
+    got = torch.cat([gt, gp[:, None]], 1)
+    assert bool((torch.abs(got - g7) <= 1e-11 * torch.abs(g7).max(0).values).all())
