@@ -231,8 +231,9 @@ class AdjointProblem:
         pb['sums'] = pb['accum'][:F * 26].view(F, 26)
         pb['moments'] = pb['accum'][F * 26:]
         # shift of the moments: the weighted mean coordinate at the base pose
-        theta0, period0 = (x.to(**f64).contiguous() for x in (self.theta0[:, :6].detach().expand(F, 6),
-                                                              self.period0.detach().expand(F)))
+        theta0, period0 = (x if x.dtype == torch.float64 and x.is_contiguous() and x.shape == shape
+                           and x.device == pb['gu'].device else x.detach().expand(shape).to(**f64).contiguous()
+                           for x, shape in ((self.theta0, (F, 6)), (self.period0, (F,))))
         pose = _lib.MxPoseArgs(n_facet=F, mode=0, theta=theta0.data_ptr(), period=period0.data_ptr(),
                                **{k: pb[k].data_ptr() for k in ('gu', 't0', 'rpost', 'zoom', 'extra', 'geom')})
         _lib.check(_lib.lib.mx_facet_pose(ctypes.byref(pose), ctypes.c_void_p(
@@ -249,11 +250,12 @@ class AdjointProblem:
         pb['src'] = {'n': int(idx.numel()), 'idx': idx,
                      'pos': self.pos[:, idx].contiguous(), 'dir': self.dir[:, idx].contiguous(),
                      'energy': self.energy[idx].contiguous(), 'weight': self.weight[idx].contiguous(),
-                     'facet': self.facet[idx].contiguous(), 'order': self.order[idx].contiguous(),
+                     'facet': facet, 'order': self.order[idx].contiguous(),
                      'ccd': self.ccd[idx].contiguous()}
-        self._tasks(pb, facet.contiguous())
-        # the buffers are read on whatever stream a later call launches on
-        torch.cuda.current_stream(self.device).synchronize()
+        self._tasks(pb, facet)
+        # the kernels that fill the buffers run on this stream (_built)
+        stream = torch.cuda.current_stream(self.device)
+        pb['built'] = (stream.cuda_stream, stream.record_event())
         self._pb = pb
         return pb
 
@@ -272,6 +274,19 @@ class AdjointProblem:
         stream = torch.cuda.current_stream(self.device).cuda_stream
         _lib.check(_lib.lib.mx_adjoint_tasks(facet.data_ptr(), n, F, size, pb['task_first'].data_ptr(),
                                              pb['task'].data_ptr(), count, ctypes.c_void_p(stream)))
+
+    @staticmethod
+    def _built(pb, built, stream):
+        """Wait for the kernels that fill the buffers, unless ``stream`` (a
+        handle) is the one they run on.  (A graph under capture cannot wait;
+        torch waits for the device before it begins one.)"""
+        if built is None or torch.cuda.is_current_stream_capturing():
+            return
+        if getattr(stream, 'value', stream) != built[0]:
+            built[1].synchronize()
+        elif not built[1].query():
+            return
+        pb['built'] = None
 
     def _step_args(self, precision):
         """Arguments of ``mx_adjoint_step`` on the buffers (a copy of those
@@ -333,6 +348,8 @@ class AdjointProblem:
         s.pose.theta, s.pose.period = pb['theta'].data_ptr(), pb['period'].data_ptr()
         if stream is None:
             stream = torch.cuda.current_stream(self.device).cuda_stream
+        if pb['built'] is not None:
+            self._built(pb, pb['built'], stream)
         _lib.check(_lib.lib.mx_adjoint_step(ctypes.byref(s), ctypes.c_void_p(stream)))
 
     @property
@@ -360,6 +377,8 @@ class AdjointProblem:
                 setattr(s.pose, name, held.data_ptr())
         s.loss_out, s.grad_theta, s.grad_period = (t.data_ptr() for t in (loss, grad_theta, grad_period))
         stream = torch.cuda.current_stream(self.device).cuda_stream
+        if pb['built'] is not None:
+            self._built(pb, pb['built'], stream)
         _lib.check(_lib.lib.mx_adjoint_step(ctypes.byref(s), ctypes.c_void_p(stream)))
         return loss, grad_theta, grad_period
 

@@ -80,27 +80,49 @@ def test_tasks_outside_the_lists(gpu, precision):
         assert torch.equal(a, b) and bool(torch.isfinite(a).all())
 
 
-def test_buffers_are_complete_when_they_are_handed_out(gpu, monkeypatch):
-    """Building the buffers waits for the kernels that fill them (delayed
-    here), so that a launch on another stream finds them filled."""
+@pytest.mark.parametrize('first', ['launch', 'current', 'graph'])
+def test_first_step_on_another_stream(gpu, monkeypatch, first):
+    """The kernels that fill the buffers (delayed here) have run when a step
+    is launched on another stream than theirs."""
     import torch
     from marxs_amd.adjoint import AdjointProblem
     prob = _problem(gpu, 50, np.full(50, 20), 8)
+    want = prob.loss_and_grad(prob.theta0, prob.period0, 64)
+    prob._pb = None
+    theta, period = prob.theta0.clone(), prob.period0.clone()
+    torch.cuda.synchronize()
     tasks = AdjointProblem._tasks
 
     def delayed(self, *args):
         torch.cuda._sleep(20_000_000)
         return tasks(self, *args)
     monkeypatch.setattr(AdjointProblem, '_tasks', delayed)
-    prob._pose_buffers()
-    assert torch.cuda.current_stream().query()
+    pb = prob._pose_buffers()
+    filled = pb['built'][1]
+    assert not filled.query()
     other = torch.cuda.Stream()
-    prob.buffers['theta'].copy_(prob.theta0)
-    prob.buffers['period'].copy_(prob.period0)
-    other.wait_stream(torch.cuda.current_stream())
-    prob.launch_loss_and_grad(64, other.cuda_stream)
+    if first == 'current':
+        with torch.cuda.stream(other):
+            got = prob.loss_and_grad(theta, period, 64)
+        assert filled.query()
+    else:
+        with torch.cuda.stream(other):
+            pb['theta'].copy_(theta)
+            pb['period'].copy_(period)
+        if first == 'graph':
+            graph = prob.capture(64)
+            for _ in range(3):
+                pb['loss'].zero_()
+                graph.replay()
+        else:
+            prob.launch_loss_and_grad(64, other.cuda_stream)
+        assert filled.query()
+        torch.cuda.synchronize()
+        got = pb['loss'][0], pb['grad7'][:, :6], pb['grad7'][:, 6]
     torch.cuda.synchronize()
-    assert float(prob.buffers['loss']) == float(prob.loss_and_grad(prob.theta0, prob.period0, 64)[0])
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
+    assert pb['built'] is None
 
 
 def test_base_pose_in_other_layouts(gpu):
