@@ -454,8 +454,8 @@ int mx_fill_i32(int32_t *dst, int64_t n, int32_t v, void *stream);
 
 /* Rows [n][4] = x, y, z, w (16-byte aligned) from three columns, and three
  * columns from the first values of rows [n][width], width >= 3 (homogeneous
- * coordinates of a photon table, marxs/optics/base.py:149-211).  Asynchronous
- * on the stream. */
+ * coordinates of a photon table, marxs/optics/base.py:149-211); n at most
+ * 2^32 - 256.  Asynchronous on the stream. */
 int mx_pack_rows(const double *x, const double *y, const double *z, double w, double *rows, int64_t n,
                  void *stream);
 int mx_unpack_rows(const double *rows, int64_t width, double *x, double *y, double *z, int64_t n,

@@ -3165,6 +3165,8 @@ __global__ __launch_bounds__(256) void mx_unpack_rows_kernel(const double *rows,
     z[i] = r[2];
 }
 
+#define MX_ROWS_MAX (((int64_t)1 << 32) - 256)  // a launch holds fewer than 2^32 work-items
+
 static int rows_launched(const char *what) {
     if (hipGetLastError() == hipSuccess) return 0;
     set_error(what);
@@ -3173,7 +3175,7 @@ static int rows_launched(const char *what) {
 
 extern "C" int mx_pack_rows(const double *x, const double *y, const double *z, double w, double *rows, int64_t n,
                             void *stream) {
-    if (n < 0 || n > ((int64_t)1 << 38)) { set_error("rows: number out of range"); return 1; }
+    if (n < 0 || n > MX_ROWS_MAX) { set_error("rows: number out of range"); return 1; }
     if (n == 0) return 0;
     if (!x || !y || !z || !rows) { set_error("rows: a pointer is NULL"); return 1; }
     if ((uintptr_t)rows & 15) { set_error("rows: not 16-byte aligned"); return 1; }
@@ -3184,7 +3186,7 @@ extern "C" int mx_pack_rows(const double *x, const double *y, const double *z, d
 
 extern "C" int mx_unpack_rows(const double *rows, int64_t width, double *x, double *y, double *z, int64_t n,
                               void *stream) {
-    if (n < 0 || n > ((int64_t)1 << 38)) { set_error("rows: number out of range"); return 1; }
+    if (n < 0 || n > MX_ROWS_MAX) { set_error("rows: number out of range"); return 1; }
     if (width < 3) { set_error("rows: fewer than 3 values"); return 1; }
     if (n == 0) return 0;
     if (!x || !y || !z || !rows) { set_error("rows: a pointer is NULL"); return 1; }

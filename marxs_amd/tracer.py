@@ -107,8 +107,10 @@ class DeviceTables:
 # Rows from which on they are turned on the device.  Its launches cost 15 to
 # 20 us each, numpy 1.5 to 4 ns a row: a table call of 3000 rows takes 543 us
 # with numpy and 573 with kernels, 6000 584 and 586, 10000 675 and 649, 40000
-# 1529 and 1263.
+# 1529 and 1263.  ROWS_MAX and more, near what a launch can hold, stay with
+# numpy too.
 ROWS_ON_DEVICE = 8192
+ROWS_MAX = 2 ** 31
 
 
 def _columns_of(rows, device):
@@ -124,7 +126,8 @@ def _columns_of(rows, device):
 
 def _rows_of(t, w):
     """Host rows (N, 4) of a (3, N) float64 device column, the last value w."""
-    if not (t.is_cuda and t.shape[-1] >= ROWS_ON_DEVICE and t.dtype == torch.float64 and t.dim() == 2 and t.shape[0] == 3 and t.stride(1) == 1):
+    if not (t.is_cuda and t.dim() == 2 and ROWS_ON_DEVICE <= t.shape[1] < ROWS_MAX and
+            t.dtype == torch.float64 and t.shape[0] == 3 and t.stride(1) == 1):
         out = np.empty((t.shape[1], 4))
         out[:, :3] = t.cpu().numpy().T
         out[:, 3] = w
@@ -174,7 +177,8 @@ class DevicePhotons:
 
         def col(name):
             rows = np.asarray(photons[name], dtype=float)
-            if dev.type == 'cuda' and rows.ndim == 2 and rows.shape[0] >= ROWS_ON_DEVICE and rows.shape[1] >= 3:
+            if (dev.type == 'cuda' and rows.ndim == 2 and ROWS_ON_DEVICE <= rows.shape[0] < ROWS_MAX and
+                    rows.shape[1] >= 3):
                 return _columns_of(np.require(rows, requirements=['C', 'W']), dev)
             return np.ascontiguousarray(rows[:, :3].T)
         pos = col('pos') if 'pos' in photons.colnames else None
