@@ -15,7 +15,8 @@
 // bins that hold a bound or the median:
 //   1. sample  one workgroup per order sorts up to 4096 photons drawn over the
 //              list and takes evenly filled bin edges from them;
-//   2. split   each workgroup takes one chunk of photons, orders its counted
+//   2. split   each workgroup takes one chunk of photons (pieces of 64 from all
+//              over the list), orders its counted
 //              values by (order, bin) in LDS and writes them back in that order
 //              with the offset of every (order, bin) piece, the piece's sums of
 //              deviations and squared deviations from an edge of the bin, and
@@ -294,8 +295,12 @@ static size_t split_lds(const OsPlan &L) {
            sizeof(uint16_t) * ((size_t)MX_OS_SPLIT_WAVES * kh + kh + 2);
 }
 
-// One chunk of photons ordered by (order, bin).  A photon's place is the start
-// of its piece, plus the photons of the piece in the waves before, plus its
+// One chunk of photons ordered by (order, bin).  The chunk takes 64 consecutive
+// photons for each row of each wave from equal steps over the whole list: in a
+// list sorted by value a chunk of consecutive photons is one long piece of one
+// bin, whose sums and copies are then one work-item's (1e7 photons sorted in two
+// orders 2942 us a call, 456 so; unsorted 600 either way).  A photon's place is
+// the start of its piece, plus the photons of the piece in the waves before, plus its
 // rank within its wave, which an LDS counter of that wave and piece returns:
 // only one wave uses it, and the lanes of one LDS instruction are served in a
 // fixed order, so places and sums are the same in every run.  Reads
@@ -315,14 +320,15 @@ __global__ __launch_bounds__(MX_OS_SPLIT, 4) void mx_os_split_kernel(MxOrderStat
     uint16_t *hist = (uint16_t *)(edges + (size_t)L.no * bins);   // [wave][kh]
     uint16_t *start = hist + MX_OS_SPLIT_WAVES * kh;              // [keys + 1]
     uint32_t *mine = (uint32_t *)(hist + w * kh);
-    const int64_t c = blockIdx.x, c0 = c * CH;
+    const int64_t c = blockIdx.x, step = (int64_t)MX_OS_SPLIT * L.chunks;
+    const int64_t first = ((int64_t)w * L.chunks + c) * 64 + lane;   // photon of row r: first + r * step
     const bool filter = (a.flags & MX_OS_FILTER) != 0;
     // columns first: their latency covers the set-up below
     int ord[ROWS];
     double pr[ROWS], val[ROWS];
 #pragma unroll
     for (int r = 0; r < ROWS; ++r) {
-        const int64_t i = c0 + r * MX_OS_SPLIT + t;
+        const int64_t i = first + r * step;
         const bool in = i < a.n;
         ord[r] = in ? a.order[i] : INT32_MIN;
         pr[r] = in ? a.prob[i] : 0.0;
@@ -350,7 +356,7 @@ __global__ __launch_bounds__(MX_OS_SPLIT, 4) void mx_os_split_kernel(MxOrderStat
         }
 #pragma unroll
         for (int r = 0; r < ROWS; ++r) {
-            const int k0 = c0 + r * MX_OS_SPLIT + t < a.n ? index_of(ord[r]) : -1;
+            const int k0 = first + r * step < a.n ? index_of(ord[r]) : -1;
 #pragma unroll
             for (int k = 0; k < MX_OS_SPLIT_WAVES; ++k) {
                 s[k] += k == k0 ? pr[r] : 0.0;
@@ -388,7 +394,7 @@ __global__ __launch_bounds__(MX_OS_SPLIT, 4) void mx_os_split_kernel(MxOrderStat
     uint32_t place[ROWS];   // piece and rank within the wave
 #pragma unroll
     for (int r = 0; r < ROWS; ++r) {
-        const bool in = c0 + r * MX_OS_SPLIT + t < a.n;
+        const bool in = first + r * step < a.n;
         const int k = in ? index_of(ord[r]) : -1;
         place[r] = 0xffffffffu;
         if (k >= 0) {
