@@ -70,6 +70,15 @@ __attribute__((visibility("hidden"))) void mx_set_error(const char *msg);
 #define MX_OS_HIST 2048        // buckets of a selection round
 #define MX_OS_CAND 64          // values ranked by counting, one per lane
 #define MX_OS_MAX_BINS 512
+// An order that holds more than MX_OS_SKEW times its even share of the sample
+// has its bins in proportion, at the cost of the others (order_bins): every
+// round of the clipping passes over the two bins with the bounds, so bins of
+// one large order among many were what a call took (1e7 photons, 97 % of them
+// in one of 64 orders: 7028 us a call with 16 bins each, 707 so; one of 15
+// orders 1963 us with 64 bins, 676).  Below that line bins are at most four times
+// larger than even ones.
+#define MX_OS_SKEW 4
+#define MX_OS_LEAST_BINS 8
 #define MX_OS_LUT 256
 
 static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
@@ -79,7 +88,7 @@ struct OsPlan {
     int32_t no, bins, keys;           // orders; bins per order; pieces per chunk
     int32_t rows, chunk, groups;      // photons per work-item and per chunk; groups of chunks
     int64_t chunks, stride;           // chunks; length of an offset row (one per piece, an entry per chunk)
-    size_t edges, off, piece, grp, place, next, psum, vals, copied, total;
+    size_t edges, off, piece, grp, place, next, lay, psum, vals, copied, total;
 };
 
 // One bin: place of its values when they were copied (-1: in pieces), their
@@ -89,7 +98,7 @@ struct BinInfo {
     double n, s1, s2;
 };
 
-// Bins per order: about 1000 (order, bin) pieces in all, so that the split
+// Bins per order (as shared evenly): about 1000 (order, bin) pieces in all, so that the split
 // kernel's counters fit beside the values in LDS; each order has one more
 // piece for the photons whose value is not counted.
 static void os_plan(int64_t n, int no, bool values, OsPlan &L) {
@@ -115,6 +124,7 @@ static void os_plan(int64_t n, int no, bool values, OsPlan &L) {
     L.grp = o;    o += align256(sizeof(BinInfo) * (size_t)L.groups * no * bins);
     L.place = o;  o += align256(sizeof(int64_t) * (size_t)no * bins);
     L.next = o;   o += align256(sizeof(unsigned long long));
+    L.lay = o;    o += align256(sizeof(int32_t) * (MX_MAX_ORDERS + 2));
     L.psum = o;   o += align256(sizeof(double) * (size_t)L.chunks * no);
     L.vals = o;   o += values ? align256(sizeof(double) * (size_t)L.chunks * L.chunk) : 0;
     L.copied = o; o += values ? align256(sizeof(double) * (size_t)(n > 0 ? n : 1)) : 0;
@@ -185,6 +195,46 @@ __device__ __forceinline__ int edge_rank(int j, int bins, int m) {
     return i < m ? i : m - 1;
 }
 
+// The bins of an order: the first among those of all orders, and their number.
+struct Bins {
+    int first, n;
+};
+// As the sample kernel shared them out: the first bin of each order and, last,
+// the end; then whether they are shared evenly.
+__device__ __forceinline__ const int32_t *layout(const OsPlan &L, const unsigned char *ws) {
+    return (const int32_t *)(ws + L.lay);
+}
+// (k: of the whole workgroup; scalar loads, the kernels that call this do not
+// write the layout)
+__device__ __forceinline__ Bins bins_of(const OsPlan &L, const unsigned char *ws, int k) {
+    const auto *lay = (const __attribute__((address_space(4))) int32_t *)layout(L, ws);
+    return {lay[k], lay[k + 1] - lay[k]};
+}
+
+// Bins of the order of this lane, by every wave for itself, from the photons of
+// each order (`count`, of lane's order) among `looked` ones: powers of two, evenly or,
+// when one order holds MX_OS_SKEW times its share, in proportion and
+// MX_OS_LEAST_BINS at least.
+__device__ __forceinline__ Bins order_bins(const OsPlan &L, int count, int looked, bool &even) {
+    const int lane = threadIdx.x & 63;
+    even = __ballot(count * L.no > MX_OS_SKEW * looked) == 0;
+    if (even) return {lane * L.bins, L.bins};
+    int total = count;
+    for (int o = 32; o > 0; o >>= 1) total += __shfl_xor(total, o);
+    int n = 0;
+    if (lane < L.no) {
+        const int share = count * (L.no * (L.bins - MX_OS_LEAST_BINS)) / total;
+        n = MX_OS_LEAST_BINS;
+        while (2 * n <= share && 2 * n <= MX_OS_MAX_BINS) n *= 2;
+    }
+    int end = n;
+    for (int d = 1; d < 64; d <<= 1) {
+        const int o = __shfl_up(end, d);
+        if (lane >= d) end += o;
+    }
+    return {end - n, n};
+}
+
 // Bin edges of one order (one workgroup each): the finite, counted values of
 // this order among MX_OS_SAMPLE photons, one from a pseudo-random place of
 // each of as many equal parts of the list, sorted; the edges split them
@@ -195,14 +245,15 @@ __device__ __forceinline__ int edge_rank(int j, int bins, int m) {
 __global__ __launch_bounds__(1024) void mx_os_sample_kernel(MxOrderStats a, OsPlan L,
                                                              unsigned char *ws) {
     __shared__ double s[MX_OS_SAMPLE];
-    __shared__ int cnt;
-    const int k = blockIdx.x, t = threadIdx.x, mine = a.orders[k];
-    const int bins = L.bins;
+    __shared__ int cnt, held[256];
+    const int k = blockIdx.x, t = threadIdx.x, lane = t & 63, mine = a.orders[k];
     double *edges = (double *)(ws + L.edges);
     if (k == 0 && t == 0) *(unsigned long long *)(ws + L.next) = 0;    // the merge kernel's allocator
     const bool filter = (a.flags & MX_OS_FILTER) != 0;
     if (t == 0) cnt = 0;
+    if (t < 256) held[t] = 0;
     __syncthreads();
+    const int number = lane < L.no ? a.orders[lane] : 0;
     const int64_t parts = a.n < MX_OS_SAMPLE ? a.n : MX_OS_SAMPLE;
     int64_t at[MX_OS_SAMPLE / 1024];
     int ord[MX_OS_SAMPLE / 1024];
@@ -220,6 +271,8 @@ __global__ __launch_bounds__(1024) void mx_os_sample_kernel(MxOrderStats a, OsPl
     double v[MX_OS_SAMPLE / 1024], pr[MX_OS_SAMPLE / 1024];
 #pragma unroll
     for (int r = 0; r < MX_OS_SAMPLE / 1024; ++r) {
+        // (for order_bins; orders that are 256 apart are counted together)
+        if (t % 16 == 0 && at[r] >= 0 && ord[r] != INT32_MIN) atomicAdd(&held[ord[r] & 255], 1);
         if (ord[r] != mine) at[r] = -1;
         v[r] = parts > 0 ? a.value[at[r] >= 0 ? at[r] : 0] : 0.0;
         pr[r] = parts > 0 && filter ? a.prob[at[r] >= 0 ? at[r] : 0] : 1.0;
@@ -233,6 +286,16 @@ __global__ __launch_bounds__(1024) void mx_os_sample_kernel(MxOrderStats a, OsPl
     while (size < m) size *= 2;
     for (int i = m + t; i < size; i += 1024) s[i] = __builtin_inf();
     __syncthreads();
+    bool even;
+    // (with few orders none can hold that many times its share)
+    const Bins lay = order_bins(L, lane < L.no && L.no > MX_OS_SKEW ? held[number & 255] : 0, (int)(parts + 15) / 16, even);
+    const int bins = __builtin_amdgcn_readlane(lay.n, k), first = __builtin_amdgcn_readlane(lay.first, k);
+    if (k == 0 && t < L.no) {
+        int32_t *all = (int32_t *)(ws + L.lay);
+        all[t] = lay.first;
+        if (t == L.no - 1) all[L.no] = lay.first + lay.n;
+        if (t == 0) all[MX_MAX_ORDERS + 1] = even ? 1 : 0;
+    }
     if (m <= 512) {
         // few values: each goes to the place that its rank says, one step
         // instead of up to 45 with a barrier each
@@ -265,8 +328,8 @@ __global__ __launch_bounds__(1024) void mx_os_sample_kernel(MxOrderStats a, OsPl
             e = s[edge_rank(j, bins, m)];
             if (j > 0 && s[edge_rank(j - 1, bins, m)] == e) e = nextafter(e, __builtin_inf());
         }
-        edges[(size_t)k * bins + j] = e;
-        ((int64_t *)(ws + L.place))[(size_t)k * bins + j] = -1;
+        edges[first + j] = e;
+        ((int64_t *)(ws + L.place))[first + j] = -1;
     }
 }
 
@@ -311,10 +374,10 @@ static size_t split_lds(const OsPlan &L) {
 template <int ROWS, bool VALUES>
 __global__ __launch_bounds__(MX_OS_SPLIT, 4) void mx_os_split_kernel(MxOrderStats a, OsPlan L, unsigned char *ws) {
     extern __shared__ __align__(16) unsigned char sm[];
-    __shared__ int ords[MX_MAX_ORDERS], lut[MX_OS_LUT], wtot[MX_OS_SPLIT_WAVES];
+    __shared__ int ords[MX_MAX_ORDERS], lut[MX_OS_LUT], wtot[MX_OS_SPLIT_WAVES], lay[MX_MAX_ORDERS + 2];
     constexpr int CH = ROWS * MX_OS_SPLIT;
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-    const int keys = L.keys, kh = (keys + 1) & ~1, bins = VALUES ? L.bins : 0;
+    const int kh = (L.keys + 1) & ~1, bins = VALUES ? L.bins : 0;
     double *buf = (double *)sm;
     double *edges = buf + CH;
     uint16_t *hist = (uint16_t *)(edges + (size_t)L.no * bins);   // [wave][kh]
@@ -337,7 +400,9 @@ __global__ __launch_bounds__(MX_OS_SPLIT, 4) void mx_os_split_kernel(MxOrderStat
     for (int j = lane; j < kh / 2; j += 64) mine[j] = 0;
     if (VALUES) {
         const double *ge = (const double *)(ws + L.edges);
+        const int entry = layout(L, ws)[t < MX_MAX_ORDERS + 2 ? t : 0];
         for (int j = t; j < L.no * bins; j += MX_OS_SPLIT) edges[j] = ge[j];
+        if (t < MX_MAX_ORDERS + 2) lay[t] = entry;
     }
     const OrderLut index_of = build_lut(a, ords, lut);
     __shared__ double part[MX_MAX_ORDERS];
@@ -391,21 +456,42 @@ __global__ __launch_bounds__(MX_OS_SPLIT, 4) void mx_os_split_kernel(MxOrderStat
         }
         return;
     }
+    // bins and pieces of order k
+    const bool even = !VALUES || __builtin_amdgcn_readfirstlane(lay[MX_MAX_ORDERS + 1]) != 0;
+    auto first_key = [&](int k) { return even ? k * (bins + 1) : lay[k] + k; };
+    const int keys = even ? L.keys : __builtin_amdgcn_readfirstlane(lay[L.no]) + L.no;
     uint32_t place[ROWS];   // piece and rank within the wave
+    auto put = [&](int r, int key) {
+        const int sh = (key & 1) * 16;
+        const uint32_t old = atomicAdd(mine + (key >> 1), 1u << sh);
+        place[r] = ((uint32_t)key << 16) | ((old >> sh) & 0xffffu);
+    };
+    if (even) {
 #pragma unroll
-    for (int r = 0; r < ROWS; ++r) {
-        const bool in = first + r * step < a.n;
-        const int k = in ? index_of(ord[r]) : -1;
-        place[r] = 0xffffffffu;
-        if (k >= 0) {
-            int key = k;
-            if (VALUES) {
-                const bool counted = isfinite(val[r]) && (!filter || pr[r] > 0.0);
-                key = k * (bins + 1) + (counted ? bin_of(edges + k * bins, bins, val[r]) : bins);
+        for (int r = 0; r < ROWS; ++r) {
+            const bool in = first + r * step < a.n;
+            const int k = in ? index_of(ord[r]) : -1;
+            place[r] = 0xffffffffu;
+            if (k >= 0) {
+                int key = k;
+                if (VALUES) {
+                    const bool counted = isfinite(val[r]) && (!filter || pr[r] > 0.0);
+                    key = k * (bins + 1) + (counted ? bin_of(edges + k * bins, bins, val[r]) : bins);
+                }
+                put(r, key);
             }
-            const int sh = (key & 1) * 16;
-            const uint32_t old = atomicAdd(mine + (key >> 1), 1u << sh);
-            place[r] = ((uint32_t)key << 16) | ((old >> sh) & 0xffffu);
+        }
+    } else {
+#pragma unroll
+        for (int r = 0; r < ROWS; ++r) {
+            const bool in = first + r * step < a.n;
+            const int k = in ? index_of(ord[r]) : -1;
+            place[r] = 0xffffffffu;
+            if (k >= 0) {
+                const bool counted = isfinite(val[r]) && (!filter || pr[r] > 0.0);
+                const int b0 = lay[k], n = lay[k + 1] - b0;
+                put(r, b0 + k + (counted ? bin_of(edges + b0, n, val[r]) : n));
+            }
         }
     }
     __syncthreads();
@@ -453,9 +539,9 @@ __global__ __launch_bounds__(MX_OS_SPLIT, 4) void mx_os_split_kernel(MxOrderStat
         const int all = start[keys];
         for (int j = t; j < all; j += MX_OS_SPLIT) out[j] = buf[j];
         double2 *piece = (double2 *)(ws + L.piece) + (size_t)c * L.no * bins;
-        for (int j = t; j < L.no * bins; j += MX_OS_SPLIT) {
-            const int k = j / bins, b = j - k * bins, e = start[j + k + 1];
-            const double ref = bin_ref(edges + k * bins, bins, b);
+        auto sum_up = [&](int j, int k, int b0, int n) {
+            const int e = start[j + k + 1];
+            const double ref = bin_ref(edges + b0, n, j - b0);
             double2 p = make_double2(0.0, 0.0);
 #pragma unroll 4
             for (int q = start[j + k]; q < e; ++q) {
@@ -464,6 +550,15 @@ __global__ __launch_bounds__(MX_OS_SPLIT, 4) void mx_os_split_kernel(MxOrderStat
                 p.y += d * d;
             }
             piece[j] = p;
+        };
+        if (even) {
+            for (int j = t; j < L.no * bins; j += MX_OS_SPLIT) sum_up(j, j / bins, j / bins * bins, bins);
+        } else {
+            for (int j = t; j < keys - L.no; j += MX_OS_SPLIT) {
+                int k = 0;
+                while (lay[k + 1] <= j) ++k;
+                sum_up(j, k, lay[k], lay[k + 1] - lay[k]);
+            }
         }
         __syncthreads();
     }
@@ -475,7 +570,7 @@ __global__ __launch_bounds__(MX_OS_SPLIT, 4) void mx_os_split_kernel(MxOrderStat
     __syncthreads();
     const int parts = L.no < MX_OS_SPLIT_WAVES ? MX_OS_SPLIT_WAVES : 1;
     for (int j = w; j < L.no * parts; j += MX_OS_SPLIT_WAVES) {
-        const int k = j / parts, b = start[k * (bins + 1)], e = start[(k + 1) * (bins + 1)];
+        const int k = j / parts, b = start[first_key(k)], e = start[first_key(k + 1)];
         double s = 0.0;
 #pragma unroll 4
         for (int q = b + (j % parts) * 64 + lane; q < e; q += 64 * parts) s += buf[q];
@@ -579,9 +674,11 @@ struct BinPieces {
     }
 };
 
-__device__ __forceinline__ BinPieces pieces_of(const OsPlan &L, const unsigned char *ws, int k, int b, int span) {
-    return {(const uint16_t *)(ws + L.off) + (k * (L.bins + 1) + b) * L.stride, (const double *)(ws + L.vals), L.chunks,
-            span * L.stride, L.chunk};
+// (key: number of the piece, its bin's among the orders' bins and the piece
+// of uncounted photons behind those of each order)
+__device__ __forceinline__ BinPieces pieces_of(const OsPlan &L, const unsigned char *ws, int key, int span) {
+    return {(const uint16_t *)(ws + L.off) + key * L.stride, (const double *)(ws + L.vals), L.chunks, span * L.stride,
+            L.chunk};
 }
 
 // Work-items per piece of m values on average: the power of two above it.
@@ -645,18 +742,19 @@ __global__ __launch_bounds__(MX_OS_MERGE) void mx_os_merge_kernel(OsPlan L, unsi
     __shared__ double red[3][MX_OS_MERGE];
     __shared__ int s_first[MX_OS_MERGE], s_wave[MX_OS_MERGE / 64];
     __shared__ long long base;
-    const int t = threadIdx.x, k = blockIdx.y;
-    const int bins = L.bins;
+    const int t = threadIdx.x, k = blockIdx.y, all = L.no * L.bins;
+    const Bins B = bins_of(L, ws, k);
+    const int bins = B.n;
     if ((int)blockIdx.x < L.groups) {
         const int b = t % bins, sub = t / bins, subs = MX_OS_MERGE / bins;
         const int64_t per = (L.chunks + L.groups - 1) / L.groups;
         const int64_t c0 = blockIdx.x * per, c1 = c0 + per < L.chunks ? c0 + per : L.chunks;
-        const BinPieces P = pieces_of(L, ws, k, b, 1);
-        const double2 *piece = (const double2 *)(ws + L.piece) + (size_t)k * bins + b;
+        const BinPieces P = pieces_of(L, ws, B.first + k + b, 1);
+        const double2 *piece = (const double2 *)(ws + L.piece) + B.first + b;
         double n = 0.0, s1 = 0.0, s2 = 0.0;
 #pragma unroll 4
         for (int64_t c = c0 + sub; c < c1; c += subs) {
-            const double2 p = piece[(size_t)c * L.no * bins];
+            const double2 p = piece[(size_t)c * all];
             n += (double)((int)P.off[P.end + c] - (int)P.off[c]);
             s1 += p.x;
             s2 += p.y;
@@ -671,7 +769,7 @@ __global__ __launch_bounds__(MX_OS_MERGE) void mx_os_merge_kernel(OsPlan L, unsi
                 s1 += red[1][q];
                 s2 += red[2][q];
             }
-            ((BinInfo *)(ws + L.grp))[((size_t)k * L.groups + blockIdx.x) * bins + b] = {0, n, s1, s2};
+            ((BinInfo *)(ws + L.grp))[(size_t)B.first * L.groups + (size_t)blockIdx.x * bins + b] = {0, n, s1, s2};
         }
         return;
     }
@@ -679,12 +777,12 @@ __global__ __launch_bounds__(MX_OS_MERGE) void mx_os_merge_kernel(OsPlan L, unsi
     const int b = j < MX_OS_ENDS ? j : (j < 2 * MX_OS_ENDS ? bins - 1 - (j - MX_OS_ENDS)
                                                            : bins / 2 - MX_OS_NEAR / 2 + (j - 2 * MX_OS_ENDS));
     if (j >= 2 * MX_OS_ENDS && (b < MX_OS_ENDS || b >= bins - MX_OS_ENDS)) return;
-    if (bin_single((const double *)(ws + L.edges) + (size_t)k * bins, b)) return;
-    const BinPieces P = pieces_of(L, ws, k, b, 1);
+    if (bin_single((const double *)(ws + L.edges) + B.first, b)) return;
+    const BinPieces P = pieces_of(L, ws, B.first + k + b, 1);
     const Share H = share_pieces<MX_OS_MERGE>(P, s_first, s_wave);
     if (t == 0) {
         base = (long long)atomicAdd((unsigned long long *)(ws + L.next), (unsigned long long)H.all);
-        ((int64_t *)(ws + L.place))[(size_t)k * bins + b] = base;
+        ((int64_t *)(ws + L.place))[B.first + b] = base;
     }
     __syncthreads();
     double *out = (double *)(ws + L.copied) + base + H.first;
@@ -696,7 +794,7 @@ __global__ __launch_bounds__(MX_OS_MERGE) void mx_os_merge_kernel(OsPlan L, unsi
 struct ClipOrder {
     const OsPlan &L;
     const unsigned char *ws;
-    int k, bins;
+    int key, bins;            // piece of bin 0; bins
     const double *edges;      // LDS
     const BinInfo *info;      // LDS
     // f(x) for every value of bin b, by the `nth` work-items tid = 0, 1, ...
@@ -714,7 +812,7 @@ struct ClipOrder {
             }
         } else {
             const int per = items_per_piece(n, L.chunks, nth);
-            pieces_of(L, ws, k, b, 1).each(tid / per, nth / per, tid & (per - 1), per, [&](double x, int64_t) { f(x); });
+            pieces_of(L, ws, key + b, 1).each(tid / per, nth / per, tid & (per - 1), per, [&](double x, int64_t) { f(x); });
         }
     }
     __device__ __forceinline__ bool single(int b) const { return bin_single(edges, b); }
@@ -731,7 +829,8 @@ struct ClipOrder {
 
 // LDS of the clipping kernel: bins, edges, list.
 static size_t clip_lds(const OsPlan &L) {
-    return (sizeof(double) + sizeof(BinInfo)) * (size_t)L.bins + sizeof(double) * MX_OS_LIST;
+    return (sizeof(double) + sizeof(BinInfo)) * (size_t)(L.no > MX_OS_SKEW ? MX_OS_MAX_BINS : L.bins) +
+           sizeof(double) * MX_OS_LIST;
 }
 
 #define MX_OS_CW (MX_OS_CLIP / 64)
@@ -1165,8 +1264,9 @@ __global__ __launch_bounds__(MX_OS_CLIP) void mx_os_clip_kernel(MxOrderStats a, 
     extern __shared__ __align__(16) unsigned char sm[];
     __shared__ ClipShared S;
     const int k = blockIdx.x, t = threadIdx.x, w = t >> 6;
-    const int bins = VALUES ? L.bins : 0;
-    const BinPieces rest = pieces_of(L, ws, k, bins, 1);
+    const Bins B = VALUES ? bins_of(L, ws, k) : Bins{0, 0};
+    const int bins = B.n, key = B.first + k;
+    const BinPieces rest = pieces_of(L, ws, key + bins, 1);
     // probability sum; photons outside the bins
     const double *psum = (const double *)(ws + L.psum) + (size_t)k * L.chunks;
     CutSums tot = {0.0, 0.0, 0.0};
@@ -1181,16 +1281,16 @@ __global__ __launch_bounds__(MX_OS_CLIP) void mx_os_clip_kernel(MxOrderStats a, 
     double *edges = (double *)(info + bins), *list = edges + bins;
     if (VALUES) {
         for (int b = t; b < bins; b += MX_OS_CLIP) {
-            BinInfo f = {((const int64_t *)(ws + L.place))[(size_t)k * bins + b], 0.0, 0.0, 0.0};
+            BinInfo f = {((const int64_t *)(ws + L.place))[B.first + b], 0.0, 0.0, 0.0};
 #pragma unroll 4
             for (int g = 0; g < L.groups; ++g) {
-                const BinInfo q = ((const BinInfo *)(ws + L.grp))[((size_t)k * L.groups + g) * bins + b];
+                const BinInfo q = ((const BinInfo *)(ws + L.grp))[(size_t)B.first * L.groups + (size_t)g * bins + b];
                 f.n += q.n;
                 f.s1 += q.s1;
                 f.s2 += q.s2;
             }
             info[b] = f;
-            edges[b] = ((const double *)(ws + L.edges))[(size_t)k * bins + b];
+            edges[b] = ((const double *)(ws + L.edges))[B.first + b];
         }
         if (t < 2) S.n[t] = 0;
     }
@@ -1207,7 +1307,7 @@ __global__ __launch_bounds__(MX_OS_CLIP) void mx_os_clip_kernel(MxOrderStats a, 
         }
         return;
     }
-    const ClipOrder O = {L, ws, k, bins, edges, info};
+    const ClipOrder O = {L, ws, key, bins, edges, info};
     Kept K = {0, bins - 1, false, 0.0, 0.0, {0.0, 0.0, 0.0}, {0.0, 0.0, 0.0}};
     double N = kept_count(O, K);
     if (t == 0) {
@@ -1222,7 +1322,7 @@ __global__ __launch_bounds__(MX_OS_CLIP) void mx_os_clip_kernel(MxOrderStats a, 
         double c = 0.0, below = 0.0;
         if (N <= (double)MX_OS_LIST) {
             // the whole order into the list, in the same places every run
-            const BinPieces P = pieces_of(L, ws, k, 0, bins);
+            const BinPieces P = pieces_of(L, ws, key, bins);
             const Share R = share_pieces<MX_OS_CLIP>(P, S.first, S.iw);
             if (t == 0) {
                 S.kmin = ~0ull;
