@@ -349,6 +349,28 @@ __device__ __forceinline__ int bin_of(const double *edges, int bins, double x) {
     return b;
 }
 
+// Sums over the lanes up to each one, by the cross-lane moves of the vector
+// unit (a move through LDS costs ten times the latency).
+template <int CTRL, int ROWS> __device__ __forceinline__ double lane_move(double v) {
+    return __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, ROWS, 0xf, false),
+                            __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROWS, 0xf, false));
+}
+__device__ __forceinline__ double wave_scan(double v) {
+    v += lane_move<0x111, 0xf>(v);    // one lane up within 16
+    v += lane_move<0x112, 0xf>(v);
+    v += lane_move<0x114, 0xf>(v);
+    v += lane_move<0x118, 0xf>(v);
+    v += lane_move<0x142, 0xa>(v);    // the last lane of 16 to the next 16
+    v += lane_move<0x143, 0xc>(v);    // the last lane of 32 to the next 32
+    return v;
+}
+__device__ __forceinline__ double lane_value(double v, int lane) {
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                            __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
+// Sum over the wave in a fixed order; every lane gets it.
+__device__ __forceinline__ double wave_add(double v) { return lane_value(wave_scan(v), 63); }
+
 // ----------------------------------------------------------------- 2 split
 // LDS of the split kernel: the chunk's values (then its probabilities), the
 // edges, one counter (16 bits) per wave and piece, piece starts.
@@ -431,13 +453,10 @@ __global__ __launch_bounds__(MX_OS_SPLIT, 4) void mx_os_split_kernel(MxOrderStat
         __shared__ int count[MX_MAX_ORDERS];
 #pragma unroll
         for (int k = 0; k < MX_OS_SPLIT_WAVES; ++k) {
-            for (int o = 32; o > 0; o >>= 1) {
-                s[k] += __shfl_xor(s[k], o);
-                m[k] += __shfl_xor(m[k], o);
-            }
-            if (lane == 0) {
-                part[k * MX_OS_SPLIT_WAVES + w] = s[k];
-                count[k * MX_OS_SPLIT_WAVES + w] = m[k];
+            const double sum = wave_scan(s[k]), n = wave_scan((double)m[k]);
+            if (lane == 63) {
+                part[k * MX_OS_SPLIT_WAVES + w] = sum;
+                count[k * MX_OS_SPLIT_WAVES + w] = (int)n;
             }
         }
         __syncthreads();
@@ -586,28 +605,6 @@ __global__ __launch_bounds__(MX_OS_SPLIT, 4) void mx_os_split_kernel(MxOrderStat
 }
 
 // ----------------------------------------------------------------- 3 merge
-// Sums over the lanes up to each one, by the cross-lane moves of the vector
-// unit (a move through LDS costs ten times the latency).
-template <int CTRL, int ROWS> __device__ __forceinline__ double lane_move(double v) {
-    return __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, ROWS, 0xf, false),
-                            __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROWS, 0xf, false));
-}
-__device__ __forceinline__ double wave_scan(double v) {
-    v += lane_move<0x111, 0xf>(v);    // one lane up within 16
-    v += lane_move<0x112, 0xf>(v);
-    v += lane_move<0x114, 0xf>(v);
-    v += lane_move<0x118, 0xf>(v);
-    v += lane_move<0x142, 0xa>(v);    // the last lane of 16 to the next 16
-    v += lane_move<0x143, 0xc>(v);    // the last lane of 32 to the next 32
-    return v;
-}
-__device__ __forceinline__ double lane_value(double v, int lane) {
-    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
-                            __builtin_amdgcn_readlane(__double2loint(v), lane));
-}
-// Sum over the wave in a fixed order; every lane gets it.
-__device__ __forceinline__ double wave_add(double v) { return lane_value(wave_scan(v), 63); }
-
 // Order-preserving integer of a finite double, and back.
 __device__ __forceinline__ uint64_t key_of(double x) {
     const uint64_t u = (uint64_t)__double_as_longlong(x);
@@ -1270,6 +1267,9 @@ __global__ __launch_bounds__(MX_OS_CLIP) void mx_os_clip_kernel(MxOrderStats a, 
     // probability sum; photons outside the bins
     const double *psum = (const double *)(ws + L.psum) + (size_t)k * L.chunks;
     CutSums tot = {0.0, 0.0, 0.0};
+    // (a list of 3e8 photons has 95 chunks for each work-item, one latency each
+    // unless the loads overlap)
+#pragma unroll 8
     for (int64_t c = t; c < L.chunks; c += MX_OS_CLIP) {
         tot.s1 += psum[c];
         tot.n += (double)((int)rest.off[rest.end + c] - (int)rest.off[c]);
