@@ -520,13 +520,15 @@ extern "C" int mx_facet_pose(const MxPoseArgs *a, void *stream) {
 // Loss and gradient over photons ordered by facet, in two kernels.  With the
 // photons of a facet together nothing needs an atomic: a task is up to a few
 // hundred photons of one facet, whose workgroup forms the facet's frame itself,
-// keeps the sums in registers and writes them once; then one wave per facet
-// adds its tasks and applies the chain rule.  The call without that order
-// (fill, frames, replay, chain rule: 4 kernels) adds every photon's 26 values
-// with atomics, in LDS up to 315 facets and in global memory beyond.  Kernel
-// times, us: 200 facets, 2.1e4 photons FP32 31 -> 14; 600 facets, 9.1e4
-// photons FP64 178 -> 18.  Bound by latency: the chain of one photon's replay
-// (two planes, the grating equation and its adjoint) and of the facet's frame.
+// keeps the sums in registers and writes them once; then two waves per facet
+// add its tasks, form its frame and apply the chain rule.  The call without
+// that order (fill, frames, replay, chain rule: 4 kernels) adds every photon's
+// 26 values with atomics, in LDS up to 315 facets and in global memory beyond.
+// Kernel times, us: 200 facets, 2.1e4 photons FP32 31 -> 14.6; 600 facets,
+// 9.1e4 photons FP64 178 -> 18.7.  Bound by the chain of one photon's replay
+// (two planes, the grating equation and its adjoint) and of the facet's frame:
+// vector unit busy 18 % of the photon kernel's time at 200 facets, 58 % at 600;
+// the facet kernel's waves wait for 65 to 72 % of theirs.
 #define AJ_TASK 128             // work-items per task
 #define AJ_SUMS (2 * AJ_NG + 3) // A, B, moments
 
@@ -555,7 +557,7 @@ static_assert(AJ_SUMS <= MX_AJ_PART, "a task's sums and moments");
 
 // The first photon of each work-item is loaded before the facet's frame is
 // formed, so that the loads are under way during that chain (8.7 -> 8.3 us for
-// 200 facets; 11.4 either way for 600).
+// 200 facets; 11.5 either way for 600).
 template <int PREC>
 __global__ __launch_bounds__(AJ_TASK) void mx_adjoint_task_kernel(MxAdjointStep S) {
     __shared__ double red[AJ_TASK / 64][AJ_SUMS];

@@ -34,9 +34,12 @@
 // values written once (8 B each); a method that keeps no table of values could
 // do with the read alone.  The two device-wide radix sorts this replaced
 // moved each value nine times.  CaptureResAeff on 8e6 photons in 15 orders:
-// 1230 us a call with them, 377 us now, 211 us of it in the kernels (160 MB: 26
-// us at the card's read rate); on 5e4 photons 400 us in 44 launches, now 223 us
-// in 4, 86 us of it in the kernels.
+// 1230 us a call with them, 320 us now, 213 us of it in the kernels (160 MB: 26
+// us at the card's read rate); on 5e4 photons 400 us in 44 launches, now 133 us
+// in 4, 88 us of it in the kernels.  The split kernel has the vector unit busy
+// for 39 % of its time and half of its waves' time waits; the kernels with one
+// workgroup per order (sample, clip) wait for loads and barriers for more than
+// half of theirs on 15 of the 256 CUs.
 
 #include <hip/hip_runtime.h>
 #include <mutex>
@@ -387,11 +390,13 @@ static size_t split_lds(const OsPlan &L) {
 // orders 2942 us a call, 456 so; unsorted 600 either way).  A photon's place is
 // the start of its piece, plus the photons of the piece in the waves before, plus its
 // rank within its wave, which an LDS counter of that wave and piece returns:
-// only one wave uses it, and the lanes of one LDS instruction are served in a
-// fixed order, so places and sums are the same in every run.  Reads
+// only one wave uses it.  That places and sums are the same in every run assumes
+// that the lanes of one LDS instruction are served in a fixed order, which no
+// document states (the tests call twice and compare); in another order values
+// would change places within a piece, and means their last bits.  Reads
 // 20 B per photon and writes 8 B per counted value plus 18 B per piece; bound
 // by the LDS work between (edge search 6 reads per value at 64 bins, counter,
-// scatter, sums): 76 us for 8e6 photons in 15 orders (247 MB: 48 us at the
+// scatter, sums): 77 us for 8e6 photons in 15 orders (247 MB: 48 us at the
 // card's copy rate).
 template <int ROWS, bool VALUES>
 __global__ __launch_bounds__(MX_OS_SPLIT, 4) void mx_os_split_kernel(MxOrderStats a, OsPlan L, unsigned char *ws) {
@@ -1253,7 +1258,7 @@ __device__ __forceinline__ void cut_bins(const ClipOrder &O, Kept &K, double c, 
 // One order: probability sum and count, then the clipping rounds.  Bound by
 // the latency of its dependent steps, so everything that can be is done by
 // every wave for itself, and a round has two barriers: one after the sums over
-// the two cut bins, one after the candidates of the median (92 us for 8e6
+// the two cut bins, one after the candidates of the median (94 us for 8e6
 // photons in 15 orders; with a workgroup-wide reduction for each sum and a
 // selection from the start for each median 179 us).
 template <bool VALUES>
