@@ -524,8 +524,8 @@ extern "C" int mx_facet_pose(const MxPoseArgs *a, void *stream) {
 // add its tasks, form its frame and apply the chain rule.  The call without
 // that order (fill, frames, replay, chain rule: 4 kernels) adds every photon's
 // 26 values with atomics, in LDS up to 315 facets and in global memory beyond.
-// Kernel times, us: 200 facets, 2.1e4 photons FP32 31 -> 14.6; 600 facets,
-// 9.1e4 photons FP64 178 -> 18.7.  Bound by the chain of one photon's replay
+// Kernel times, us: 200 facets, 2.1e4 photons FP32 31 -> 13.4; 600 facets,
+// 9.1e4 photons FP64 178 -> 17.9.  Bound by the chain of one photon's replay
 // (two planes, the grating equation and its adjoint) and of the facet's frame:
 // vector unit busy 18 % of the photon kernel's time at 200 facets, 58 % at 600;
 // the facet kernel's waves wait for 65 to 72 % of theirs.
@@ -655,15 +655,15 @@ __global__ __launch_bounds__(AJ_MOMENTS) void mx_adjoint_moments_kernel(MxAdjoin
 // Two waves per facet: the first adds the sums of the facet's tasks and, for
 // itself, the moments of all tasks, while the second forms the facet's frame
 // and its derivatives.  Bound by latency: one wave doing both, with the moments
-// 256 bytes apart, took 9.9 us for 200 facets and 16.5 us for 600, this 6.0 and
-// 7.0.  (MANY: the moments are there, from mx_adjoint_moments_kernel.)
+// 256 bytes apart, took 9.9 us for 200 facets and 16.5 us for 600, this 5.1 and
+// 6.4.  (MANY: the moments are there, from mx_adjoint_moments_kernel.)
 template <bool MANY>
 __global__ __launch_bounds__(128) void mx_adjoint_finish_kernel(MxAdjointStep S) {
     __shared__ double sums[2 * AJ_NG];
     __shared__ PoseParts parts;
     const int f = blockIdx.x, lane = threadIdx.x & 63;
     const MxPoseArgs &P = S.pose;
-    double m[3] = {0.0, 0.0, 0.0};
+    double m[3] = {0.0, 0.0, 0.0}, geom[MX_AJ_GEOM];
     if (threadIdx.x < 64) {
         int most = S.n_tasks;
         asm volatile("" : "+s"(most));
@@ -686,19 +686,18 @@ __global__ __launch_bounds__(128) void mx_adjoint_finish_kernel(MxAdjointStep S)
     } else {
         PoseParts p;
         pose_parts(P, f, p);
-        double geom[MX_AJ_GEOM];
         pose_geometry(P, f, p, geom);
+        if (lane == 0) parts = p;
+    }
+    __syncthreads();
+    if (threadIdx.x >= 64) {
+        // (stores here, as the barrier would wait for them)
         if (lane == 0) {
-            parts = p;
             for (int k = 0; k < MX_AJ_GEOM; ++k) P.geom[(size_t)f * MX_AJ_GEOM + k] = geom[k];
             if (S.theta_out)
                 for (int k = 0; k < 6; ++k) S.theta_out[(size_t)f * 6 + k] = P.theta[(size_t)f * 6 + k];
             if (S.period_out) S.period_out[f] = P.period[f];
         }
-    }
-    __syncthreads();
-    if (threadIdx.x >= 64) {
-        // (here, as the barrier would wait for the stores)
         if (S.sums_out && lane < 2 * AJ_NG) S.sums_out[(size_t)f * (2 * AJ_NG) + lane] = sums[lane];
         return;
     }
