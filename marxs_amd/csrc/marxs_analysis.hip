@@ -204,13 +204,11 @@ struct Bins {
 };
 // As the sample kernel shared them out: the first bin of each order and, last,
 // the end; then whether they are shared evenly.
-__device__ __forceinline__ const int32_t *layout(const OsPlan &L, const unsigned char *ws) {
-    return (const int32_t *)(ws + L.lay);
-}
-// (k: of the whole workgroup; scalar loads, the kernels that call this do not
-// write the layout)
+// (Read by scalar loads: the kernels that read it do not write it.)
+typedef const __attribute__((address_space(4))) int32_t *Layout;
+__device__ __forceinline__ Layout layout(const OsPlan &L, const unsigned char *ws) { return (Layout)(ws + L.lay); }
 __device__ __forceinline__ Bins bins_of(const OsPlan &L, const unsigned char *ws, int k) {
-    const auto *lay = (const __attribute__((address_space(4))) int32_t *)layout(L, ws);
+    const Layout lay = layout(L, ws);
     return {lay[k], lay[k + 1] - lay[k]};
 }
 
@@ -274,12 +272,15 @@ __global__ __launch_bounds__(1024) void mx_os_sample_kernel(MxOrderStats a, OsPl
     double v[MX_OS_SAMPLE / 1024], pr[MX_OS_SAMPLE / 1024];
 #pragma unroll
     for (int r = 0; r < MX_OS_SAMPLE / 1024; ++r) {
-        // (for order_bins; orders that are 256 apart are counted together)
-        if (t % 16 == 0 && at[r] >= 0 && ord[r] != INT32_MIN) atomicAdd(&held[ord[r] & 255], 1);
         if (ord[r] != mine) at[r] = -1;
         v[r] = parts > 0 ? a.value[at[r] >= 0 ? at[r] : 0] : 0.0;
         pr[r] = parts > 0 && filter ? a.prob[at[r] >= 0 ? at[r] : 0] : 1.0;
     }
+    // (for order_bins, while the values are on their way; orders that are 256
+    // apart are counted together)
+#pragma unroll
+    for (int r = 0; r < MX_OS_SAMPLE / 1024; ++r)
+        if (t % 16 == 0 && t + 1024 * r < parts && ord[r] != INT32_MIN) atomicAdd(&held[ord[r] & 255], 1);
 #pragma unroll
     for (int r = 0; r < MX_OS_SAMPLE / 1024; ++r)
         if (at[r] >= 0 && isfinite(v[r]) && (!filter || pr[r] > 0.0)) s[atomicAdd(&cnt, 1)] = v[r];
@@ -401,7 +402,7 @@ static size_t split_lds(const OsPlan &L) {
 template <int ROWS, bool VALUES>
 __global__ __launch_bounds__(MX_OS_SPLIT, 4) void mx_os_split_kernel(MxOrderStats a, OsPlan L, unsigned char *ws) {
     extern __shared__ __align__(16) unsigned char sm[];
-    __shared__ int ords[MX_MAX_ORDERS], lut[MX_OS_LUT], wtot[MX_OS_SPLIT_WAVES], lay[MX_MAX_ORDERS + 2];
+    __shared__ int ords[MX_MAX_ORDERS], lut[MX_OS_LUT], wtot[MX_OS_SPLIT_WAVES], lay[MX_MAX_ORDERS + 1];
     constexpr int CH = ROWS * MX_OS_SPLIT;
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
     const int kh = (L.keys + 1) & ~1, bins = VALUES ? L.bins : 0;
@@ -413,6 +414,7 @@ __global__ __launch_bounds__(MX_OS_SPLIT, 4) void mx_os_split_kernel(MxOrderStat
     const int64_t c = blockIdx.x, step = (int64_t)MX_OS_SPLIT * L.chunks;
     const int64_t first = ((int64_t)w * L.chunks + c) * 64 + lane;   // photon of row r: first + r * step
     const bool filter = (a.flags & MX_OS_FILTER) != 0;
+    const bool even = !VALUES || layout(L, ws)[MX_MAX_ORDERS + 1] != 0;
     // columns first: their latency covers the set-up below
     int ord[ROWS];
     double pr[ROWS], val[ROWS];
@@ -427,9 +429,8 @@ __global__ __launch_bounds__(MX_OS_SPLIT, 4) void mx_os_split_kernel(MxOrderStat
     for (int j = lane; j < kh / 2; j += 64) mine[j] = 0;
     if (VALUES) {
         const double *ge = (const double *)(ws + L.edges);
-        const int entry = layout(L, ws)[t < MX_MAX_ORDERS + 2 ? t : 0];
         for (int j = t; j < L.no * bins; j += MX_OS_SPLIT) edges[j] = ge[j];
-        if (t < MX_MAX_ORDERS + 2) lay[t] = entry;
+        if (!even && t <= L.no) lay[t] = ((const int32_t *)(ws + L.lay))[t];
     }
     const OrderLut index_of = build_lut(a, ords, lut);
     __shared__ double part[MX_MAX_ORDERS];
@@ -481,7 +482,6 @@ __global__ __launch_bounds__(MX_OS_SPLIT, 4) void mx_os_split_kernel(MxOrderStat
         return;
     }
     // bins and pieces of order k
-    const bool even = !VALUES || __builtin_amdgcn_readfirstlane(lay[MX_MAX_ORDERS + 1]) != 0;
     auto first_key = [&](int k) { return even ? k * (bins + 1) : lay[k] + k; };
     const int keys = even ? L.keys : __builtin_amdgcn_readfirstlane(lay[L.no]) + L.no;
     uint32_t place[ROWS];   // piece and rank within the wave
